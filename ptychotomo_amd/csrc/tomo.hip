@@ -4,8 +4,8 @@
 // divphi, unpaddivphi, fftshiftc, fftshift1c, wrap, wrapadj, takexy, gather,
 // scatter, circ, pad, pad2) and its three cuFFT plans.
 //
-// Same mathematics as the reference chain (Gaussian gridding on the 2N x 2N
-// oversampled grid, N = 3n/2, mu and M from eps = 1e-6), restructured:
+// Same mathematics as the reference chain (gridding on the 2N x 2N oversampled
+// grid, N = 3n/2), restructured:
 //  * The checkerboard multiplications around each FFT are centred DFTs; they
 //    are realised as index rotations on load/store (free).
 //  * The 2N-point centred DFT of an input that is non-zero only on the
@@ -20,9 +20,9 @@
 //    only the n object rows are transformed.
 //  * The periodic halo of the gridding grid (wrap/wrapadj) is an index
 //    modulo 2N.
-//  * gather: one workgroup per (angle, slice) line; taps with separable
-//    weights exp(-beta*dx^2)*exp(-beta*dy^2); the 1D inverse DFT, the
-//    fftshift1c signs and the detector crop are fused in the same kernel.
+//  * The forward's buffers hold pairs of slices interleaved, so that a grid
+//    point or a polar sample of a pair is one 16-byte access.
+//  * gather: 8 x 8 Kaiser-Bessel taps (see below) from grid tiles staged in LDS.
 //  * scatter: deterministic and free of atomics.  At set_theta time every
 //    16 x 8 grid tile gets the list of polar samples whose 15 x 15
 //    footprint covers part of it (wrapadj folded into the periodic
@@ -39,7 +39,7 @@
 namespace {
 constexpr double kPiRef = 3.1415926535;  // kernels.cuh:1
 constexpr int kTile = 32;                // scatter tile edge (grid points)
-constexpr int kWorkMax = 1024;           // samples per gather work item
+constexpr int kWorkMax = 256;            // samples per gather work item
 }  // namespace
 
 struct pt_tomo {
@@ -48,14 +48,18 @@ struct pt_tomo {
   pt::LinePlan plan;
   float2* tw = nullptr;      // [N] exp(-2 pi i m/N)
   float2* twist = nullptr;   // [N] exp(-i pi j/N), j = idx - N/2
-  float* dphi = nullptr;     // [N] exp(mu a^2)/(2N), a = idx - N/2
+  float* dphi = nullptr;     // [N] forward: 1/(kernel's transform) at a/(2N), a = idx - N/2
+  float* dphia = nullptr;    // [N] adjoint: exp(mu a^2)/(2N)
   float* filt = nullptr;     // [N] detector-frequency filter of the adjoint, or null
   int2* mrange = nullptr;    // [N] circ mask column range [lo, hi) per row
   float2* spos = nullptr;    // [ntheta*N] sample positions (x, y)
   int2* sfloor = nullptr;    // [ntheta*N] floor(2N*x), floor(2N*y)
-  float2* A = nullptr;       // [pz][N][2N]
-  float2* Bg = nullptr;      // [pz][2N][2N]
-  float2* Q = nullptr;       // polar samples: fwd G[z][sample], adj Q[sample][z]
+  int2* ffloor = nullptr;    // [ntheta*N] the same of the exact products (forward)
+  float* wfwd = nullptr;     // [ntheta*N][16] gridding weights of the forward
+  // buffers of both directions (pz rounded up to whole slice pairs)
+  float2* A = nullptr;       // fwd [pz/2][N][2N][2], adj [pz][n][2N]
+  float2* Bg = nullptr;      // fwd [pz/2][2N][2N][2], adj [pz][2N][2N]
+  float2* Q = nullptr;       // polar samples: fwd [pz/2][sample][2], adj [sample][pz]
   // gather bins: samples by kTile x kTile tile of their floor position
   int ntile1 = 0;            // tiles per axis
   int* wi_tile = nullptr;    // [nwi] tile index
@@ -88,13 +92,15 @@ __device__ __forceinline__ int wrap2n(int v, int twoN) {
 
 // ------------------------------------------------------------------ forward row pass
 // For rows q of slice z: x[p] = mask*u[clamp]*dphi[q]*dphi[p] (pad2, circ,
-// divphi), centred 2N-point DFT along p -> A[z][q][kx], kx = k' + N.
+// divphi), centred 2N-point DFT along p -> A[z/2][q][kx][z%2], kx = k' + N.
+// (A last pair with one slice carries a copy of it in the other half.)
+// A workgroup takes `rows` of the pair's 2 N (row, slice) lines.
 __global__ __launch_bounds__(256) void k_row_fwd(float2* __restrict__ A, const float2* __restrict__ u,
                           const float2* __restrict__ tw, const float2* __restrict__ twist,
                           const float* __restrict__ dphi, const int2* __restrict__ mrange,
-                          LinePlan plan, int n, int rows) {
+                          LinePlan plan, int n, int rows, int pz) {
   extern __shared__ float2 lds[];
-  const int N = plan.N, z = blockIdx.y, q0 = blockIdx.x * rows;
+  const int N = plan.N, r0 = blockIdx.x * rows;
   const int o = N / 6;
   const int nl = 2 * rows;  // line 2r: plain, 2r+1: twisted
   float2* lb = lds + nl * (N + 1);  // ping-pong partner
@@ -102,7 +108,8 @@ __global__ __launch_bounds__(256) void k_row_fwd(float2* __restrict__ A, const f
   for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = tw[i];
   for (int i = threadIdx.x; i < nl * N; i += blockDim.x) {
     const int line = i / N, c = i - line * N;
-    const int r = line >> 1, q = q0 + r;
+    const int r = r0 + (line >> 1), q = r >> 1;
+    const int z = min(2 * (int)blockIdx.y + (r & 1), pz - 1);
     float2 val = make_float2(0.f, 0.f);
     if (q < N) {
       const int2 mr = mrange[q];
@@ -121,11 +128,11 @@ __global__ __launch_bounds__(256) void k_row_fwd(float2* __restrict__ A, const f
   const float2* res = lds_fft_pp<-1>(lds, lb, N + 1, nl, plan, twl, threadIdx.x, blockDim.x);
   for (int i = threadIdx.x; i < nl * N; i += blockDim.x) {
     const int line = i / N, b = i - line * N;
-    const int r = line >> 1, q = q0 + r;
+    const int r = r0 + (line >> 1), q = r >> 1;
     if (q >= N) continue;
     const int m = b < N / 2 ? b : b - N;  // centred frequency
     const int kx = 2 * m + N + (line & 1);
-    A[((long)z * N + q) * (2 * N) + kx] = res[line * (N + 1) + b];
+    A[(((long)blockIdx.y * N + q) * (2 * N) + kx) * 2 + (r & 1)] = res[line * (N + 1) + b];
   }
 }
 
@@ -133,8 +140,8 @@ __global__ __launch_bounds__(256) void k_row_fwd(float2* __restrict__ A, const f
 // Column tiles run in XCD-contiguous order (xcd_contig): neighbouring tiles
 // read the same cache lines of the rows (8 columns = 64 bytes per row).
 //
-// C = 2^lc columns kx of one slice per workgroup: y[q] = A[z][q][kx] ->
-// centred 2N-point DFT along q -> B[z][ky][kx], as the plain N-point DFT
+// C = 2^lc of the 4N columns (kx, slice) of one slice pair z per workgroup:
+// y[q] = A[z][q][kx] -> centred 2N-point DFT along q -> B[z][ky][kx], as the plain N-point DFT
 // (even ky - N) and the twisted one (odd ky - N) run one after the other in
 // the same C padded LDS lines (ping-pong pair).  The N x C tile stays in
 // registers between the two; the twiddle table is staged in LDS.
@@ -143,8 +150,8 @@ __global__ __launch_bounds__(256) void k_col_fwd(float2* __restrict__ Bg, const 
                           const float2* __restrict__ tw, const float2* __restrict__ twist,
                           LinePlan plan, int lc) {
   extern __shared__ float2 lds[];
-  const int N = plan.N, twoN = 2 * N, S = N + 1, C = 1 << lc;
-  const int gx = (twoN + C - 1) >> lc;
+  const int N = plan.N, W = 4 * N, S = N + 1, C = 1 << lc;  // W: columns of a slice pair
+  const int gx = (W + C - 1) >> lc;
   const int L = xcd_contig(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
   const int z = L / gx, k0 = (L - z * gx) << lc;
   float2* la = lds;
@@ -152,17 +159,17 @@ __global__ __launch_bounds__(256) void k_col_fwd(float2* __restrict__ Bg, const 
   float2* twl = lb + C * S;
   for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = tw[i];
   const int nv = (N * C + 255) >> 8;
-  const float2* Az = A + (long)z * N * twoN + k0;
+  const float2* Az = A + (long)z * N * W + k0;
   float2 reg[kColVpt];
 #pragma unroll
   for (int v = 0; v < kColVpt; ++v) {
     if (v < nv) {
       const int i = threadIdx.x + v * 256;
       const int q = i >> lc, cc = i & (C - 1);
-      reg[v] = (q < N && k0 + cc < twoN) ? Az[(long)q * twoN + cc] : make_float2(0.f, 0.f);
+      reg[v] = (q < N && k0 + cc < W) ? Az[(long)q * W + cc] : make_float2(0.f, 0.f);
     }
   }
-  float2* Bz = Bg + (long)z * twoN * twoN + k0;
+  float2* Bz = Bg + (long)z * (2 * N) * W + k0;
   for (int par = 0; par < 2; ++par) {
 #pragma unroll
     for (int v = 0; v < kColVpt; ++v) {
@@ -180,141 +187,134 @@ __global__ __launch_bounds__(256) void k_col_fwd(float2* __restrict__ Bg, const 
     const float2* res = lds_fft_pp<-1>(la, lb, S, C, plan, twl, threadIdx.x, blockDim.x);
     for (int i = threadIdx.x; i < N * C; i += blockDim.x) {
       const int r = i >> lc, cc = i & (C - 1);
-      if (k0 + cc >= twoN) continue;
+      if (k0 + cc >= W) continue;
       const int m = r - N / 2;  // ky - N = 2m + par
       const int b = m < 0 ? m + N : m;
-      Bz[(long)(2 * m + par + N) * twoN + cc] = res[cc * S + b];
+      Bz[(long)(2 * m + par + N) * W + cc] = res[cc * S + b];
     }
     __syncthreads();
   }
 }
 
+// ------------------------------------------------------------------ gridding kernel
+// Interpolation between the oversampled grid and the polar samples with the
+// Kaiser-Bessel kernel I0(beta sqrt(1 - (2d/w)^2)) / I0(beta) of width w = 8
+// grid points, beta = pi sqrt((w/s)^2 (s - 1/2)^2 - 0.8) for oversampling
+// s = 2 (Beatty, Nishimura and Pauly 2005); its Fourier transform
+// w sinh(r)/r / I0(beta), r = sqrt(beta^2 - (pi w xi)^2), is divided out of the
+// object points (dphi).  The reference's Gaussian with 15 x 15 taps
+// (kernels.cuh:97-158, eps = 1e-6) approximates the same nonuniform Fourier
+// sums: in 64 bits, on white-noise objects, it is 2.5e-7 from the direct sums,
+// this kernel with 8 x 8 taps 6e-8 (7 taps: 6e-7).
+constexpr int kW = 8;
+constexpr int kWLo = kW / 2 - 1;  // taps floor(x) - kWLo .. floor(x) + kW/2
+constexpr double kBeta = 18.638856593895362;
+
+__host__ __device__ inline double bessel_i0(double x) {
+  const double t = 0.25 * x * x;
+  double term = 1.0, sum = 1.0;
+#pragma unroll
+  for (int k = 1; k < 64; ++k) {
+    term *= t * (1.0 / ((double)k * k));
+    sum += term;
+  }
+  return sum;
+}
+// 1 / Fourier transform of the kernel at frequency xi (cycles per grid point)
+double kb_inverse_ft(double xi) {
+  const double a = kPi * kW * xi, r = std::sqrt(kBeta * kBeta - a * a);
+  return r * bessel_i0(kBeta) / (kW * std::sinh(r));
+}
+
+// Weights of all samples, FP64 rounded to FP32: w[s][0..7] of the columns
+// floor(G x) - 3 .. floor(G x) + 4, w[s][8..15] of the rows (y).
+__global__ __launch_bounds__(256) void k_kb_weights(float* __restrict__ w,
+                                                    const float2* __restrict__ spos, long ns,
+                                                    int G, double peak) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= ns * 2 * kW) return;
+  const int k = (int)(i % (2 * kW));
+  const float2 p = spos[i / (2 * kW)];
+  const double x = (double)G * (double)(k < kW ? p.x : p.y);
+  const double d = (floor(x) - kWLo + (k % kW) - x) / (kW / 2);
+  w[i] = (float)(bessel_i0(kBeta * sqrt(fmax(0.0, 1.0 - d * d))) / peak);
+}
+
 // ------------------------------------------------------------------ gather
-// One workgroup per (32 x 32 grid tile bin chunk, kGatherZ slice pairs): the
-// tile plus an M-point halo (periodic in 2N) is staged in LDS as
-// [y][x][z-pair]; each lane interpolates polar samples of the bin with
-// separable Gaussian weights (kernels.cuh:97-126).  Output G[z][sample].
-// The slice pairs are pipelined: the loads of pair j+1's tile are in flight
-// (registers) while pair j is interpolated from LDS, and the lane's sample
-// positions are loaded once for all pairs, so the interpolation issues no
-// global load that would wait behind the prefetch.
-constexpr int kGatherStage = 9;  // staged points per thread: (kTile + 14)^2 <= 2304
-constexpr int kGatherZ = 4;      // slice pairs per workgroup
-constexpr int kGatherSpl = kWorkMax / 256;  // samples per lane
-static_assert(kGatherSpl * 256 == kWorkMax, "a gather work item's samples fill whole lanes");
-__global__ __launch_bounds__(256) void k_gather_tile(float2* __restrict__ G,
-                                                     const float2* __restrict__ Bg,
-                                                     const float2* __restrict__ spos,
-                                                     const int2* __restrict__ sfloor,
-                                                     const int* __restrict__ wi_tile,
-                                                     const int2* __restrict__ wi_range,
-                                                     const int* __restrict__ bin_sample, int N,
-                                                     int M, float beta, int ntile1, int ns,
-                                                     int pz) {
-  extern __shared__ float4 lds4[];  // [E][E] pairs of complex (z, z+1)
-  const int twoN = 2 * N, E = kTile + 2 * M;
-  // XCD-contiguous order: adjacent tiles' staged regions overlap by 2M
+// One workgroup per (32 x 32 grid tile bin chunk, zper slice pairs): the
+// tile plus the footprint's halo (periodic in 2N) is staged in LDS as
+// [y][x][slice of the pair]; each lane interpolates its polar samples with
+// separable weights held in registers for all of the workgroup's pairs.
+// Output G[z/2][sample][z%2].  The loads of the next pair's tile are in flight
+// (registers) while a pair is interpolated from LDS.
+// Bound: LDS reads, 64 taps x 16 bytes per sample and slice pair (0.25 ms at
+// 256^3, 384 angles, at 128 bytes per cycle and CU), beside 1.5 GB of grid and
+// samples (0.3 ms): 0.38 ms per launch there, 1.44 ms with the 15 x 15
+// Gaussian taps; at 32^2 x 8 slices, 48 angles, 169 -> 8 us.  One sample per
+// lane: with two, the weights and the reads in flight took 211 registers (two
+// waves per SIMD, 0.54 ms); 512 lanes per workgroup measured 1 % slower.
+constexpr int kGE = kTile + kW - 1;                                // staged tile edge
+constexpr int kGatherStage = (kGE * kGE + kWorkMax - 1) / kWorkMax;  // staged points per lane
+typedef float f4v __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(kWorkMax, 4) void k_gather_tile(
+    f4v* __restrict__ G, const f4v* __restrict__ Bg, const f4v* __restrict__ wts,
+    const int2* __restrict__ sfloor, const int* __restrict__ wi_tile,
+    const int2* __restrict__ wi_range, const int* __restrict__ bin_sample, int N, int ntile1,
+    int ns, int npair, int zper) {
+  __shared__ f4v lds4[kGatherStage * kWorkMax];  // [y][x], then slots of the staging's last round
+  const int twoN = 2 * N;
+  // XCD-contiguous order: adjacent tiles' staged regions overlap
   const int lw = xcd_contig(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int zb = lw / gridDim.x;
   const int wi = lw - zb * gridDim.x;
-  const int npair = (pz + 1) / 2;
-  const int jp0 = zb * kGatherZ, jp1 = min(jp0 + kGatherZ, npair);
+  const int jp0 = zb * zper, jp1 = min(jp0 + zper, npair);
   const int tile = wi_tile[wi];
-  const int ty0 = (tile / ntile1) * kTile - N, tx0 = (tile % ntile1) * kTile - N;
+  const int ty0 = (tile / ntile1) * kTile, tx0 = (tile % ntile1) * kTile;
   const int2 rg = wi_range[wi];
-  // this lane's samples (at most kGatherSpl: rg.y - rg.x <= kWorkMax)
-  int sid[kGatherSpl];
-  float2 sp[kGatherSpl];
-  int2 sf[kGatherSpl];
+  // this lane's sample, its weights and its footprint's offset in the staged tile
+  const int bi = rg.x + threadIdx.x;
+  const int sid = bi < rg.y ? bin_sample[bi] : -1;
+  const int2 f = sfloor[max(sid, 0)];
+  const int off = sid < 0 ? 0 : (f.y + N - ty0) * kGE + f.x + N - tx0;
+  const f4v* wp = wts + (long)max(sid, 0) * (2 * kW / 4);
+  const f4v wx[2] = {wp[0], wp[1]}, wy[2] = {wp[2], wp[3]};
+  // grid offsets of this lane's staged points
+  int goff[kGatherStage];
 #pragma unroll
-  for (int q = 0; q < kGatherSpl; ++q) {
-    const int bi = rg.x + threadIdx.x + q * 256;
-    sid[q] = bi < rg.y ? bin_sample[bi] : -1;
+  for (int u = 0; u < kGatherStage; ++u) {
+    const int i = min((int)threadIdx.x + u * kWorkMax, kGE * kGE - 1);
+    const int y = i / kGE, x = i - y * kGE;
+    int gy = ty0 - kWLo + y, gx = tx0 - kWLo + x;
+    gy = gy < 0 ? gy + twoN : gy;
+    gx = gx < 0 ? gx + twoN : gx;
+    goff[u] = (gy % twoN) * twoN + gx % twoN;
   }
+  f4v va[kGatherStage];
+  const f4v* B = Bg + (long)jp0 * twoN * twoN;
 #pragma unroll
-  for (int q = 0; q < kGatherSpl; ++q) {
-    sp[q] = sid[q] >= 0 ? spos[sid[q]] : make_float2(0.f, 0.f);
-    sf[q] = sid[q] >= 0 ? sfloor[sid[q]] : make_int2(0, 0);
-  }
-  float2 va[kGatherStage], vb[kGatherStage];
-  auto load_pair = [&](int jp) {
-    const int z0 = 2 * jp;
-    const bool two = z0 + 1 < pz;
-    const float2* B0 = Bg + (long)z0 * twoN * twoN;
-    const float2* B1 = two ? B0 + (long)twoN * twoN : B0;
-#pragma unroll
-    for (int u = 0; u < kGatherStage; ++u) {
-      const int i = threadIdx.x + u * 256;
-      const int y = i / E, x = i - y * E;
-      const int gy = wrap2n(N + ty0 - M + y, twoN), gx = wrap2n(N + tx0 - M + x, twoN);
-      const long off = (long)gy * twoN + gx;
-      const bool in = i < E * E;
-      va[u] = in ? B0[off] : make_float2(0.f, 0.f);
-      vb[u] = in && two ? B1[off] : make_float2(0.f, 0.f);
-    }
-  };
-  load_pair(jp0);
-  const float inv2N = 1.0f / (float)twoN;
+  for (int u = 0; u < kGatherStage; ++u) va[u] = B[goff[u]];
   for (int jp = jp0; jp < jp1; ++jp) {
     __syncthreads();  // the previous pair's interpolation has read the tile
 #pragma unroll
-    for (int u = 0; u < kGatherStage; ++u) {
-      const int i = threadIdx.x + u * 256;
-      if (i < E * E) lds4[i] = make_float4(va[u].x, va[u].y, vb[u].x, vb[u].y);
-    }
+    for (int u = 0; u < kGatherStage; ++u) lds4[threadIdx.x + u * kWorkMax] = va[u];
     __syncthreads();
-    if (jp + 1 < jp1) load_pair(jp + 1);
-    const int z0 = 2 * jp;
-    const bool two = z0 + 1 < pz;
-    // the lane's samples in turn from slot 0, rotated once per sample (four
-    // rotations restore the order for the next pair; registers, no dynamic
-    // indexing)
-#pragma unroll 1
-    for (int q = 0; q < kGatherSpl; ++q) {
-      const int s = sid[0];
-      const float2 p = sp[0];
-      const int2 fl = sf[0];
+    if (jp + 1 < jp1) {
+      B += (long)twoN * twoN;
 #pragma unroll
-      for (int k = 0; k < kGatherSpl - 1; ++k) {
-        sid[k] = sid[k + 1];
-        sp[k] = sp[k + 1];
-        sf[k] = sf[k + 1];
-      }
-      sid[kGatherSpl - 1] = s;
-      sp[kGatherSpl - 1] = p;
-      sf[kGatherSpl - 1] = fl;
-      if (s < 0) continue;
-      float ex[15], ey[15];
-#pragma unroll
-      for (int k = 0; k < 15; ++k) {
-        const float dx = (float)(fl.x - M + k) * inv2N - p.x;
-        const float dy = (float)(fl.y - M + k) * inv2N - p.y;
-        ex[k] = (k <= 2 * M) ? __expf(-beta * dx * dx) : 0.f;
-        ey[k] = (k <= 2 * M) ? __expf(-beta * dy * dy) : 0.f;
-      }
-      const int row = fl.y - ty0, col = fl.x - tx0;  // footprint origin in the staged tile
-      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int k1 = 0; k1 <= 2 * M; ++k1) {
-        const float4* rp = lds4 + (row + k1) * E + col;
-        float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int k0 = 0; k0 < 15; ++k0) {
-          if (k0 <= 2 * M) {
-            const float4 v = rp[k0];
-            r.x += ex[k0] * v.x;
-            r.y += ex[k0] * v.y;
-            r.z += ex[k0] * v.z;
-            r.w += ex[k0] * v.w;
-          }
-        }
-        acc.x += ey[k1] * r.x;
-        acc.y += ey[k1] * r.y;
-        acc.z += ey[k1] * r.z;
-        acc.w += ey[k1] * r.w;
-      }
-      G[(long)z0 * ns + s] = make_float2(acc.x, acc.y);
-      if (two) G[(long)(z0 + 1) * ns + s] = make_float2(acc.z, acc.w);
+      for (int u = 0; u < kGatherStage; ++u) va[u] = B[goff[u]];
     }
+    if (sid < 0) continue;
+    const f4v* rp = lds4 + off;
+    f4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k1 = 0; k1 < kW; ++k1) {
+      f4v r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k0 = 0; k0 < kW; ++k0) r += wx[k0 / 4][k0 % 4] * rp[k1 * kGE + k0];
+      acc += wy[k1 / 4][k1 % 4] * r;
+      __builtin_amdgcn_sched_barrier(0);  // one row's reads in flight per wave: no spills
+    }
+    G[(long)jp * ns + sid] = acc;
   }
 }
 
@@ -335,7 +335,8 @@ __global__ __launch_bounds__(256) void k_line_idft(float2* __restrict__ g, const
     int a = k - N / 2;  // kappa -> kappa mod N
     if (a < 0) a += N;
     lds[zz * (N + 1) + a] =
-        zz < nzl ? G[(long)(z0 + zz) * ntheta * N + (long)th * N + k] : make_float2(0.f, 0.f);
+        zz < nzl ? G[(((long)((z0 + zz) >> 1) * ntheta + th) * N + k) * 2 + ((z0 + zz) & 1)]
+                 : make_float2(0.f, 0.f);
   }
   __syncthreads();
   const float2* res = lds_fft_pp<1>(lds, lb, N + 1, zq, plan, twl, threadIdx.x, blockDim.x);
@@ -679,21 +680,24 @@ constexpr size_t reg_lds_bytes() {
   return sizeof(float2) * ((size_t)(nt_of<N>() / LineReg<N>::T) * (N + 1) + N);
 }
 
-// forward row pass: rows q of slice z, lines (2 r + par); lane = par + 2 (t + T r)
+// forward row pass: rows q of slice pair z, lines (r, parity, slice); lane =
+// slice + 2 (par + 2 (t + T r))
 template <int N>
 __global__ __launch_bounds__(kNT) void k_row_fwd_r(float2* __restrict__ A,
                                                    const float2* __restrict__ u,
                                                    const float2* __restrict__ tw,
                                                    const float2* __restrict__ twist,
                                                    const float* __restrict__ dphi,
-                                                   const int2* __restrict__ mrange, int n) {
-  constexpr int P = kLineP, H = P / 2, T = LineReg<N>::T, NL = nt_of<N>() / T, ROWS = NL / 2,
+                                                   const int2* __restrict__ mrange, int n,
+                                                   int pz) {
+  constexpr int P = kLineP, H = P / 2, T = LineReg<N>::T, NL = nt_of<N>() / T, ROWS = NL / 4,
                 o = N / 6;
   extern __shared__ float2 lds[];
   float2* twl = lds + NL * (N + 1);
   stage_twiddles<N>(twl, tw);
-  const int tid = threadIdx.x, par = tid & 1, t = (tid >> 1) % T, r = tid / (2 * T);
-  const int z = blockIdx.y, q = blockIdx.x * ROWS + r;
+  const int tid = threadIdx.x, zz = tid & 1, par = (tid >> 1) & 1, t = (tid >> 2) % T,
+            r = tid / (4 * T);
+  const int z = min(2 * (int)blockIdx.y + zz, pz - 1), q = blockIdx.x * ROWS + r;
   const bool rowok = q < N;
   const int2 mr = rowok ? mrange[q] : make_int2(0, 0);
   const float dq = rowok ? dphi[q] : 0.f;
@@ -713,36 +717,37 @@ __global__ __launch_bounds__(kNT) void k_row_fwd_r(float2* __restrict__ A,
     v[m] = (c >= mr.x && c < mr.y) ? (par ? xt : x) : make_float2(0.f, 0.f);
   });
   __syncthreads();
-  line_reg_fft<N, -1>(v, lds + (2 * r + par) * (N + 1), twl, t);
+  line_reg_fft<N, -1>(v, lds + (4 * r + 2 * zz + par) * (N + 1), twl, t);
   if (!rowok) return;
-  float2* Ar = A + ((long)z * N + q) * (2 * N);
+  float2* Ar = A + ((long)blockIdx.y * N + q) * (4 * N) + 2 * par + zz;
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const int b = t + T * m;
-    Ar[(m < H ? 2 * b + N : 2 * b - N) + par] = v[m];
+    Ar[2 * (m < H ? 2 * b + N : 2 * b - N)] = v[m];
   });
 }
 
-// forward column pass: C = NT / (2T) columns, lines (par C + cc); lane = cc + C (par + 2 t)
+// forward column pass: C = NT / (2T) of the 4N columns (kx, slice) of slice
+// pair z, lines (par C + cc); lane = cc + C (par + 2 t)
 template <int N>
 __global__ __launch_bounds__(kNT) void k_col_fwd_r(float2* __restrict__ Bg,
                                                    const float2* __restrict__ A,
                                                    const float2* __restrict__ tw,
                                                    const float2* __restrict__ twist) {
-  constexpr int P = kLineP, H = P / 2, T = LineReg<N>::T, C = nt_of<N>() / (2 * T),
-                twoN = 2 * N, gx = twoN / C;
-  static_assert(twoN % C == 0, "column tiles");
+  constexpr int P = kLineP, H = P / 2, T = LineReg<N>::T, C = nt_of<N>() / (2 * T), W = 4 * N,
+                gx = W / C;
+  static_assert(W % C == 0, "column tiles");
   extern __shared__ float2 lds[];
   float2* twl = lds + 2 * C * (N + 1);
   stage_twiddles<N>(twl, tw);
   const int tid = threadIdx.x, cc = tid % C, par = (tid / C) & 1, t = tid / (2 * C);
   const int L = xcd_contig(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
   const int z = L / gx, k0 = (L - z * gx) * C;
-  const float2* Az = A + (long)z * N * twoN + k0 + cc;
+  const float2* Az = A + (long)z * N * W + k0 + cc;
   float2 v[P];
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
-    v[m] = Az[(long)(t + T * ((m + H) % P)) * twoN];
+    v[m] = Az[(long)(t + T * ((m + H) % P)) * W];
   });
   if (par) {
     static_for<0, P>([&](auto mc) {
@@ -752,15 +757,15 @@ __global__ __launch_bounds__(kNT) void k_col_fwd_r(float2* __restrict__ Bg,
   }
   __syncthreads();
   line_reg_fft<N, -1>(v, lds + (par * C + cc) * (N + 1), twl, t);
-  float2* Bz = Bg + (long)z * twoN * twoN + k0 + cc;
+  float2* Bz = Bg + (long)z * (2 * N) * W + k0 + cc;
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const int b = t + T * m;
-    Bz[(long)((m < H ? 2 * b + N : 2 * b - N) + par) * twoN] = v[m];
+    Bz[(long)((m < H ? 2 * b + N : 2 * b - N) + par) * W] = v[m];
   });
 }
 
-// forward detector lines: ZQ = NT / T slices of angle th; lane = t + T zz
+// forward detector lines: ZQ = NT / T slices of angle th; lane = zz%2 + 2 (t + T (zz/2))
 template <int N>
 __global__ __launch_bounds__(kNT) void k_line_idft_r(float2* __restrict__ g,
                                                      const float2* __restrict__ G,
@@ -771,14 +776,14 @@ __global__ __launch_bounds__(kNT) void k_line_idft_r(float2* __restrict__ g,
   extern __shared__ float2 lds[];
   float2* twl = lds + ZQ * (N + 1);
   stage_twiddles<N>(twl, tw);
-  const int tid = threadIdx.x, t = tid % T, zz = tid / T;
-  const int th = blockIdx.x, z = blockIdx.y * ZQ + zz;
+  const int tid = threadIdx.x, t = (tid >> 1) % T, zz = 2 * (tid / (2 * T)) + (tid & 1);
+  const int th = blockIdx.x, z = blockIdx.y * ZQ + zz, zc = min(z, pz - 1);
   const bool ok = z < pz;
-  const float2* Gl = G + (long)min(z, pz - 1) * ntheta * N + (long)th * N;
+  const float2* Gl = G + (((long)(zc >> 1) * ntheta + th) * N) * 2 + (zc & 1);
   float2 v[P];
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
-    v[m] = Gl[t + T * ((m + H) % P)];  // row clamped: a lane past pz transforms a copy
+    v[m] = Gl[2 * (t + T * ((m + H) % P))];  // row clamped: a lane past pz transforms a copy
   });
   __syncthreads();
   line_reg_fft<N, 1>(v, lds + zz * (N + 1), twl, t);
@@ -969,17 +974,18 @@ int with_reg_n(int N, F&& fn) {
 
 template <int N>
 int fwd_grid_r(pt_tomo* h, const float2* f, hipStream_t st) {
-  constexpr int T = LineReg<N>::T, ROWS = nt_of<N>() / (2 * T), C = nt_of<N>() / (2 * T);
+  constexpr int T = LineReg<N>::T, ROWS = nt_of<N>() / (4 * T), C = nt_of<N>() / (2 * T);
   constexpr size_t lds = reg_lds_bytes<N>();
+  const int npair = (h->pz + 1) / 2;
   {
     ProfScope prof("tomo_row_fwd", st);
-    hipLaunchKernelGGL(k_row_fwd_r<N>, dim3((N + ROWS - 1) / ROWS, h->pz), dim3(nt_of<N>()), lds,
-                       st, h->A, f, h->tw, h->twist, h->dphi, h->mrange, h->n);
+    hipLaunchKernelGGL(k_row_fwd_r<N>, dim3((N + ROWS - 1) / ROWS, npair), dim3(nt_of<N>()), lds,
+                       st, h->A, f, h->tw, h->twist, h->dphi, h->mrange, h->n, h->pz);
     PT_LAUNCH_CHECK();
   }
   {
     ProfScope prof("tomo_col_fwd", st);
-    hipLaunchKernelGGL(k_col_fwd_r<N>, dim3(2 * N / C, h->pz), dim3(nt_of<N>()), lds, st, h->Bg, h->A,
+    hipLaunchKernelGGL(k_col_fwd_r<N>, dim3(4 * N / C, npair), dim3(nt_of<N>()), lds, st, h->Bg, h->A,
                        h->tw, h->twist);
     PT_LAUNCH_CHECK();
   }
@@ -1019,14 +1025,14 @@ int adj_grid_r(pt_tomo* h, float2* f, float scale, hipStream_t st) {
   {
     ProfScope prof("tomo_row_adj", st);
     hipLaunchKernelGGL(k_row_adj_r<N>, dim3((h->n + ROWS - 1) / ROWS, h->pz), dim3(nt_of<N>()), lds, st,
-                       f, h->A, h->tw, h->twist, h->dphi, h->mrange, scale);
+                       f, h->A, h->tw, h->twist, h->dphia, h->mrange, scale);
     PT_LAUNCH_CHECK();
   }
   return PT_OK;
 }
 
 int run_fwd(pt_tomo* h, float2* g, const float2* f, float scale, hipStream_t st) {
-  const int N = h->N;
+  const int N = h->N, npair = (h->pz + 1) / 2;
   const int nthr = 256;
   const bool rl = reg_lines(h);
   if (rl) {
@@ -1035,34 +1041,37 @@ int run_fwd(pt_tomo* h, float2* g, const float2* f, float scale, hipStream_t st)
   }
   if (!rl) {
     const int rows = h->rows_per_wg;
-    dim3 grid((N + rows - 1) / rows, h->pz);
+    dim3 grid((2 * N + rows - 1) / rows, npair);
     size_t lds = line_lds_bytes(N, 2 * rows);
     ProfScope prof("tomo_row_fwd", st);
     hipLaunchKernelGGL(k_row_fwd, grid, dim3(nthr), lds, st, h->A, f, h->tw, h->twist, h->dphi,
-                       h->mrange, h->plan, h->n, rows);
+                       h->mrange, h->plan, h->n, rows, h->pz);
     PT_LAUNCH_CHECK();
   }
   if (!rl) {
     const int cols = h->cols_per_wg;
-    dim3 grid((2 * N + cols - 1) / cols, h->pz);
+    dim3 grid((4 * N + cols - 1) / cols, npair);
     ProfScope prof("tomo_col_fwd", st);
     hipLaunchKernelGGL(k_col_fwd, grid, dim3(nthr), col_lds_bytes(N, cols), st, h->Bg, h->A, h->tw,
                        h->twist, h->plan, ilog2(cols));
     PT_LAUNCH_CHECK();
   }
   {
-    const float beta = (float)(kPiRef * kPiRef / (double)h->mu);
-    const int E = kTile + 2 * h->M;
-    dim3 grid(h->nwi, ((h->pz + 1) / 2 + kGatherZ - 1) / kGatherZ);
+    // slice pairs per workgroup: up to 8, so that the next pair's loads overlap
+    // the interpolation, but fewer where that leaves under 2048 workgroups
+    // (8 per CU)
+    int zper = 8;
+    while (zper > 1 && (long)h->nwi * ((npair + zper - 1) / zper) < 2048) zper /= 2;
+    dim3 grid(h->nwi, (npair + zper - 1) / zper);
     ProfScope prof("tomo_gather", st);
-    hipLaunchKernelGGL(k_gather_tile, grid, dim3(256), sizeof(float4) * E * E, st, h->Q, h->Bg,
-                       h->spos, h->sfloor, h->wi_tile, h->wi_range, h->bin_sample, N, h->M, beta,
-                       h->ntile1, h->ntheta * N, h->pz);
+    hipLaunchKernelGGL(k_gather_tile, grid, dim3(kWorkMax), 0, st, (f4v*)h->Q, (const f4v*)h->Bg,
+                       (const f4v*)h->wfwd, h->ffloor, h->wi_tile, h->wi_range, h->bin_sample, N,
+                       h->ntile1, h->ntheta * N, npair, zper);
     PT_LAUNCH_CHECK();
   }
   {
     const double sgn = ((N / 2) % 2) ? -1.0 : 1.0;
-    const float oscale = (float)(sgn * kPiRef / (double)h->mu / (double)N * (double)scale);
+    const float oscale = (float)(sgn / (double)N * (double)scale);
     if (rl) return with_reg_n(N, [&](auto nc) { return fwd_lines_r<decltype(nc)::value>(h, g, oscale, st); });
     const int zq = h->adj_lines;    // detector lines per workgroup (fits the LDS FFT)
     dim3 grid(h->ntheta, (h->pz + zq - 1) / zq);
@@ -1125,7 +1134,7 @@ int run_adj(pt_tomo* h, float2* f, const float2* g, float scale, hipStream_t st)
     dim3 grid((h->n + rows - 1) / rows, h->pz);
     size_t lds = line_lds_bytes(N, 2 * rows);
     ProfScope prof("tomo_row_adj", st);
-    hipLaunchKernelGGL(k_row_adj, grid, dim3(nthr), lds, st, f, h->A, h->tw, h->twist, h->dphi,
+    hipLaunchKernelGGL(k_row_adj, grid, dim3(nthr), lds, st, f, h->A, h->tw, h->twist, h->dphia,
                        h->mrange, h->plan, h->n, rows, scale);
     PT_LAUNCH_CHECK();
   }
@@ -1203,7 +1212,7 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
   h->adj_lines = lines_fit(plan, kZQ, cap);
   // host tables
   std::vector<float2> tw(N), twist(N);
-  std::vector<float> dphi(N);
+  std::vector<float> dphi(N), dphia(N);
   std::vector<int2> mr(N);
   for (int m = 0; m < N; ++m) {
     double a = -2.0 * kPi * m / N;
@@ -1211,7 +1220,8 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
     const int j = m - N / 2;
     double b = -kPi * j / N;
     twist[m] = make_float2((float)std::cos(b), (float)std::sin(b));
-    dphi[m] = (float)(std::exp((double)h->mu * (double)j * (double)j) / (2.0 * N));
+    dphi[m] = (float)kb_inverse_ft((double)j / (2.0 * N));
+    dphia[m] = (float)(std::exp((double)h->mu * (double)j * (double)j) / (2.0 * N));
   }
   // circ mask (kernels.cuh:160-172), float32 arithmetic without contraction
   for (int q = 0; q < N; ++q) {
@@ -1242,16 +1252,21 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
   if ((e = hipMalloc(&h->tw, sizeof(float2) * N))) return fail(e, "tables");
   if ((e = hipMalloc(&h->twist, sizeof(float2) * N))) return fail(e, "tables");
   if ((e = hipMalloc(&h->dphi, sizeof(float) * N))) return fail(e, "tables");
+  if ((e = hipMalloc(&h->dphia, sizeof(float) * N))) return fail(e, "tables");
   if ((e = hipMalloc(&h->mrange, sizeof(int2) * N))) return fail(e, "tables");
   if ((e = hipMalloc(&h->spos, sizeof(float2) * (size_t)ntheta * N))) return fail(e, "positions");
   if ((e = hipMalloc(&h->sfloor, sizeof(int2) * (size_t)ntheta * N))) return fail(e, "positions");
+  if ((e = hipMalloc(&h->ffloor, sizeof(int2) * (size_t)ntheta * N))) return fail(e, "positions");
   if ((e = hipMalloc(&h->bin_sample, sizeof(int) * (size_t)ntheta * N))) return fail(e, "bins");
-  if ((e = hipMalloc(&h->A, sizeof(float2) * (size_t)pnz * N * 2 * N))) return fail(e, "row buffer");
-  if ((e = hipMalloc(&h->Bg, sizeof(float2) * (size_t)pnz * 4 * N * N))) return fail(e, "grid");
-  if ((e = hipMalloc(&h->Q, sizeof(float2) * (size_t)pnz * ntheta * N))) return fail(e, "samples");
+  if ((e = hipMalloc(&h->wfwd, sizeof(float) * 2 * kW * (size_t)ntheta * N))) return fail(e, "weights");
+  const size_t pzp = (size_t)(pnz + 1) / 2 * 2;
+  if ((e = hipMalloc(&h->A, sizeof(float2) * pzp * N * 2 * N))) return fail(e, "row buffer");
+  if ((e = hipMalloc(&h->Bg, sizeof(float2) * pzp * 4 * N * N))) return fail(e, "grid");
+  if ((e = hipMalloc(&h->Q, sizeof(float2) * pzp * ntheta * N))) return fail(e, "samples");
   if ((e = hipMemcpy(h->tw, tw.data(), sizeof(float2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->twist, twist.data(), sizeof(float2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->dphi, dphi.data(), sizeof(float) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
+  if ((e = hipMemcpy(h->dphia, dphia.data(), sizeof(float) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->mrange, mr.data(), sizeof(int2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   *out = h;
   return PT_OK;
@@ -1277,8 +1292,8 @@ static int upload(T** dst, const std::vector<T>& v, hipStream_t st) {
 
 extern "C" int pt_tomo_destroy(pt_tomo* h) {
   if (!h) return PT_OK;
-  (void)hipFree(h->tw); (void)hipFree(h->twist); (void)hipFree(h->dphi); (void)hipFree(h->filt); (void)hipFree(h->mrange);
-  (void)hipFree(h->spos); (void)hipFree(h->sfloor); (void)hipFree(h->A); (void)hipFree(h->Bg); (void)hipFree(h->Q);
+  (void)hipFree(h->tw); (void)hipFree(h->twist); (void)hipFree(h->dphi); (void)hipFree(h->dphia); (void)hipFree(h->wfwd); (void)hipFree(h->filt); (void)hipFree(h->mrange);
+  (void)hipFree(h->spos); (void)hipFree(h->sfloor); (void)hipFree(h->ffloor); (void)hipFree(h->A); (void)hipFree(h->Bg); (void)hipFree(h->Q);
   (void)hipFree(h->bin_sample);
   free_bins(h);
   delete h;
@@ -1295,7 +1310,7 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   // takexy (kernels.cuh:84-95): FP64 then float32, clamp at 0.5
   const long ns = (long)nt * N;
   std::vector<float2> pos(ns);
-  std::vector<int2> fl(ns);
+  std::vector<int2> fl(ns), ff(ns);  // ff: exact floors, as the weights' (k_kb_weights)
   const float lim = (float)(0.5 - 1e-5);
   const float twoN = (float)(2 * N);
   for (int t = 0; t < nt; ++t) {
@@ -1309,6 +1324,8 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
       volatile float px = twoN * x, py = twoN * y;
       pos[(long)t * N + i] = make_float2(x, y);
       fl[(long)t * N + i] = make_int2((int)std::floor(px), (int)std::floor(py));
+      ff[(long)t * N + i] =
+          make_int2((int)std::floor(2.0 * N * x), (int)std::floor(2.0 * N * y));
     }
   }
   for (long q = 0; q < ns; ++q) {
@@ -1324,19 +1341,19 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   const long ntiles = (long)nt1 * nt1;
   std::vector<int> cnt(ntiles + 1, 0);
   for (long q = 0; q < ns; ++q)
-    cnt[(long)((fl[q].y + N) / kTile) * nt1 + (fl[q].x + N) / kTile + 1]++;
+    cnt[(long)((ff[q].y + N) / kTile) * nt1 + (ff[q].x + N) / kTile + 1]++;
   for (long i = 0; i < ntiles; ++i) cnt[i + 1] += cnt[i];
   std::vector<int> fillp(cnt.begin(), cnt.end() - 1), list(ns);
   for (long q = 0; q < ns; ++q)
-    list[fillp[(long)((fl[q].y + N) / kTile) * nt1 + (fl[q].x + N) / kTile]++] = (int)q;
+    list[fillp[(long)((ff[q].y + N) / kTile) * nt1 + (ff[q].x + N) / kTile]++] = (int)q;
   // within a bin, samples in row-major order of their floor position: the
   // lanes of a wavefront then read neighbouring LDS words for each tap (few
   // bank conflicts); each lane still computes its own sample, so the order
   // does not change any result
   for (long tI = 0; tI < ntiles; ++tI)
     std::sort(list.begin() + cnt[tI], list.begin() + cnt[tI + 1], [&](int a, int b) {
-      if (fl[a].y != fl[b].y) return fl[a].y < fl[b].y;
-      if (fl[a].x != fl[b].x) return fl[a].x < fl[b].x;
+      if (ff[a].y != ff[b].y) return ff[a].y < ff[b].y;
+      if (ff[a].x != ff[b].x) return ff[a].x < ff[b].x;
       return a < b;
     });
   std::vector<int> wtile;
@@ -1348,7 +1365,6 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   // lanes on distinct 32-bank sets).  Row-major order put neighbouring lanes a
   // few float4 apart, i.e. on overlapping banks.  Each lane still computes its
   // own samples, so the order changes no result.
-  const int E = kTile + 2 * M;
   std::vector<int> bucket[16];
   for (long tI = 0; tI < ntiles; ++tI)
     for (int s0 = cnt[tI]; s0 < cnt[tI + 1]; s0 += kWorkMax) {
@@ -1356,8 +1372,8 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
       const int ty0 = (int)(tI / nt1) * kTile - N, tx0 = (int)(tI % nt1) * kTile - N;
       for (auto& b : bucket) b.clear();
       for (int i = s0; i < s1; ++i) {
-        const int2 f = fl[list[i]];
-        bucket[((f.y - ty0) * E + (f.x - tx0)) & 15].push_back(list[i]);
+        const int2 f = ff[list[i]];
+        bucket[((f.y - ty0) * kGE + (f.x - tx0)) & 15].push_back(list[i]);
       }
       int at = s0;
       for (size_t r = 0; at < s1; ++r)
@@ -1438,7 +1454,11 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
                    sizeof(float2) * (size_t)std::max(nslots, 1) * h->pz * kTSY * kTSX));
   PT_HIP(hipMemcpyAsync(h->spos, pos.data(), sizeof(float2) * ns, hipMemcpyHostToDevice, st));
   PT_HIP(hipMemcpyAsync(h->sfloor, fl.data(), sizeof(int2) * ns, hipMemcpyHostToDevice, st));
+  PT_HIP(hipMemcpyAsync(h->ffloor, ff.data(), sizeof(int2) * ns, hipMemcpyHostToDevice, st));
   PT_HIP(hipMemcpyAsync(h->bin_sample, list.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_kb_weights, dim3((unsigned)((ns * 2 * kW + 255) / 256)), dim3(256), 0, st,
+                     h->wfwd, h->spos, ns, 2 * N, bessel_i0(kBeta));
+  PT_LAUNCH_CHECK();
   PT_HIP(hipStreamSynchronize(st));
   h->ntile1 = nt1;
   h->nwi = (int)wtile.size();

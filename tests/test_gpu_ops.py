@@ -153,6 +153,31 @@ def test_tomo_large_vs_direct_nudft(n):
     assert err < 1e-5, err
 
 
+@pytest.mark.parametrize("n,pz", [(4, 1), (8, 3), (20, 2), (36, 1), (60, 5), (64, 17), (100, 1),
+                                  (128, 3)])
+def test_tomo_fwd_vs_direct_sums(n, pz):
+    """The forward against the FP64 direct nonuniform DFT, at sizes around the
+    edges of the gridding kernel: a grid smaller than a tile and its halo,
+    partial last tiles, odd slice counts, angles on the grid axes (integer
+    sample positions).  Tolerance: the gridding kernel's 1e-7 plus a few ulp
+    per FFT pass over three transforms, under 1e-6."""
+    from ptychotomo_amd.radonusfft import radonusfft
+    print(f"tomo forward direct sums n={n} pz={pz}", flush=True)
+    rng = np.random.default_rng(n + pz)
+    theta = np.concatenate([[0, np.pi / 4, np.pi / 2, np.pi], rng.uniform(0, np.pi, 3)])
+    theta = theta.astype(np.float32)
+    u = crandn(rng, (pz, n, n))
+    op = radonusfft(theta.size, pz, n)
+    th = dev(theta)
+    op.setobj(th.data_ptr())
+    out = torch.zeros((theta.size, pz, n), dtype=torch.complex64, device="cuda")
+    ud = dev(u)
+    op.fwd(out.data_ptr(), ud.data_ptr())
+    err = rel(out.cpu().numpy(), ousfft.fwd_exact(u, theta))
+    print(f"rel {err:.2e}")
+    assert err < 1e-6, err
+
+
 def test_tomo_adjoint_zero_border():
     """With a zero object border and zero detector edges the boundary pads
     vanish and the operator pair is exactly adjoint."""
