@@ -366,8 +366,8 @@ __device__ inline float2* lds_fft_pp(float2* a, float2* b, int stride, int nline
 }
 
 // ---------------------------------------------------------------- register line FFT
-// Unnormalised DFT of R points in registers, R = 2^a or 3 x 2^a (a <= 3):
-// 2, 4, 8 (dft_ct), 3 (dft3), 6, 12, 24 as decimation in time R = 3 x B:
+// Unnormalised DFT of R points in registers, R = 2^a (a <= 4) or 3 x 2^a (a <= 3):
+// 2, 4, 8 (dft_ct), 16 (reg_fft), 3 (dft3), 6, 12, 24 as decimation in time R = 3 x B:
 //   X[k1 + 3 k2] = sum_n2 W_B^(n2 k2) W_R^(n2 k1) sum_n1 x[B n1 + n2] W_3^(n1 k1).
 template <int R, int SIGN>
 __device__ __forceinline__ void dft_r(float2* a);
@@ -404,6 +404,11 @@ __device__ __forceinline__ void dft_r(float2* a) {
     dft3<SIGN>(a);
   } else if constexpr (R == 2 || R == 4 || R == 8) {
     dft_ct<R, SIGN>(a);
+  } else if constexpr (R == 16) {
+    float2 v[16];
+    static_for<0, 16>([&](auto c) { v[decltype(c)::value] = a[decltype(c)::value]; });
+    reg_fft<16, SIGN>(v);
+    static_for<0, 16>([&](auto c) { a[decltype(c)::value] = v[decltype(c)::value]; });
   } else {
     static_assert(R == 6 || R == 12 || R == 24, "radix");
     dft_3b<R / 3, SIGN>(a);
@@ -419,28 +424,30 @@ constexpr int ilog2_ct(int v) {
   return e;
 }
 
-// Points per lane of the register line FFT (24 or 12) and the workgroup size
-// of its kernels (the same number of lines per workgroup either way).
+// Points per lane of the register line FFT for lines of 3n/2 points and the
+// workgroup size of its kernels; lines of n = 2^e points take 16 per lane.
 constexpr int kLineP = 24;
 constexpr int kLineThreads = 6144 / kLineP;
 
-// Compile-time plan of an N-point line FFT held P = kLineP points per lane by
+// Compile-time plan of an N-point line FFT held P points per lane by
 // T = N / P lanes: lane t holds the points at positions t + T m, m < P, in
-// registers.  Stockham passes of radices that divide P = 3 x 2^a (each lane
-// then does P / R whole butterflies per pass and reads its inputs from the
-// positions it holds): the factors 3 one per pass from the first, a factors
-// 2 per pass from the last, the rest of the 2s in the first pass; with
-// P = 24: N = 384: 6, 8, 8; 768: 12, 8, 8; 192: 3, 8, 8; 96: 12, 8.
-template <int N>
+// registers.  Stockham passes of radices that divide P (24 = 3 x 2^3, or 16;
+// each lane then does P / R whole butterflies per pass and reads its inputs
+// from the positions it holds): the factors 3 one per pass from the first, a
+// factors 2 per pass from the last, the rest of the 2s in the first pass; with
+// P = 24: N = 384: 6, 8, 8; 768: 12, 8, 8; 192: 3, 8, 8; 96: 12, 8; with
+// P = 16: N = 64: 4, 16; 128: 8, 16; 256: 16, 16; 512: 2, 16, 16.
+template <int N, int P_ = kLineP>
 struct LineReg {
-  static constexpr int P = kLineP;
-  static_assert(P == 24 || P == 12, "register line FFT: 24 or 12 points per lane");
+  static constexpr int P = P_;
+  static_assert(P == 24 || P == 16, "register line FFT: 24 or 16 points per lane");
   static_assert(N % P == 0 && N % 27 != 0, "register line FFT: N = P T with at most 3^2");
   static constexpr int T = N / P;
-  static constexpr int amax = ilog2_ct(P / 3);
-  static constexpr int n3 = (N % 9 == 0) ? 2 : 1;
-  static constexpr int e = ilog2_ct(N / (n3 == 2 ? 9 : 3));
-  static_assert((N / (n3 == 2 ? 9 : 3)) == (1 << e), "register line FFT: N = 3^b 2^e");
+  static constexpr int amax = P == 16 ? 4 : 3;
+  static constexpr int n3 = (N % 9 == 0) ? 2 : (N % 3 == 0) ? 1 : 0;
+  static constexpr int m3 = n3 == 2 ? 9 : n3 == 1 ? 3 : 1;
+  static constexpr int e = ilog2_ct(N / m3);
+  static_assert((N / m3) == (1 << e), "register line FFT: N = 3^b 2^e");
   static constexpr int np = n3 > (e + amax - 1) / amax ? n3 : (e + amax - 1) / amax;
   static constexpr int radix(int p) {
     return (p < n3 ? 3 : 1) << (p == 0 ? e - amax * (np - 1) : amax);
@@ -458,10 +465,10 @@ struct LineReg {
 // radix-R DFT.  An inner pass stores its outputs at Stockham positions
 // (j div Ns) Ns R + k + Ns i in ln; the last pass (Ns R = N) puts output i
 // back at position j + (N/R) i, i.e. in place in the registers.
-template <int N, int SIGN, int p>
-__device__ __forceinline__ void line_reg_pass(float2 (&v)[kLineP], float2* __restrict__ ln,
+template <int N, int SIGN, int p, int P>
+__device__ __forceinline__ void line_reg_pass(float2 (&v)[P], float2* __restrict__ ln,
                                               const float2* __restrict__ tw, int t) {
-  using L = LineReg<N>;
+  using L = LineReg<N, P>;
   constexpr int R = L::radix(p), Ns = L::ns(p), B = L::P / R, T = L::T;
   static_for<0, B>([&](auto bc) {
     constexpr int b = decltype(bc)::value;
@@ -491,13 +498,13 @@ __device__ __forceinline__ void line_reg_pass(float2 (&v)[kLineP], float2* __res
 // Every lane of the workgroup calls it together: the LDS exchanges between
 // passes end with a barrier each, and the caller's LDS writes before the
 // call (e.g. the twiddle table) must be behind a barrier already.
-template <int N, int SIGN>
-__device__ __forceinline__ void line_reg_fft(float2 (&v)[kLineP], float2* __restrict__ ln,
+template <int N, int SIGN, int P>
+__device__ __forceinline__ void line_reg_fft(float2 (&v)[P], float2* __restrict__ ln,
                                              const float2* __restrict__ tw, int t) {
-  using L = LineReg<N>;
+  using L = LineReg<N, P>;
   static_for<0, L::np>([&](auto pc) {
     constexpr int p = decltype(pc)::value;
-    line_reg_pass<N, SIGN, p>(v, ln, tw, t);
+    line_reg_pass<N, SIGN, p, P>(v, ln, tw, t);
     if constexpr (p < L::np - 1) {
       __syncthreads();
       static_for<0, L::P>([&](auto mc) {

@@ -16,20 +16,20 @@
 //    exchanges between passes), otherwise LDS transforms with a run-time
 //    mixed-radix plan (2/3/4/5/8).
 //  * pad2 + circ + divphi are applied while loading the object rows; the
-//    adjoint's unpaddivphi + circ + crop are applied while storing them, and
-//    only the n object rows are transformed.
+//    adjoint's unpaddivphi + circ + crop are applied while storing them.  The
+//    adjoint only needs the n x n object points (the forward transforms the
+//    N x N extended object), so its grid is 2n x 2n and its lines have n points.
 //  * The periodic halo of the gridding grid (wrap/wrapadj) is an index
-//    modulo 2N.
-//  * The forward's buffers hold pairs of slices interleaved, so that a grid
-//    point or a polar sample of a pair is one 16-byte access.
+//    modulo the grid edge.
+//  * Grid buffers hold pairs of slices interleaved, so that a grid point of a
+//    pair is one 16-byte access.
 //  * gather: 8 x 8 Kaiser-Bessel taps (see below) from grid tiles staged in LDS.
 //  * scatter: deterministic and free of atomics.  At set_theta time every
-//    16 x 8 grid tile gets the list of polar samples whose 15 x 15
-//    footprint covers part of it (wrapadj folded into the periodic
-//    offsets); one wavefront owns a (tile, list chunk, 16 slices) work item
-//    and accumulates the tile as FP32 matrix-core products (row weights x
-//    column-weighted sample values); tiles with several chunks sum their
-//    partials in a fixed order in a fix-up kernel.
+//    8 x 8 grid tile gets the list of polar samples whose footprint covers
+//    part of it (wrapadj folded into the periodic offsets); one wavefront owns
+//    a (tile, list chunk, slices) work item and accumulates the tile as FP32
+//    matrix-core products; tiles with several chunks sum their partials in a
+//    fixed order in a fix-up kernel.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -37,45 +37,45 @@
 #include "common.hpp"
 
 namespace {
-constexpr double kPiRef = 3.1415926535;  // kernels.cuh:1
-constexpr int kTile = 32;                // scatter tile edge (grid points)
+constexpr int kTile = 32;                // gather tile edge (grid points)
 constexpr int kWorkMax = 256;            // samples per gather work item
 }  // namespace
 
 struct pt_tomo {
-  int ntheta, pz, n, N, M;
-  float mu;
-  pt::LinePlan plan;
+  int ntheta, pz, n, N;
+  int pzs;                   // pz rounded up to whole blocks of 8 slices
+  pt::LinePlan plan, plann;  // lines of N and of n points
   float2* tw = nullptr;      // [N] exp(-2 pi i m/N)
   float2* twist = nullptr;   // [N] exp(-i pi j/N), j = idx - N/2
+  float2* twn = nullptr;     // [n], [n]: the same for n
+  float2* twistn = nullptr;
   float* dphi = nullptr;     // [N] forward: 1/(kernel's transform) at a/(2N), a = idx - N/2
-  float* dphia = nullptr;    // [N] adjoint: exp(mu a^2)/(2N)
+  float* dphia = nullptr;    // [n] adjoint: the same at a/(2n), a = idx - n/2
   float* filt = nullptr;     // [N] detector-frequency filter of the adjoint, or null
   int2* mrange = nullptr;    // [N] circ mask column range [lo, hi) per row
   float2* spos = nullptr;    // [ntheta*N] sample positions (x, y)
   int2* sfloor = nullptr;    // [ntheta*N] floor(2N*x), floor(2N*y)
-  int2* ffloor = nullptr;    // [ntheta*N] the same of the exact products (forward)
-  float* wfwd = nullptr;     // [ntheta*N][16] gridding weights of the forward
-  // buffers of both directions (pz rounded up to whole slice pairs)
-  float2* A = nullptr;       // fwd [pz/2][N][2N][2], adj [pz][n][2N]
-  float2* Bg = nullptr;      // fwd [pz/2][2N][2N][2], adj [pz][2N][2N]
-  float2* Q = nullptr;       // polar samples: fwd [pz/2][sample][2], adj [sample][pz]
+  float* wfwd = nullptr;     // [ntheta*N][16] gridding weights, forward and adjoint
+  float* wadj = nullptr;
+  // buffers of both directions (pz rounded up to whole blocks)
+  float2* A = nullptr;       // fwd [pz/2][N][2N][2], adj [pz/2][n][2n][2]
+  float2* Bg = nullptr;      // fwd [pz/2][2N][2N][2], adj [pz/2][2n][2n][2]
+  float2* Q = nullptr;       // polar samples: fwd [pz/2][sample][2], adj [sample][pzs]
   // gather bins: samples by kTile x kTile tile of their floor position
   int ntile1 = 0;            // tiles per axis
   int* wi_tile = nullptr;    // [nwi] tile index
   int2* wi_range = nullptr;  // [nwi] [s0, s1) into bin_sample
   int* bin_sample = nullptr; // [ntheta*N]
   int nwi = 0;
-  // scatter: per kTSY x kTSX grid tile, the samples whose footprint covers it
-  int nt8 = 0;
-  int* ent_s = nullptr;      // [nent] sample
-  int* ent_o = nullptr;      // [nent] packed footprint offset (ox+64) | (oy+64) << 8
+  // scatter: per 8 x 8 tile of the 2n x 2n grid, the samples whose footprint covers it
+  int nts = 0;               // tiles per axis
+  int2* ent = nullptr;       // [nent] sample, footprint origin - tile: x + 8 | y << 8
   int* swi_tile = nullptr;   // [nswi]
   int2* swi_range = nullptr; // [nswi] entry range
   int* swi_slot = nullptr;   // [nswi] partial slot, -1 = direct write
   int4* sfix = nullptr;      // [nfix] (tile, first slot, nslots, 0)
-  int nswi = 0, nfix = 0;
-  float2* spart = nullptr;   // [nslots][pz][64]
+  int nswi = 0, nfix = 0, szb = 1;
+  float2* spart = nullptr;   // [nslots][pzs/2][64][2]
   int rows_per_wg = 1, cols_per_wg = 1, adj_lines = 1;
   int line_kind = PT_LINES_AUTO;  // line passes: register FFT where N allows, or generic
   bool ready = false;
@@ -83,12 +83,6 @@ struct pt_tomo {
 
 namespace pt {
 namespace {
-
-// ------------------------------------------------------------------ helpers
-__device__ __forceinline__ int wrap2n(int v, int twoN) {
-  v %= twoN;
-  return v < 0 ? v + twoN : v;
-}
 
 // ------------------------------------------------------------------ forward row pass
 // For rows q of slice z: x[p] = mask*u[clamp]*dphi[q]*dphi[p] (pad2, circ,
@@ -349,12 +343,13 @@ __global__ __launch_bounds__(256) void k_line_idft(float2* __restrict__ g, const
 }
 
 // ------------------------------------------------------------------ adjoint line: pad + 1D DFT
-// ZQ slices of one angle per workgroup; output Q[sample][z] (z fastest) for
-// the owner-computes scatter.
+// ZQ slices of one angle per workgroup; output Q[sample][z] (z fastest, pzs =
+// pz rounded up to 8 slices, the rest zeros) for the owner-computes scatter.
 constexpr int kZQ = 8;
 __global__ __launch_bounds__(256) void k_adj_line(float2* __restrict__ Q, const float2* __restrict__ g,
                            const float2* __restrict__ tw, const float* __restrict__ filt,
-                           LinePlan plan, float oscale, int n, int ntheta, int pz, int zq) {
+                           LinePlan plan, float oscale, int n, int ntheta, int pz, int pzs,
+                           int zq) {
   extern __shared__ float2 lds[];
   const int N = plan.N, th = blockIdx.x, z0 = blockIdx.y * zq;
   const int nzl = min(zq, pz - z0);
@@ -377,204 +372,173 @@ __global__ __launch_bounds__(256) void k_adj_line(float2* __restrict__ Q, const 
   const float2* res = lds_fft_pp<-1>(lds, lb, N + 1, zq, plan, twl, threadIdx.x, blockDim.x);
   for (int t = threadIdx.x; t < zq * N; t += blockDim.x) {
     const int i = t / zq, zz = t - i * zq;
-    if (zz >= nzl) continue;
+    if (z0 + zz >= pzs) continue;
     int b = i - N / 2;  // kappa
     if (b < 0) b += N;
     const float w = filt ? oscale * filt[i] : oscale;
-    Q[((long)th * N + i) * pz + z0 + zz] = cscale(res[zz * (N + 1) + b], w);
+    Q[((long)th * N + i) * pzs + z0 + zz] = cscale(res[zz * (N + 1) + b], w);
   }
 }
 
 // ------------------------------------------------------------------ scatter (owner computes)
 // Adjoint gridding (kernels.cuh:128-158 transposed, wrapadj folded in by the
-// periodic entry offsets) as a matrix product per grid tile of kTSY x kTSX
-// points and kZS slices:
-//   G[y][(z, part, x)] = sum_entries wy_e(y) * (wx_e(x) * Q_e[z].part),
-// K = the tile's entries (samples whose 15 x 15 footprint covers part of the
-// tile, in list order), M = the 16 tile rows, N = 16 slices x (re, im) x 8
-// columns, on FP32 matrix cores: one 16x16x4 MFMA per slice and 4 entries.
-// A wavefront takes one (tile entry chunk, kZS slices).  Per chunk of 32
-// entries, lanes 0-31 stage the row and column weights of entry `lane` (zero
-// outside its footprint) and lanes 32-63 its slice values in LDS; the MFMA A
-// operand is a row weight, the B operand a column weight times a slice value.
+// periodic entry offsets) onto the 2n x 2n grid -- the n object points are
+// oversampled by 2 -- as a matrix product per grid tile of 8 x 8 points:
+//   G[(z, part)][point] = sum_entries Q_e[(z, part)] * (wx_e wy_e)[point],
+// K = the tile's entries (samples whose 8 x 8 footprint covers part of the
+// tile, in list order), on FP32 matrix cores: one 16x16x4 MFMA takes 4
+// entries, 8 slices (16 rows: slice, re/im) and 16 points (8 columns x 2
+// rows).  A wavefront takes one tile entry chunk and 8 ZB slices, i.e. 4 ZB
+// MFMAs per 4 entries; the A operand is read straight from the samples
+// (16 adjacent lanes: 64 contiguous bytes), the B operand is the product of a
+// column and a row weight.  Per 32 entries, lane l stages the column (l < 32)
+// or row weights of entry l % 32, clipped to the tile, in LDS; the weights of
+// the next 32 entries and the index of the ones after are loaded meanwhile.
 // MFMA 16x16x4 f32 operand layout (lane l): A[i][k]: i = l%16, k = l/16;
-// B[k][j]: j = l%16, k = l/16; D[i][j]: j = l%16, i = 4*(l/16) + r.  Column j
-// of N-tile t is slice z0 + t, part j/8, grid column x = j%8: a row's 8
-// complex points are written by 16 adjacent lanes (64 contiguous bytes).
-constexpr int kTSY = 16;  // scatter tile rows
-constexpr int kTSX = 8;   // scatter tile columns
-constexpr int kZS = 16;   // slices per work item
-constexpr int kSChunk = 1024;
+// B[k][j]: j = l%16, k = l/16; D[i][j]: j = l%16, i = 4*(l/16) + r, so a lane
+// ends with one point of one slice pair: a 16-byte store, 8 adjacent points.
+// Bound: matrix cores.  A footprint meets (15/8)^2 = 3.5 tiles, so 450
+// multiply-adds per sample and slice (0.22 ms at 256^3, 384 angles); tiles of
+// 16 x 8 points would take 690.  Measured there: 0.45 ms per launch, 1.39 ms with
+// 15 x 15 Gaussian footprints on the 3n x 3n grid (whose column pass took 0.39
+// ms and row pass 0.12, now 0.19 and 0.11).
+constexpr int kTS = 8;    // scatter tile edge
+constexpr int kSE = 32;   // entries per staged chunk
 typedef float f4m __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(64) void k_scatter_own(float2* __restrict__ Bg,
-                                                    float2* __restrict__ part,
-                                                    const float2* __restrict__ Q,
-                                                    const float2* __restrict__ spos,
-                                                    const int2* __restrict__ sfloor,
-                                                    const int* __restrict__ ent_s,
-                                                    const int* __restrict__ ent_o,
+template <int ZB>
+__global__ __launch_bounds__(64) void k_scatter_own(f4m* __restrict__ Bg, f4m* __restrict__ part,
+                                                    const float* __restrict__ Q,
+                                                    const f4m* __restrict__ wts,
+                                                    const int2* __restrict__ ent,
                                                     const int* __restrict__ wi_tile,
                                                     const int2* __restrict__ wi_range,
-                                                    const int* __restrict__ wi_slot, int N,
-                                                    int M, float beta, int ntx, int pz) {
-  constexpr int kSE = 32;  // entries per staged chunk
-  __shared__ float wys[kSE][kTSY + 1];
-  __shared__ float wxs[kSE][kTSX + 1];
-  __shared__ float4 qs[kSE][2][kZS / 4 + 1];  // [entry][re, im][16 slices]
-  const int twoN = 2 * N;
+                                                    const int* __restrict__ wi_slot, int ntx,
+                                                    int pzs) {
+  __shared__ float wl[2][kSE][kTS + 1];  // column, row weights on the tile
+  __shared__ int sl[kSE];                // samples
   // XCD-contiguous order: adjacent tiles share the samples of their entries
   const int lw = xcd_contig(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int zb = lw / gridDim.x;
-  const int wi = lw - zb * gridDim.x, z0 = zb * kZS;
+  const int wi = lw - zb * gridDim.x, z0 = zb * 8 * ZB;
+  const int nzb = min(ZB, (pzs - z0) / 8);  // blocks of 8 slices
   const int lane = threadIdx.x, j16 = lane & 15, kq = lane >> 4;
-  const int xl = j16 & 7, prt = j16 >> 3;
+  const int el = lane & (kSE - 1), ax = lane / kSE;
   const int tile = wi_tile[wi];
-  const int tx0 = (tile % ntx) * kTSX, ty0 = (tile / ntx) * kTSY;
   const int2 rg = wi_range[wi];
-  const float inv2N = 1.0f / (float)twoN;
-  f4m acc[kZS];
+  f4m acc[ZB][4];
 #pragma unroll
-  for (int t = 0; t < kZS; ++t) acc[t] = f4m{0.f, 0.f, 0.f, 0.f};
-  const int el = lane & (kSE - 1);
-  // software pipeline over the chunks: the entry index of chunk i+2 and the
-  // sample data of chunk i+1 are loaded while chunk i is multiplied, so a
-  // chunk's staging waits on no memory round trip
-  auto fetch_idx = [&](int c0) -> int { return c0 + el < rg.y ? ent_s[c0 + el] : -1; };
-  int on = 0;
-  float2 pn = make_float2(0.f, 0.f);
-  int2 fln = make_int2(0, 0);
-  float2 qn[kZS];
-  auto fetch_data = [&](int c0, int sidx) {
-    if (sidx < 0) return;
-    if (lane < kSE) {
-      on = ent_o[c0 + el];
-      pn = spos[sidx];
-      fln = sfloor[sidx];
-    } else {
-      const float2* qsrc = Q + (long)sidx * pz + z0;
+  for (int t = 0; t < ZB; ++t)
 #pragma unroll
-      for (int j = 0; j < kZS; ++j) qn[j] = (z0 + j < pz) ? qsrc[j] : make_float2(0.f, 0.f);
-    }
-  };
-  int sc = fetch_idx(rg.x);
-  fetch_data(rg.x, sc);
-  int sn = fetch_idx(rg.x + kSE);
+    for (int b = 0; b < 4; ++b) acc[t][b] = f4m{0.f, 0.f, 0.f, 0.f};
+  // entry (sample, offsets) of this lane; past the end: sample -1
+  auto fetch_ent = [&](int c0) { return c0 + el < rg.y ? ent[c0 + el] : make_int2(-1, 0); };
+  int2 ec = fetch_ent(rg.x), en = fetch_ent(rg.x + kSE);
+  const f4m* wp = wts + (long)max(ec.x, 0) * 4 + 2 * ax;
+  f4m w0 = wp[0], w1 = wp[1];
+  const float* Qz = Q + 2 * (long)z0 + j16;
   for (int c0 = rg.x; c0 < rg.y; c0 += kSE) {
-    const int ne = min(kSE, rg.y - c0);
-    const bool has = sc >= 0;
-    __syncthreads();  // the previous chunk's operands are read
-    if (lane < kSE) {
-      const int ox = (on & 255) - 64, oy = ((on >> 8) & 255) - 64;  // footprint origin - tile
-      const float2 p = pn;
-      const int2 fl = fln;
+    __syncthreads();  // the previous chunk's weights are read
+    {
+      const int o = ax ? ec.y >> 8 : (ec.y & 255) - 8;  // footprint origin - tile
+      float* row = wl[ax][el];
 #pragma unroll
-      for (int i = 0; i < kTSY; ++i) {
-        const int k1 = i - oy;  // footprint row of tile row i
-        const float dy = (float)(fl.y - M + k1) * inv2N - p.y;
-        wys[el][i] = (has && k1 >= 0 && k1 <= 2 * M) ? __expf(-beta * dy * dy) : 0.f;
-      }
+      for (int k = 0; k < kTS; ++k) row[k] = 0.f;
+      if (ec.x >= 0) {
 #pragma unroll
-      for (int x = 0; x < kTSX; ++x) {
-        const int k0 = x - ox;
-        const float dx = (float)(fl.x - M + k0) * inv2N - p.x;
-        wxs[el][x] = (has && k0 >= 0 && k0 <= 2 * M) ? __expf(-beta * dx * dx) : 0.f;
+        for (int k = 0; k < kW; ++k) {
+          const int x = k + o;
+          if (x >= 0 && x < kTS) row[x] = k < 4 ? w0[k] : w1[k - 4];
+        }
       }
-    } else {
-#pragma unroll
-      for (int j = 0; j < kZS / 4; ++j) {
-        const float2 v0 = has ? qn[4 * j] : make_float2(0.f, 0.f);
-        const float2 v1 = has ? qn[4 * j + 1] : make_float2(0.f, 0.f);
-        const float2 v2 = has ? qn[4 * j + 2] : make_float2(0.f, 0.f);
-        const float2 v3 = has ? qn[4 * j + 3] : make_float2(0.f, 0.f);
-        qs[el][0][j] = make_float4(v0.x, v1.x, v2.x, v3.x);
-        qs[el][1][j] = make_float4(v0.y, v1.y, v2.y, v3.y);
-      }
+      if (!ax) sl[el] = max(ec.x, 0);  // a sample of zero weight past the end
     }
     __syncthreads();
-    // prefetch: data of the next chunk, index of the one after
-    sc = sn;
-    fetch_data(c0 + kSE, sc);
-    sn = fetch_idx(c0 + 2 * kSE);
-    // entries past ne were staged with zero weights and values
-#pragma unroll 1
-    for (int e0 = 0; e0 < ne; e0 += 4) {
-      const int e = e0 + kq;
-      const float a = wys[e][j16];
-      const float wx = wxs[e][xl];
-      float qv[kZS];
+    const int ng = (min(kSE, rg.y - c0) + 3) / 4;
+    // all samples of the chunk in flight
+    float q[kSE / 4][ZB];
 #pragma unroll
-      for (int j = 0; j < kZS / 4; ++j) {
-        const float4 q = qs[e][prt][j];
-        qv[4 * j] = q.x; qv[4 * j + 1] = q.y; qv[4 * j + 2] = q.z; qv[4 * j + 3] = q.w;
+    for (int g = 0; g < kSE / 4; ++g) {
+      const float* qp = Qz + (long)sl[4 * g + kq] * (2 * pzs);
+#pragma unroll
+      for (int t = 0; t < ZB; ++t) q[g][t] = (g < ng && t < nzb) ? qp[16 * t] : 0.f;
+    }
+    ec = en;
+    wp = wts + (long)max(ec.x, 0) * 4 + 2 * ax;
+    w0 = wp[0];
+    w1 = wp[1];
+    en = fetch_ent(c0 + 2 * kSE);
+#pragma unroll
+    for (int g = 0; g < kSE / 4; ++g) {
+      if (g < ng) {
+        const int e = 4 * g + kq;
+        const float wx = wl[0][e][j16 & 7];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const float w = wx * wl[1][e][2 * b + (j16 >> 3)];
+#pragma unroll
+          for (int t = 0; t < ZB; ++t)
+            acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[g][t], w, acc[t][b], 0, 0, 0);
+        }
       }
-#pragma unroll
-      for (int t = 0; t < kZS; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, wx * qv[t], acc[t], 0, 0, 0);
     }
   }
-  const int slot = wi_slot[wi];
-  float* Bf = reinterpret_cast<float*>(Bg);
-  float* Pf = reinterpret_cast<float*>(part);
-  const int gx = tx0 + xl;
+  const int slot = wi_slot[wi], G = kTS * ntx, npair = pzs / 2;
+  const int x = j16 & 7, y = j16 >> 3;
 #pragma unroll
-  for (int t = 0; t < kZS; ++t) {
-    const int z = z0 + t;
-    if (z >= pz) break;
+  for (int t = 0; t < ZB; ++t) {
+    if (t >= nzb) break;
+    const long pr = z0 / 2 + 4 * t + kq;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int yl = 4 * kq + r, gy = ty0 + yl;
-      if (slot < 0) {
-        if (gx < twoN && gy < twoN) Bf[(((long)z * twoN + gy) * twoN + gx) * 2 + prt] = acc[t][r];
-      } else {
-        Pf[(((long)slot * pz + z) * (kTSY * kTSX) + yl * kTSX + xl) * 2 + prt] = acc[t][r];
-      }
+    for (int b = 0; b < 4; ++b) {
+      if (slot < 0)
+        Bg[(pr * G + (tile / ntx) * kTS + 2 * b + y) * G + (tile % ntx) * kTS + x] = acc[t][b];
+      else
+        part[(slot * (long)npair + pr) * (kTS * kTS) + (2 * b + y) * kTS + x] = acc[t][b];
     }
   }
 }
 
 // tiles whose entry list spans several chunks: sum the chunk partials in order
-__global__ __launch_bounds__(kTSY * kTSX) void k_scatter_fix(float2* __restrict__ Bg,
-                                                             const float2* __restrict__ part,
-                                                             const int4* __restrict__ fix, int N,
-                                                             int ntx, int pz) {
+__global__ __launch_bounds__(kTS * kTS) void k_scatter_fix(f4m* __restrict__ Bg,
+                                                           const f4m* __restrict__ part,
+                                                           const int4* __restrict__ fix, int ntx,
+                                                           int npair) {
   const int4 f = fix[blockIdx.x];  // (tile, first slot, nslots, -)
-  const int z = blockIdx.y, p = threadIdx.x;
-  const int twoN = 2 * N;
-  const int gx = (f.x % ntx) * kTSX + p % kTSX, gy = (f.x / ntx) * kTSY + p / kTSX;
-  if (gx >= twoN || gy >= twoN) return;
-  float2 s = make_float2(0.f, 0.f);
-  for (int k = 0; k < f.z; ++k) s = cadd(s, part[((long)(f.y + k) * pz + z) * (kTSY * kTSX) + p]);
-  Bg[((long)z * twoN + gy) * twoN + gx] = s;
+  const int pr = blockIdx.y, p = threadIdx.x, G = kTS * ntx;
+  f4m s = {0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < f.z; ++k) s += part[((f.y + k) * (long)npair + pr) * (kTS * kTS) + p];
+  Bg[((long)pr * G + (f.x / ntx) * kTS + p / kTS) * G + (f.x % ntx) * kTS + p % kTS] = s;
 }
 
 // ------------------------------------------------------------------ adjoint column pass
-// C = 2^lc columns kx per workgroup: centred inverse 2N-point DFT along ky
-// evaluated at the n object rows q in [o, o+n), as the even and the odd
-// N-point inverse DFTs run one after the other in the same C LDS lines
-// (ping-pong pair); the even half at the output rows waits in registers.
+// C = 2^lc of the 4n columns (kx, slice) of slice pair z per workgroup: centred
+// inverse 2n-point DFT along ky evaluated at the n object rows, as the even
+// and the odd n-point inverse DFTs run one after the other in the same C LDS
+// lines (ping-pong pair); the even half waits in registers.
+// Bg[z][2n][2n][2] -> A[z][n][2n][2].
 __global__ __launch_bounds__(256) void k_col_adj(float2* __restrict__ A, const float2* __restrict__ Bg,
                           const float2* __restrict__ tw, const float2* __restrict__ twist,
-                          LinePlan plan, int n, int lc) {
+                          LinePlan plan, int lc) {
   extern __shared__ float2 lds[];
-  const int N = plan.N, twoN = 2 * N, S = N + 1, o = N / 6, C = 1 << lc;
-  const int gx = (twoN + C - 1) >> lc;
+  const int n = plan.N, W = 4 * n, S = n + 1, C = 1 << lc;
+  const int gx = (W + C - 1) >> lc;
   const int L = xcd_contig(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
   const int z = L / gx, k0 = (L - z * gx) << lc;
   float2* la = lds;
   float2* lb = la + C * S;
   float2* twl = lb + C * S;
-  for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = tw[i];
-  const int nv = (n * C + 255) >> 8;  // n * C <= 256 * kColVpt since n = 2N/3
-  const float2* Bz = Bg + (long)z * twoN * twoN + k0;
-  float2* Az = A + (long)z * n * twoN + k0;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+  const int nv = (n * C + 255) >> 8;  // n * C <= 256 * kColVpt since 3n/2 * C is
+  const float2* Bz = Bg + (long)z * (2 * n) * W + k0;
+  float2* Az = A + (long)z * n * W + k0;
   // lines of parity par of the C columns -> LDS, inverse FFT
   auto phase = [&](int par) -> const float2* {
-    for (int i = threadIdx.x; i < N * C; i += blockDim.x) {
+    for (int i = threadIdx.x; i < n * C; i += blockDim.x) {
       const int r = i >> lc, cc = i & (C - 1);
-      const int m = r - N / 2;  // ky - N = 2m + par
-      const int b = m < 0 ? m + N : m;
-      la[cc * S + b] = (k0 + cc < twoN) ? Bz[(long)(2 * m + par + N) * twoN + cc]
-                                        : make_float2(0.f, 0.f);
+      const int m = r - n / 2;  // ky - n = 2m + par
+      const int b = m < 0 ? m + n : m;
+      la[cc * S + b] = (k0 + cc < W) ? Bz[(long)(2 * m + par + n) * W + cc]
+                                     : make_float2(0.f, 0.f);
     }
     __syncthreads();
     return lds_fft_pp<1>(la, lb, S, C, plan, twl, threadIdx.x, blockDim.x);
@@ -584,100 +548,103 @@ __global__ __launch_bounds__(256) void k_col_adj(float2* __restrict__ A, const f
 #pragma unroll
   for (int v = 0; v < kColVpt; ++v) {
     const int i = threadIdx.x + v * 256;
-    const int qi = i >> lc, cc = i & (C - 1);
-    int a = qi + o - N / 2;
-    if (a < 0) a += N;
-    if (v < nv && qi < n) ev[v] = res[cc * S + a];
+    const int q = i >> lc, cc = i & (C - 1);
+    int a = q - n / 2;
+    if (a < 0) a += n;
+    if (v < nv && q < n) ev[v] = res[cc * S + a];
   }
   __syncthreads();
   res = phase(1);
 #pragma unroll
   for (int v = 0; v < kColVpt; ++v) {
     const int i = threadIdx.x + v * 256;
-    const int qi = i >> lc, cc = i & (C - 1);
-    if (v < nv && qi < n && k0 + cc < twoN) {
-      const int q = qi + o;  // row index, centred q - N/2
-      int a = q - N / 2;
-      if (a < 0) a += N;
-      Az[(long)qi * twoN + cc] = cadd(ev[v], cmulc(res[cc * S + a], twist[q]));
+    const int q = i >> lc, cc = i & (C - 1);
+    if (v < nv && q < n && k0 + cc < W) {
+      int a = q - n / 2;
+      if (a < 0) a += n;
+      Az[(long)q * W + cc] = cadd(ev[v], cmulc(res[cc * S + a], twist[q]));
     }
   }
 }
 
 // ------------------------------------------------------------------ adjoint row pass
+// A workgroup takes `rows` of the pair's 2 n (row, slice) lines; unpaddivphi +
+// circ + crop while storing.
 __global__ __launch_bounds__(256) void k_row_adj(float2* __restrict__ f, const float2* __restrict__ A,
                           const float2* __restrict__ tw, const float2* __restrict__ twist,
                           const float* __restrict__ dphi, const int2* __restrict__ mrange,
-                          LinePlan plan, int n, int rows, float scale) {
+                          LinePlan plan, int rows, float scale, int pz) {
   extern __shared__ float2 lds[];
-  const int N = plan.N, z = blockIdx.y, r0 = blockIdx.x * rows;
-  const int o = N / 6;
+  const int n = plan.N, r0 = blockIdx.x * rows, pr = blockIdx.y;
+  const int o = n / 4;  // (3n/2) / 6
   const int nl = 2 * rows;
-  float2* lb = lds + nl * (N + 1);
-  float2* twl = lb + nl * (N + 1);
-  for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = tw[i];
-  for (int i = threadIdx.x; i < 2 * N * rows; i += blockDim.x) {
-    const int r = i / (2 * N), kx = i - r * 2 * N;
-    const int qi = r0 + r;
+  float2* lb = lds + nl * (n + 1);
+  float2* twl = lb + nl * (n + 1);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+  for (int i = threadIdx.x; i < 2 * n * rows; i += blockDim.x) {
+    const int rl = i / (2 * n), kx = i - rl * 2 * n;
+    const int r = r0 + rl;
     float2 val = make_float2(0.f, 0.f);
-    if (qi < n) val = A[((long)z * n + qi) * (2 * N) + kx];
-    const int kp = kx - N;
+    if (r < 2 * n) val = A[(((long)pr * n + (r >> 1)) * (2 * n) + kx) * 2 + (r & 1)];
+    const int kp = kx - n;
     const int par = kp & 1;
     const int m = (kp - par) / 2;
-    const int b = m < 0 ? m + N : m;
-    lds[(2 * r + par) * (N + 1) + b] = val;
+    const int b = m < 0 ? m + n : m;
+    lds[(2 * rl + par) * (n + 1) + b] = val;
   }
   __syncthreads();
-  const float2* res = lds_fft_pp<1>(lds, lb, N + 1, nl, plan, twl, threadIdx.x, blockDim.x);
+  const float2* res = lds_fft_pp<1>(lds, lb, n + 1, nl, plan, twl, threadIdx.x, blockDim.x);
   for (int i = threadIdx.x; i < n * rows; i += blockDim.x) {
-    const int r = i / n, pi = i - r * n;
-    const int qi = r0 + r;
-    if (qi >= n) continue;
-    const int q = qi + o, p = pi + o;
-    int a = p - N / 2;
-    if (a < 0) a += N;
-    const float2 e = res[(2 * r) * (N + 1) + a];
-    const float2 od = res[(2 * r + 1) * (N + 1) + a];
-    float2 v = cadd(e, cmulc(od, twist[p]));
-    const int2 mr = mrange[q];
-    const float w = (p >= mr.x && p < mr.y) ? dphi[q] * dphi[p] * scale : 0.f;
-    f[((long)z * n + qi) * n + pi] = cscale(v, w);
+    const int rl = i / n, p = i - rl * n;
+    const int r = r0 + rl, q = r >> 1, z = 2 * pr + (r & 1);
+    if (q >= n || z >= pz) continue;
+    int a = p - n / 2;
+    if (a < 0) a += n;
+    const float2 e = res[(2 * rl) * (n + 1) + a];
+    const float2 od = res[(2 * rl + 1) * (n + 1) + a];
+    const float2 v = cadd(e, cmulc(od, twist[p]));
+    const int2 mr = mrange[q + o];
+    const float w = (p + o >= mr.x && p + o < mr.y) ? dphi[q] * dphi[p] * scale : 0.f;
+    f[((long)z * n + q) * n + p] = cscale(v, w);
   }
 }
 
 // ------------------------------------------------------------------ register line FFT passes
-// The six line passes above for N = P T with T = N / P (P = kLineP points per
-// lane; n = 64, 96, 128, 192, 256, 512), on the register line FFT (LineReg):
-// every lane holds P points of one line, the passes' index arithmetic is
-// compile-time, and LDS is used only for the exchanges between Stockham
-// passes.  A workgroup of NT = nt_of<N>() lanes holds NT / T lines, each
-// with one LDS row; the twiddle table follows them.  Each kernel computes the
-// same quantities as its generic counterpart (same index maps; FP32 sums in a
-// different order).
+// The six line passes above on the register line FFT (LineReg) for n = 64, 96,
+// 128, 192, 256, 512: every lane holds P points of one line, the passes' index
+// arithmetic is compile-time, and LDS is used only for the exchanges between
+// Stockham passes.  Lines of N = 3n/2 points (the forward's grid passes and the
+// detector lines) take P = 24; lines of n points (the adjoint's grid passes)
+// P = 16 for powers of two, else 24.  A workgroup of NT = nt_of<N, P>() lanes
+// holds NT / T lines (T = N / P), each with one LDS row; the twiddle table
+// follows them.  Each kernel computes the same quantities as its generic
+// counterpart (same index maps; FP32 sums in a different order).
 //
 // The centred index maps become register rotations: the rotated FFT position
 // a = t + T m of an input at centred index c = a + N/2 (mod N) is
 // c = t + T ((m + P/2) mod P), and output position b = t + T m is centred
-// frequency b (m < P/2) or b - N (m >= P/2).  Of the N points of a line, the
-// n = 2N/3 object or detector points are m in [2P/3, P) and [0, P/3) in the
-// rotated order.
+// frequency b (m < P/2) or b - N (m >= P/2).  Of the N points of a detector
+// line, the n = 2N/3 pixels are m in [2P/3, P) and [0, P/3) in the rotated order.
 constexpr int kNT = kLineThreads;
-// lanes of a workgroup for N: 2 T C with C, the columns of a column tile, the
+// lanes of a workgroup: 2 T C with C, the columns of a column tile, the
 // largest power of two that fits kNT (T = 16: 256 lanes; T = 6, 12: 192)
-template <int N>
+template <int N, int P = kLineP>
 constexpr int nt_of() {
-  constexpr int T = LineReg<N>::T;
+  constexpr int T = LineReg<N, P>::T;
   int c = 1;
   while (4 * T * c <= kNT) c *= 2;
   return 2 * T * c;
 }
+// points per lane of the adjoint's n-point lines
+template <int n>
+constexpr int pa_of() { return n % 3 == 0 ? 24 : 16; }
 template <int N>
 __device__ __forceinline__ void stage_twiddles(float2* twl, const float2* __restrict__ tw) {
   for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = tw[i];
 }
-template <int N>
+template <int N, int P = kLineP>
 constexpr size_t reg_lds_bytes() {
-  return sizeof(float2) * ((size_t)(nt_of<N>() / LineReg<N>::T) * (N + 1) + N);
+  return sizeof(float2) * ((size_t)(nt_of<N, P>() / LineReg<N, P>::T) * (N + 1) + N);
 }
 
 // forward row pass: rows q of slice pair z, lines (r, parity, slice); lane =
@@ -804,7 +771,7 @@ __global__ __launch_bounds__(kNT) void k_adj_line_r(float2* __restrict__ Q,
                                                     const float2* __restrict__ g,
                                                     const float2* __restrict__ tw,
                                                     const float* __restrict__ filt, float oscale,
-                                                    int ntheta, int pz) {
+                                                    int ntheta, int pz, int pzs) {
   constexpr int P = kLineP, H = P / 2, T = LineReg<N>::T, ZQ = nt_of<N>() / T, n = 2 * N / 3,
                 o = N / 6;
   extern __shared__ float2 lds[];
@@ -822,105 +789,108 @@ __global__ __launch_bounds__(kNT) void k_adj_line_r(float2* __restrict__ Q,
   });
   __syncthreads();
   line_reg_fft<N, -1>(v, lds + zz * (N + 1), twl, t);
-  if (!ok) return;
+  if (z >= pzs) return;
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const int i = t + T * ((m + H) % P);  // sample index along the line
     const float w = filt ? oscale * filt[i] : oscale;
-    Q[((long)th * N + i) * pz + z] = cscale(v[m], w);
+    Q[((long)th * N + i) * pzs + z] = cscale(v[m], ok ? w : 0.f);
   });
 }
 
-// Parity halves of an adjoint 2N-point line: the even (par 0) and odd
-// (par 1) inverse DFTs of one output line sit in partner lanes (lane ^ pm).
-// Output positions m in [0, P/3) are finished by the par 0 lane, m in
-// [2P/3, P) by the par 1 lane (the others lie outside the n object points);
-// each lane sends the P/3 values its partner needs.
-constexpr int kP3 = kLineP / 3;
-__device__ __forceinline__ void parity_swap(const float2 (&v)[kLineP], int par, int pm,
-                                            float2 (&E)[kP3], float2 (&O)[kP3]) {
-  static_for<0, kP3>([&](auto kc) {
+// Parity halves of an adjoint 2n-point line: the even (par 0) and odd (par 1)
+// inverse DFTs of one output line sit in partner lanes (lane ^ pm).  Output
+// positions m in [0, P/2) are finished by the par 0 lane, the others by the
+// par 1 lane; each lane sends the P/2 values its partner needs.
+template <int P>
+__device__ __forceinline__ void parity_swap(const float2 (&v)[P], int par, int pm,
+                                            float2 (&E)[P / 2], float2 (&O)[P / 2]) {
+  static_for<0, P / 2>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    const float2 s = par ? v[k] : v[2 * kP3 + k];
+    const float2 s = par ? v[k] : v[P / 2 + k];
     float2 r;
     r.x = __shfl_xor(s.x, pm, 64);
     r.y = __shfl_xor(s.y, pm, 64);
     E[k] = par ? r : v[k];
-    O[k] = par ? v[2 * kP3 + k] : r;
+    O[k] = par ? v[P / 2 + k] : r;
   });
 }
 
-// adjoint column pass: C columns, lines (par C + cc); lane = cc + C (par + 2 t)
-template <int N>
+// adjoint column pass: C of the 4n columns (kx, slice) of slice pair z, lines
+// (par C + cc); lane = cc + C (par + 2 t)
+template <int n>
 __global__ __launch_bounds__(kNT) void k_col_adj_r(float2* __restrict__ A,
                                                    const float2* __restrict__ Bg,
                                                    const float2* __restrict__ tw,
                                                    const float2* __restrict__ twist) {
-  constexpr int P = kLineP, H = P / 2, P3 = kP3, T = LineReg<N>::T, C = nt_of<N>() / (2 * T),
-                twoN = 2 * N, gx = twoN / C, o = N / 6, n = 2 * N / 3;
+  constexpr int P = pa_of<n>(), H = P / 2, T = LineReg<n, P>::T, C = nt_of<n, P>() / (2 * T),
+                W = 4 * n, gx = W / C;
+  static_assert(W % C == 0, "column tiles");
   static_assert(C <= 32 && (C & (C - 1)) == 0, "parity partner lane ^ C in the same wavefront");
   extern __shared__ float2 lds[];
-  float2* twl = lds + 2 * C * (N + 1);
-  stage_twiddles<N>(twl, tw);
+  float2* twl = lds + 2 * C * (n + 1);
+  stage_twiddles<n>(twl, tw);
   const int tid = threadIdx.x, cc = tid % C, par = (tid / C) & 1, t = tid / (2 * C);
   const int L = xcd_contig(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
   const int z = L / gx, k0 = (L - z * gx) * C;
-  const float2* Bz = Bg + (long)z * twoN * twoN + k0 + cc;
+  const float2* Bz = Bg + (long)z * (2 * n) * W + k0 + cc;
   float2 v[P];
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const int b = t + T * m;
-    v[m] = Bz[(long)((m < H ? 2 * b + N : 2 * b - N) + par) * twoN];
+    v[m] = Bz[(long)((m < H ? 2 * b + n : 2 * b - n) + par) * W];
   });
   __syncthreads();
-  line_reg_fft<N, 1>(v, lds + (par * C + cc) * (N + 1), twl, t);
-  float2 E[P3], O[P3];
-  parity_swap(v, par, C, E, O);
-  float2* Az = A + (long)z * n * twoN + k0 + cc;
-  static_for<0, P3>([&](auto kc) {
+  line_reg_fft<n, 1>(v, lds + (par * C + cc) * (n + 1), twl, t);
+  float2 E[H], O[H];
+  parity_swap<P>(v, par, C, E, O);
+  float2* Az = A + (long)z * n * W + k0 + cc;
+  static_for<0, H>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    const int q = t + T * (par ? k + P / 6 : k + H);  // object row, centred q - N/2
-    Az[(long)(q - o) * twoN] = cadd(E[k], cmulc(O[k], twist[q]));
+    const int q = t + T * (par ? k : k + H);  // object row: rotated position q - n/2
+    Az[(long)q * W] = cadd(E[k], cmulc(O[k], twist[q]));
   });
 }
 
-// adjoint row pass: object rows qi, lines (2 r + par); lane = par + 2 (t + T r)
-template <int N>
+// adjoint row pass: object rows q of slice pair z, lines (r, slice, parity);
+// lane = slice + 2 (par + 2 (t + T r))
+template <int n>
 __global__ __launch_bounds__(kNT) void k_row_adj_r(float2* __restrict__ f,
                                                    const float2* __restrict__ A,
                                                    const float2* __restrict__ tw,
                                                    const float2* __restrict__ twist,
                                                    const float* __restrict__ dphi,
-                                                   const int2* __restrict__ mrange, float scale) {
-  constexpr int P = kLineP, H = P / 2, P3 = kP3, T = LineReg<N>::T, NL = nt_of<N>() / T,
-                ROWS = NL / 2, o = N / 6, n = 2 * N / 3;
+                                                   const int2* __restrict__ mrange, float scale,
+                                                   int pz) {
+  constexpr int P = pa_of<n>(), H = P / 2, T = LineReg<n, P>::T, NL = nt_of<n, P>() / T,
+                ROWS = NL / 4, o = n / 4;
+  static_assert(n % ROWS == 0, "whole row tiles");
   extern __shared__ float2 lds[];
-  float2* twl = lds + NL * (N + 1);
-  stage_twiddles<N>(twl, tw);
-  const int tid = threadIdx.x, par = tid & 1, t = (tid >> 1) % T, r = tid / (2 * T);
-  const int z = blockIdx.y, qi = blockIdx.x * ROWS + r;
-  const bool ok = qi < n;
-  const float2* Ar = A + ((long)z * n + min(qi, n - 1)) * (2 * N);
+  float2* twl = lds + NL * (n + 1);
+  stage_twiddles<n>(twl, tw);
+  const int tid = threadIdx.x, zz = tid & 1, par = (tid >> 1) & 1, t = (tid >> 2) % T,
+            r = tid / (4 * T);
+  const int q = blockIdx.x * ROWS + r, z = 2 * blockIdx.y + zz;
+  const float2* Ar = A + ((long)blockIdx.y * n + q) * (4 * n) + 2 * par + zz;
   float2 v[P];
   static_for<0, P>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const int b = t + T * m;
-    v[m] = Ar[(m < H ? 2 * b + N : 2 * b - N) + par];  // row clamped past n
+    v[m] = Ar[2 * (m < H ? 2 * b + n : 2 * b - n)];
   });
   __syncthreads();
-  line_reg_fft<N, 1>(v, lds + (2 * r + par) * (N + 1), twl, t);
-  float2 E[P3], O[P3];
-  parity_swap(v, par, 1, E, O);
-  if (!ok) return;
-  const int q = qi + o;
-  const int2 mr = mrange[q];
+  line_reg_fft<n, 1>(v, lds + (4 * r + 2 * zz + par) * (n + 1), twl, t);
+  float2 E[H], O[H];
+  parity_swap<P>(v, par, 2, E, O);
+  if (z >= pz) return;
+  const int2 mr = mrange[q + o];
   const float dq = dphi[q];
-  float2* fr = f + ((long)z * n + qi) * n;
-  static_for<0, P3>([&](auto kc) {
+  float2* fr = f + ((long)z * n + q) * n;
+  static_for<0, H>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    const int p = t + T * (par ? k + P / 6 : k + H);  // object column, centred p - N/2
-    const float w = (p >= mr.x && p < mr.y) ? dq * dphi[p] * scale : 0.f;
-    fr[p - o] = cscale(cadd(E[k], cmulc(O[k], twist[p])), w);
+    const int p = t + T * (par ? k : k + H);  // object column: rotated position p - n/2
+    const float w = (p + o >= mr.x && p + o < mr.y) ? dq * dphi[p] * scale : 0.f;
+    fr[p] = cscale(cadd(E[k], cmulc(O[k], twist[p])), w);
   });
 }
 
@@ -1006,28 +976,41 @@ template <int N>
 int adj_lines_r(pt_tomo* h, const float2* g, float oscale, hipStream_t st) {
   constexpr int ZQ = nt_of<N>() / LineReg<N>::T;
   ProfScope prof("tomo_adj_line", st);
-  hipLaunchKernelGGL(k_adj_line_r<N>, dim3(h->ntheta, (h->pz + ZQ - 1) / ZQ), dim3(nt_of<N>()),
-                     reg_lds_bytes<N>(), st, h->Q, g, h->tw, h->filt, oscale, h->ntheta, h->pz);
+  hipLaunchKernelGGL(k_adj_line_r<N>, dim3(h->ntheta, (h->pzs + ZQ - 1) / ZQ), dim3(nt_of<N>()),
+                     reg_lds_bytes<N>(), st, h->Q, g, h->tw, h->filt, oscale, h->ntheta, h->pz,
+                     h->pzs);
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
 
 template <int N>
 int adj_grid_r(pt_tomo* h, float2* f, float scale, hipStream_t st) {
-  constexpr int T = LineReg<N>::T, ROWS = nt_of<N>() / (2 * T), C = nt_of<N>() / (2 * T);
-  constexpr size_t lds = reg_lds_bytes<N>();
+  constexpr int n = 2 * N / 3, P = pa_of<n>(), T = LineReg<n, P>::T, NT = nt_of<n, P>(),
+                ROWS = NT / (4 * T), C = NT / (2 * T);
+  constexpr size_t lds = reg_lds_bytes<n, P>();
+  const int npair = (h->pz + 1) / 2;
   {
     ProfScope prof("tomo_col_adj", st);
-    hipLaunchKernelGGL(k_col_adj_r<N>, dim3(2 * N / C, h->pz), dim3(nt_of<N>()), lds, st, h->A, h->Bg,
-                       h->tw, h->twist);
+    hipLaunchKernelGGL(k_col_adj_r<n>, dim3(4 * n / C, npair), dim3(NT), lds, st, h->A, h->Bg,
+                       h->twn, h->twistn);
     PT_LAUNCH_CHECK();
   }
   {
     ProfScope prof("tomo_row_adj", st);
-    hipLaunchKernelGGL(k_row_adj_r<N>, dim3((h->n + ROWS - 1) / ROWS, h->pz), dim3(nt_of<N>()), lds, st,
-                       f, h->A, h->tw, h->twist, h->dphia, h->mrange, scale);
+    hipLaunchKernelGGL(k_row_adj_r<n>, dim3(n / ROWS, npair), dim3(NT), lds, st, f, h->A, h->twn,
+                       h->twistn, h->dphia, h->mrange, scale, h->pz);
     PT_LAUNCH_CHECK();
   }
+  return PT_OK;
+}
+
+template <int ZB>
+int scatter(pt_tomo* h, hipStream_t st) {
+  ProfScope prof("tomo_scatter", st);
+  hipLaunchKernelGGL(k_scatter_own<ZB>, dim3(h->nswi, (h->pzs / 8 + ZB - 1) / ZB), dim3(64), 0, st,
+                     (f4m*)h->Bg, (f4m*)h->spart, (const float*)h->Q, (const f4m*)h->wadj, h->ent,
+                     h->swi_tile, h->swi_range, h->swi_slot, h->nts, h->pzs);
+  PT_LAUNCH_CHECK();
   return PT_OK;
 }
 
@@ -1065,7 +1048,7 @@ int run_fwd(pt_tomo* h, float2* g, const float2* f, float scale, hipStream_t st)
     dim3 grid(h->nwi, (npair + zper - 1) / zper);
     ProfScope prof("tomo_gather", st);
     hipLaunchKernelGGL(k_gather_tile, grid, dim3(kWorkMax), 0, st, (f4v*)h->Q, (const f4v*)h->Bg,
-                       (const f4v*)h->wfwd, h->ffloor, h->wi_tile, h->wi_range, h->bin_sample, N,
+                       (const f4v*)h->wfwd, h->sfloor, h->wi_tile, h->wi_range, h->bin_sample, N,
                        h->ntile1, h->ntheta * N, npair, zper);
     PT_LAUNCH_CHECK();
   }
@@ -1084,58 +1067,47 @@ int run_fwd(pt_tomo* h, float2* g, const float2* f, float scale, hipStream_t st)
 }
 
 int run_adj(pt_tomo* h, float2* f, const float2* g, float scale, hipStream_t st) {
-  const int N = h->N, M = h->M;
-  const int nthr = 256;
+  const int N = h->N, npair = (h->pz + 1) / 2;
   const bool rl = reg_lines(h);
+  const double sgn = ((N / 2) % 2) ? -1.0 : 1.0;
+  const float oscale = (float)(sgn / (double)N);
   if (rl) {
-    const double sgn = ((N / 2) % 2) ? -1.0 : 1.0;
-    const float oscale = (float)(sgn * kPiRef / (double)h->mu / (double)N);
     const int rc = with_reg_n(N, [&](auto nc) { return adj_lines_r<decltype(nc)::value>(h, g, oscale, st); });
     if (rc) return rc;
-  }
-  if (!rl) {
-    const double sgn = ((N / 2) % 2) ? -1.0 : 1.0;
-    const float oscale = (float)(sgn * kPiRef / (double)h->mu / (double)N);
+  } else {
     const int zq = h->adj_lines;
-    dim3 grid(h->ntheta, (h->pz + zq - 1) / zq);
+    dim3 grid(h->ntheta, (h->pzs + zq - 1) / zq);
     ProfScope prof("tomo_adj_line", st);
     hipLaunchKernelGGL(k_adj_line, grid, dim3(256), line_lds_bytes(N, zq), st, h->Q, g, h->tw,
-                       h->filt, h->plan, oscale, h->n, h->ntheta, h->pz, zq);
+                       h->filt, h->plan, oscale, h->n, h->ntheta, h->pz, h->pzs, zq);
     PT_LAUNCH_CHECK();
   }
   {
-    const float beta = (float)(kPiRef * kPiRef / (double)h->mu);
-    dim3 grid(h->nswi, (h->pz + kZS - 1) / kZS);
-    {
-      ProfScope prof("tomo_scatter", st);
-      hipLaunchKernelGGL(k_scatter_own, grid, dim3(64), 0, st, h->Bg, h->spart, h->Q, h->spos,
-                         h->sfloor, h->ent_s, h->ent_o, h->swi_tile, h->swi_range, h->swi_slot, N,
-                         M, beta, h->nt8, h->pz);
-      PT_LAUNCH_CHECK();
-    }
+    const int rc = h->szb == 4 ? scatter<4>(h, st) : h->szb == 2 ? scatter<2>(h, st)
+                                                                  : scatter<1>(h, st);
+    if (rc) return rc;
     if (h->nfix) {
       ProfScope prof("tomo_scatter_fix", st);
-      hipLaunchKernelGGL(k_scatter_fix, dim3(h->nfix, h->pz), dim3(kTSY * kTSX), 0, st, h->Bg,
-                         h->spart, h->sfix, N, h->nt8, h->pz);
+      hipLaunchKernelGGL(k_scatter_fix, dim3(h->nfix, npair), dim3(kTS * kTS), 0, st,
+                         (f4m*)h->Bg, (const f4m*)h->spart, h->sfix, h->nts, h->pzs / 2);
       PT_LAUNCH_CHECK();
     }
   }
   if (rl) return with_reg_n(N, [&](auto nc) { return adj_grid_r<decltype(nc)::value>(h, f, scale, st); });
   {
     const int cols = h->cols_per_wg;
-    dim3 grid((2 * N + cols - 1) / cols, h->pz);
+    dim3 grid((4 * h->n + cols - 1) / cols, npair);
     ProfScope prof("tomo_col_adj", st);
-    hipLaunchKernelGGL(k_col_adj, grid, dim3(nthr), col_lds_bytes(N, cols), st, h->A, h->Bg, h->tw,
-                       h->twist, h->plan, h->n, ilog2(cols));
+    hipLaunchKernelGGL(k_col_adj, grid, dim3(256), col_lds_bytes(h->n, cols), st, h->A, h->Bg,
+                       h->twn, h->twistn, h->plann, ilog2(cols));
     PT_LAUNCH_CHECK();
   }
   {
     const int rows = h->rows_per_wg;
-    dim3 grid((h->n + rows - 1) / rows, h->pz);
-    size_t lds = line_lds_bytes(N, 2 * rows);
+    dim3 grid((2 * h->n + rows - 1) / rows, npair);
     ProfScope prof("tomo_row_adj", st);
-    hipLaunchKernelGGL(k_row_adj, grid, dim3(nthr), lds, st, f, h->A, h->tw, h->twist, h->dphia,
-                       h->mrange, h->plan, h->n, rows, scale);
+    hipLaunchKernelGGL(k_row_adj, grid, dim3(256), line_lds_bytes(h->n, 2 * rows), st, f, h->A,
+                       h->twn, h->twistn, h->dphia, h->mrange, h->plann, rows, scale, h->pz);
     PT_LAUNCH_CHECK();
   }
   return PT_OK;
@@ -1189,18 +1161,9 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
   PT_REQUIRE(line_lds_bytes(N, 2) <= kLdsCap && col_fits(plan, 1), PT_ERR_SIZE,
              "pt_tomo_create: n too large");
   pt_tomo* h = new pt_tomo();
-  h->ntheta = ntheta; h->pz = pnz; h->n = n; h->N = N; h->plan = plan;
-  // radonusfft.cu:10-12
-  const float eps = 1e-6f;
-  h->mu = (float)(-std::log((double)eps) / (2.0 * N * N));
-  h->M = (int)std::ceil(2 * N / kPiRef *
-                        std::sqrt(-(double)h->mu * std::log((double)eps) +
-                                  ((double)h->mu * N) * ((double)h->mu * N) / 4));
-  if (h->M > 7) {
-    set_error("pt_tomo_create: gridding half-width above 7 is not supported");
-    delete h;
-    return PT_ERR_SIZE;
-  }
+  h->ntheta = ntheta; h->pz = pnz; h->pzs = (pnz + 7) / 8 * 8; h->n = n; h->N = N;
+  h->plan = plan;
+  make_line_plan(n, &h->plann);  // n = 2/3 N factors as N does
   // LDS lines per workgroup of the row and detector-line passes (<= 48 KB);
   // columns per workgroup of the column passes (up to 16: whole cache lines)
   const size_t cap = 48 * 1024;
@@ -1211,18 +1174,22 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
   h->cols_per_wg = cols;
   h->adj_lines = lines_fit(plan, kZQ, cap);
   // host tables
-  std::vector<float2> tw(N), twist(N);
-  std::vector<float> dphi(N), dphia(N);
+  auto line_tables = [](int L, std::vector<float2>& tw, std::vector<float2>& twist,
+                        std::vector<float>& dphi) {
+    tw.resize(L); twist.resize(L); dphi.resize(L);
+    for (int m = 0; m < L; ++m) {
+      const int j = m - L / 2;
+      const double a = -2.0 * kPi * m / L, b = -kPi * j / L;
+      tw[m] = make_float2((float)std::cos(a), (float)std::sin(a));
+      twist[m] = make_float2((float)std::cos(b), (float)std::sin(b));
+      dphi[m] = (float)kb_inverse_ft((double)j / (2.0 * L));
+    }
+  };
+  std::vector<float2> tw, twist, twn, twistn;
+  std::vector<float> dphi, dphia;
   std::vector<int2> mr(N);
-  for (int m = 0; m < N; ++m) {
-    double a = -2.0 * kPi * m / N;
-    tw[m] = make_float2((float)std::cos(a), (float)std::sin(a));
-    const int j = m - N / 2;
-    double b = -kPi * j / N;
-    twist[m] = make_float2((float)std::cos(b), (float)std::sin(b));
-    dphi[m] = (float)kb_inverse_ft((double)j / (2.0 * N));
-    dphia[m] = (float)(std::exp((double)h->mu * (double)j * (double)j) / (2.0 * N));
-  }
+  line_tables(N, tw, twist, dphi);
+  line_tables(n, twn, twistn, dphia);
   // circ mask (kernels.cuh:160-172), float32 arithmetic without contraction
   for (int q = 0; q < N; ++q) {
     volatile float y = (float)(q - N / 2) / (float)N;
@@ -1249,32 +1216,39 @@ extern "C" int pt_tomo_create(int ntheta, int pnz, int n, pt_tomo** out) {
     return PT_ERR_HIP;
   };
   hipError_t e;
+  const size_t ns = (size_t)ntheta * N;
   if ((e = hipMalloc(&h->tw, sizeof(float2) * N))) return fail(e, "tables");
   if ((e = hipMalloc(&h->twist, sizeof(float2) * N))) return fail(e, "tables");
+  if ((e = hipMalloc(&h->twn, sizeof(float2) * n))) return fail(e, "tables");
+  if ((e = hipMalloc(&h->twistn, sizeof(float2) * n))) return fail(e, "tables");
   if ((e = hipMalloc(&h->dphi, sizeof(float) * N))) return fail(e, "tables");
-  if ((e = hipMalloc(&h->dphia, sizeof(float) * N))) return fail(e, "tables");
+  if ((e = hipMalloc(&h->dphia, sizeof(float) * n))) return fail(e, "tables");
   if ((e = hipMalloc(&h->mrange, sizeof(int2) * N))) return fail(e, "tables");
-  if ((e = hipMalloc(&h->spos, sizeof(float2) * (size_t)ntheta * N))) return fail(e, "positions");
-  if ((e = hipMalloc(&h->sfloor, sizeof(int2) * (size_t)ntheta * N))) return fail(e, "positions");
-  if ((e = hipMalloc(&h->ffloor, sizeof(int2) * (size_t)ntheta * N))) return fail(e, "positions");
-  if ((e = hipMalloc(&h->bin_sample, sizeof(int) * (size_t)ntheta * N))) return fail(e, "bins");
-  if ((e = hipMalloc(&h->wfwd, sizeof(float) * 2 * kW * (size_t)ntheta * N))) return fail(e, "weights");
-  const size_t pzp = (size_t)(pnz + 1) / 2 * 2;
+  if ((e = hipMalloc(&h->spos, sizeof(float2) * ns))) return fail(e, "positions");
+  if ((e = hipMalloc(&h->sfloor, sizeof(int2) * ns))) return fail(e, "positions");
+  if ((e = hipMalloc(&h->bin_sample, sizeof(int) * ns))) return fail(e, "bins");
+  if ((e = hipMalloc(&h->wfwd, sizeof(float) * 2 * kW * ns))) return fail(e, "weights");
+  if ((e = hipMalloc(&h->wadj, sizeof(float) * 2 * kW * ns))) return fail(e, "weights");
+  // the adjoint's 2n x 2n grid in blocks of 8 slices, the forward's 2N x 2N in pairs
+  const size_t pzp = (size_t)(pnz + 1) / 2 * 2, pzs = h->pzs;
   if ((e = hipMalloc(&h->A, sizeof(float2) * pzp * N * 2 * N))) return fail(e, "row buffer");
-  if ((e = hipMalloc(&h->Bg, sizeof(float2) * pzp * 4 * N * N))) return fail(e, "grid");
-  if ((e = hipMalloc(&h->Q, sizeof(float2) * pzp * ntheta * N))) return fail(e, "samples");
+  if ((e = hipMalloc(&h->Bg, sizeof(float2) * std::max(pzp * 4 * N * N, pzs * 4 * n * n))))
+    return fail(e, "grid");
+  if ((e = hipMalloc(&h->Q, sizeof(float2) * pzs * ns))) return fail(e, "samples");
   if ((e = hipMemcpy(h->tw, tw.data(), sizeof(float2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->twist, twist.data(), sizeof(float2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
+  if ((e = hipMemcpy(h->twn, twn.data(), sizeof(float2) * n, hipMemcpyHostToDevice))) return fail(e, "copy");
+  if ((e = hipMemcpy(h->twistn, twistn.data(), sizeof(float2) * n, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->dphi, dphi.data(), sizeof(float) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
-  if ((e = hipMemcpy(h->dphia, dphia.data(), sizeof(float) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
+  if ((e = hipMemcpy(h->dphia, dphia.data(), sizeof(float) * n, hipMemcpyHostToDevice))) return fail(e, "copy");
   if ((e = hipMemcpy(h->mrange, mr.data(), sizeof(int2) * N, hipMemcpyHostToDevice))) return fail(e, "copy");
   *out = h;
   return PT_OK;
 }
 
 static void free_bins(pt_tomo* h) {
-  void** ptrs[] = {(void**)&h->wi_tile, (void**)&h->wi_range, (void**)&h->ent_s,
-                   (void**)&h->ent_o, (void**)&h->swi_tile, (void**)&h->swi_range,
+  void** ptrs[] = {(void**)&h->wi_tile, (void**)&h->wi_range, (void**)&h->ent,
+                   (void**)&h->swi_tile, (void**)&h->swi_range,
                    (void**)&h->swi_slot, (void**)&h->sfix, (void**)&h->spart};
   for (void** p : ptrs) {
     if (*p) (void)hipFree(*p);
@@ -1292,8 +1266,9 @@ static int upload(T** dst, const std::vector<T>& v, hipStream_t st) {
 
 extern "C" int pt_tomo_destroy(pt_tomo* h) {
   if (!h) return PT_OK;
-  (void)hipFree(h->tw); (void)hipFree(h->twist); (void)hipFree(h->dphi); (void)hipFree(h->dphia); (void)hipFree(h->wfwd); (void)hipFree(h->filt); (void)hipFree(h->mrange);
-  (void)hipFree(h->spos); (void)hipFree(h->sfloor); (void)hipFree(h->ffloor); (void)hipFree(h->A); (void)hipFree(h->Bg); (void)hipFree(h->Q);
+  void* ptrs[] = {h->tw, h->twist, h->twn, h->twistn, h->dphi, h->dphia, h->filt, h->mrange,
+                  h->spos, h->sfloor, h->wfwd, h->wadj, h->A, h->Bg, h->Q};
+  for (void* p : ptrs) (void)hipFree(p);
   (void)hipFree(h->bin_sample);
   free_bins(h);
   delete h;
@@ -1310,9 +1285,8 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   // takexy (kernels.cuh:84-95): FP64 then float32, clamp at 0.5
   const long ns = (long)nt * N;
   std::vector<float2> pos(ns);
-  std::vector<int2> fl(ns), ff(ns);  // ff: exact floors, as the weights' (k_kb_weights)
+  std::vector<int2> ff(ns);  // exact floors, as the weights' (k_kb_weights)
   const float lim = (float)(0.5 - 1e-5);
-  const float twoN = (float)(2 * N);
   for (int t = 0; t < nt; ++t) {
     const double c = std::cos((double)th[t]), s = std::sin((double)th[t]);
     for (int i = 0; i < N; ++i) {
@@ -1321,20 +1295,18 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
       float y = (float)(-k / N * s);
       if (x >= 0.5f) x = lim;
       if (y >= 0.5f) y = lim;
-      volatile float px = twoN * x, py = twoN * y;
       pos[(long)t * N + i] = make_float2(x, y);
-      fl[(long)t * N + i] = make_int2((int)std::floor(px), (int)std::floor(py));
       ff[(long)t * N + i] =
           make_int2((int)std::floor(2.0 * N * x), (int)std::floor(2.0 * N * y));
     }
   }
   for (long q = 0; q < ns; ++q) {
-    if (fl[q].x < -N || fl[q].x >= N || fl[q].y < -N || fl[q].y >= N) {
+    if (ff[q].x < -N || ff[q].x >= N || ff[q].y < -N || ff[q].y >= N) {
       set_error("pt_tomo_set_theta: sample outside the gridding domain");
       return PT_ERR_ARG;
     }
   }
-  const int M = h->M, twoNi = 2 * N;
+  const int twoNi = 2 * N;
   // gather bins: samples by kTile x kTile tile of their floor position,
   // chunks of at most kWorkMax samples
   const int nt1 = (twoNi + kTile - 1) / kTile;
@@ -1382,62 +1354,57 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
       wtile.push_back((int)tI);
       wrange.push_back(make_int2(s0, s1));
     }
-  // scatter lists: for every kTSY x kTSX grid tile, the samples whose 15 x 15
-  // footprint (periodic in 2N) covers part of it, in sample order, with the
-  // footprint origin relative to the tile in [-2M, tile edge - 1]
-  const int nt8 = (twoNi + kTSX - 1) / kTSX, nty8 = (twoNi + kTSY - 1) / kTSY;
-  const long ntl8 = (long)nt8 * nty8;
-  auto tiles_of = [&](int origin, int edge, int* tl, int* off) {
-    int cntt = 0;
-    for (int k = 0; k <= 2 * M; ++k) {
-      int g = origin + k;
-      g %= twoNi;
-      if (g < 0) g += twoNi;
-      const int t = g / edge;
-      bool seen = false;
-      for (int j = 0; j < cntt; ++j) seen |= (tl[j] == t);
-      if (seen) continue;
-      int o = (origin - t * edge) % twoNi;
-      if (o < 0) o += twoNi;
-      if (o > edge - 1) o -= twoNi;
-      tl[cntt] = t;
-      off[cntt] = o;
-      ++cntt;
-    }
-    return cntt;
+  // scatter lists: for every 8 x 8 tile of the 2n x 2n grid, the samples whose
+  // 8 x 8 footprint (periodic) covers part of it, in sample order, with the
+  // footprint's origin relative to the tile in [-7, 7]; along each axis a
+  // footprint meets the tile of its origin and, unless aligned, the next one
+  const int n = h->n, nts = 2 * n / kTS;
+  const long ntl = (long)nts * nts;
+  auto tiles_of = [&](float x, int* tl, int* off) {
+    int org = n + (int)std::floor(2.0 * n * x) - kWLo;
+    org = org < 0 ? org + 2 * n : org >= 2 * n ? org - 2 * n : org;
+    tl[0] = org / kTS;
+    off[0] = org - tl[0] * kTS;
+    tl[1] = tl[0] + 1 == nts ? 0 : tl[0] + 1;
+    off[1] = off[0] - kTS;
+    return off[0] ? 2 : 1;
   };
-  std::vector<int> ecnt(ntl8 + 1, 0);
-  int tx[4], ox[4], ty[4], oy[4];
+  std::vector<int> ecnt(ntl + 1, 0);
+  int tx[2], ox[2], ty[2], oy[2];
   for (long q = 0; q < ns; ++q) {
-    const int nx = tiles_of(N + fl[q].x - M, kTSX, tx, ox);
-    const int ny = tiles_of(N + fl[q].y - M, kTSY, ty, oy);
+    const int nx = tiles_of(pos[q].x, tx, ox), ny = tiles_of(pos[q].y, ty, oy);
     for (int a = 0; a < ny; ++a)
-      for (int b = 0; b < nx; ++b) ecnt[(long)ty[a] * nt8 + tx[b] + 1]++;
+      for (int b = 0; b < nx; ++b) ecnt[(long)ty[a] * nts + tx[b] + 1]++;
   }
-  for (long i = 0; i < ntl8; ++i) ecnt[i + 1] += ecnt[i];
-  std::vector<int> efill(ecnt.begin(), ecnt.end() - 1), es(ecnt[ntl8]), eo(ecnt[ntl8]);
+  for (long i = 0; i < ntl; ++i) ecnt[i + 1] += ecnt[i];
+  std::vector<int> efill(ecnt.begin(), ecnt.end() - 1);
+  std::vector<int2> ents(ecnt[ntl]);
   for (long q = 0; q < ns; ++q) {
-    const int nx = tiles_of(N + fl[q].x - M, kTSX, tx, ox);
-    const int ny = tiles_of(N + fl[q].y - M, kTSY, ty, oy);
+    const int nx = tiles_of(pos[q].x, tx, ox), ny = tiles_of(pos[q].y, ty, oy);
     for (int a = 0; a < ny; ++a)
-      for (int b = 0; b < nx; ++b) {
-        const long tI = (long)ty[a] * nt8 + tx[b];
-        const int at = efill[tI]++;
-        es[at] = (int)q;
-        eo[at] = (ox[b] + 64) | ((oy[a] + 64) << 8);
-      }
+      for (int b = 0; b < nx; ++b)
+        ents[efill[(long)ty[a] * nts + tx[b]]++] =
+            make_int2((int)q, (ox[b] + kTS) | (int)((unsigned)oy[a] << 8));
   }
+  // Slices per work item (8 szb): as many as leave 4096 wavefronts (4 per SIMD),
+  // since each staged weight and sample index then serves more products.
+  // Entries per work item: at most 512, fewer in small problems, where the
+  // dense tiles around the grid's centre would outlast the others.
+  int szb = 4;
+  while (szb > 1 && ntl * ((h->pzs / 8 + szb - 1) / szb) < 4096) szb /= 2;
+  const long share = (long)ecnt[ntl] * ((h->pzs / 8 + szb - 1) / szb) / 2048;
+  const int chunk = (int)std::min(512L, std::max(64L, share / kSE * kSE));
   std::vector<int> stile, sslot;
   std::vector<int2> srange;
   std::vector<int4> sfix;
   int nslots = 0;
-  for (long tI = 0; tI < ntl8; ++tI) {
+  for (long tI = 0; tI < ntl; ++tI) {
     const int e0 = ecnt[tI], e1 = ecnt[tI + 1];
-    const int nch = std::max(1, (e1 - e0 + kSChunk - 1) / kSChunk);
+    const int nch = std::max(1, (e1 - e0 + chunk - 1) / chunk);
     if (nch > 1) sfix.push_back(make_int4((int)tI, nslots, nch, 0));
     for (int c = 0; c < nch; ++c) {
       stile.push_back((int)tI);
-      srange.push_back(make_int2(std::min(e0 + c * kSChunk, e1), std::min(e0 + (c + 1) * kSChunk, e1)));
+      srange.push_back(make_int2(std::min(e0 + c * chunk, e1), std::min(e0 + (c + 1) * chunk, e1)));
       sslot.push_back(nch > 1 ? nslots + c : -1);
     }
     if (nch > 1) nslots += nch;
@@ -1446,23 +1413,25 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   h->ready = false;
   int rc;
   if ((rc = upload(&h->wi_tile, wtile, st)) || (rc = upload(&h->wi_range, wrange, st)) ||
-      (rc = upload(&h->ent_s, es, st)) || (rc = upload(&h->ent_o, eo, st)) ||
-      (rc = upload(&h->swi_tile, stile, st)) || (rc = upload(&h->swi_range, srange, st)) ||
+      (rc = upload(&h->ent, ents, st)) || (rc = upload(&h->swi_tile, stile, st)) || (rc = upload(&h->swi_range, srange, st)) ||
       (rc = upload(&h->swi_slot, sslot, st)) || (rc = upload(&h->sfix, sfix, st)))
     return rc;
   PT_HIP(hipMalloc(&h->spart,
-                   sizeof(float2) * (size_t)std::max(nslots, 1) * h->pz * kTSY * kTSX));
+                   sizeof(float2) * (size_t)std::max(nslots, 1) * h->pzs * kTS * kTS));
   PT_HIP(hipMemcpyAsync(h->spos, pos.data(), sizeof(float2) * ns, hipMemcpyHostToDevice, st));
-  PT_HIP(hipMemcpyAsync(h->sfloor, fl.data(), sizeof(int2) * ns, hipMemcpyHostToDevice, st));
-  PT_HIP(hipMemcpyAsync(h->ffloor, ff.data(), sizeof(int2) * ns, hipMemcpyHostToDevice, st));
+  PT_HIP(hipMemcpyAsync(h->sfloor, ff.data(), sizeof(int2) * ns, hipMemcpyHostToDevice, st));
   PT_HIP(hipMemcpyAsync(h->bin_sample, list.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_kb_weights, dim3((unsigned)((ns * 2 * kW + 255) / 256)), dim3(256), 0, st,
-                     h->wfwd, h->spos, ns, 2 * N, bessel_i0(kBeta));
-  PT_LAUNCH_CHECK();
+  for (int dir = 0; dir < 2; ++dir) {
+    hipLaunchKernelGGL(k_kb_weights, dim3((unsigned)((ns * 2 * kW + 255) / 256)), dim3(256), 0, st,
+                       dir ? h->wadj : h->wfwd, h->spos, ns, dir ? 2 * n : 2 * N,
+                       bessel_i0(kBeta));
+    PT_LAUNCH_CHECK();
+  }
   PT_HIP(hipStreamSynchronize(st));
   h->ntile1 = nt1;
   h->nwi = (int)wtile.size();
-  h->nt8 = nt8;
+  h->nts = nts;
+  h->szb = szb;
   h->nswi = (int)stile.size();
   h->nfix = (int)sfix.size();
   h->ready = true;

@@ -178,6 +178,34 @@ def test_tomo_fwd_vs_direct_sums(n, pz):
     assert err < 1e-6, err
 
 
+@pytest.mark.parametrize("n,pz,nth", [(4, 1, 7), (8, 3, 7), (20, 2, 7), (36, 9, 7), (60, 5, 40),
+                                      (64, 17, 96), (100, 1, 7), (96, 70, 7), (128, 3, 200)])
+def test_tomo_adj_vs_direct_sums(n, pz, nth):
+    """The adjoint against the FP64 direct adjoint, at sizes around the edges
+    of the gridding: a footprint that wraps onto its own tile (n = 4), slice
+    counts around the blocks of 8, dense centre tiles of several entry chunks,
+    angles on the grid axes.  Tolerance: the gridding kernel's 1e-7 of all
+    samples, of which the edge-replicating pad puts up to four times the
+    output's norm outside the cropped object, plus a few ulp per FFT pass:
+    under 2e-6."""
+    from ptychotomo_amd.radonusfft import radonusfft
+    print(f"tomo adjoint direct sums n={n} pz={pz} nth={nth}", flush=True)
+    rng = np.random.default_rng(n + pz)
+    theta = np.concatenate([[0, np.pi / 4, np.pi / 2, np.pi], rng.uniform(0, np.pi, nth - 4)])
+    theta = theta.astype(np.float32)
+    g = crandn(rng, (nth, pz, n))
+    op = radonusfft(nth, pz, n)
+    th = dev(theta)
+    op.setobj(th.data_ptr())
+    back = torch.zeros((pz, n, n), dtype=torch.complex64, device="cuda")
+    gd = dev(g)
+    op.adj(back.data_ptr(), gd.data_ptr())
+    z = sorted({0, pz // 2, pz - 1})   # the direct sums of some slices
+    err = rel(back.cpu().numpy()[z], ousfft.adj_exact(g[:, z], theta))
+    print(f"rel {err:.2e}")
+    assert err < 2e-6, err
+
+
 def test_tomo_adjoint_zero_border():
     """With a zero object border and zero detector edges the boundary pads
     vanish and the operator pair is exactly adjoint."""
