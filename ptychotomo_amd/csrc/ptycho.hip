@@ -489,6 +489,336 @@ void k_minf(double* __restrict__ partial,
   }
 }
 
+// ------------------------------------------------------------------ one wave per frame
+// Frame transforms of large detectors with 16 values per lane.  A lane that
+// holds a whole frame row (k_minf, tile_body) needs D complex values per array:
+// at D = 32 one wave per SIMD fits, at D = 64 the line search spills (10 ms for
+// a sweep over 14400 frames).
+//
+// D = 32: two lanes per row.  Lane l = 2 ix + s holds the row's elements
+// 2 j + s, j < 16: a 16-point FFT in registers, then one radix-2 step between
+// the two lanes (DPP), after which lane s holds outputs k + 16 s.  The same along
+// the columns after an LDS exchange: lane l = 2 ky + s ends with far-field
+// elements (kx = m + 16 s, ky), m < 16.
+//
+// D = 64, probes up to 16 pixels: only 16 x 16 frame elements are not zero.  With
+// o the probe's offset, output 4 k1 + k0 of a line is
+//   W^(o (4 k1 + k0)) sum_j (x_j W_64^(j k0)) W_16^(j k1):
+// four 16-point FFTs of twisted inputs (K = 4 sub-transforms).  Lane l = ix + 16
+// k0 transforms a row's sub-transform k0; after the exchange lane l = ky takes
+// its column's four sub-transforms in turn (kx = 4 m + c).  5 FFTs of 16 points
+// per lane and frame.  The factor W^(o k) has modulus 1 and is left out: the
+// functional only sees moduli, and the gradient's residual commutes with it.
+template <int D>
+struct WaveFrame;
+
+// the partner lane's value (lane ^ 1)
+__device__ __forceinline__ int dpp_xor1(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true);
+}
+__device__ __forceinline__ float lane_xor1(float x) {
+  return __int_as_float(dpp_xor1(__float_as_int(x)));
+}
+__device__ __forceinline__ double lane_xor1(double x) {
+  return __hiloint2double(dpp_xor1(__double2hiint(x)), dpp_xor1(__double2loint(x)));
+}
+
+// 32-bit words of the 16 complex values of a lane exchanged through the
+// wave's LDS buffer: value j goes to wr(j), comes back from rd(j)
+template <typename C, class FW, class FR>
+__device__ __forceinline__ void wave_exchange(C (&v)[16], float* Ts, FW wr, FR rd) {
+  using R = decltype(v[0].x);
+  int* Ti = reinterpret_cast<int*>(Ts);
+  constexpr int words = sizeof(C) / 4;
+  static_for<0, words>([&](auto pc) {
+    constexpr int part = decltype(pc)::value;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const R x = part < words / 2 ? v[j].x : v[j].y;
+      if constexpr (words == 2) Ti[wr(j)] = __float_as_int(x);
+      else Ti[wr(j)] = (part & 1) ? __double2hiint(x) : __double2loint(x);
+    }
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int b = Ti[rd(j)];
+      R& x = part < words / 2 ? v[j].x : v[j].y;
+      if constexpr (words == 2) x = __int_as_float(b);
+      else x = (part & 1) ? __hiloint2double(b, __double2loint(x))
+                          : __hiloint2double(__double2hiint(x), b);
+    }
+    wave_sync();
+  });
+}
+
+template <>
+struct WaveFrame<32> {
+  static constexpr int kSub = 1;            // column sub-transforms
+  static constexpr int kBuf = 32 * 33;      // floats of the exchange buffer
+  int l, s;
+  __device__ explicit WaveFrame(int lane) : l(lane), s(lane & 1) {}
+  // frame element of value j before the transform; far-field element after it
+  __device__ int ix() const { return l >> 1; }
+  __device__ int iy(int j) const { return 2 * j + s; }
+  __device__ int ky() const { return l >> 1; }
+  __device__ int kx(int m, int) const { return m + 16 * s; }
+  __device__ int wr(int j) const { return (l >> 1) * 33 + j + 16 * s; }
+  __device__ int rd(int j) const { return (2 * j + s) * 33 + (l >> 1); }
+  template <typename C>
+  __device__ __forceinline__ void fwd32(C (&v)[16]) const {
+    using R = decltype(v[0].x);
+    const R sg = s ? (R)-1 : (R)1;
+    reg_fft<16, -1>(v);
+    static_for<0, 16>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const C t = twiddle_ct<32, k, -1>(v[k]);
+      const C u = cmake(t, s ? t.x : v[k].x, s ? t.y : v[k].y);
+      v[k] = cmake(t, lane_xor1(u.x) + sg * u.x, lane_xor1(u.y) + sg * u.y);
+    });
+  }
+  __device__ __forceinline__ void inv32(float2 (&v)[16]) const {
+    const float sg = s ? -1.f : 1.f;
+    static_for<0, 16>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const float2 u = make_float2(lane_xor1(v[k].x) + sg * v[k].x,
+                                   lane_xor1(v[k].y) + sg * v[k].y);
+      const float2 t = twiddle_ct<32, k, 1>(u);
+      v[k] = make_float2(s ? t.x : u.x, s ? t.y : u.y);
+    });
+    reg_fft<16, 1>(v);
+  }
+  // probe element of value j as it enters the transform (tw unused)
+  __device__ float2 twist(float2 x, int, const double2*) const { return x; }
+  template <typename C>
+  __device__ __forceinline__ void rows(C (&v)[16], float* T, const double2*) const {
+    fwd32(v);
+    wave_exchange(v, T, [&](int j) { return wr(j); }, [&](int j) { return rd(j); });
+  }
+  template <typename C>
+  __device__ __forceinline__ void cols(const C (&x)[16], C (&y)[16], int, const double2*) const {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) y[j] = x[j];
+    fwd32(y);
+  }
+  // z += column inverse of sub-transform c (c = 0: the whole)
+  __device__ __forceinline__ void cols_inv(float2 (&y)[16], float2 (&z)[16], int,
+                                           const double2*) const {
+    inv32(y);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) z[j] = y[j];
+  }
+  __device__ __forceinline__ void rows_inv(float2 (&z)[16], float* T, const double2*) const {
+    wave_exchange(z, T, [&](int j) { return rd(j); }, [&](int j) { return wr(j); });
+    inv32(z);
+  }
+  // frame values of a lane after rows_inv: all 16, element (ix, iy(j))
+  static constexpr int kOut = 16;
+  __device__ int out_iy(int j) const { return iy(j); }
+  __device__ float2 out(const float2 (&z)[16], int j) const { return z[j]; }
+  __device__ __forceinline__ void combine(float2 (&)[16]) const {}
+};
+
+template <>
+struct WaveFrame<64> {
+  static constexpr int kSub = 4;
+  static constexpr int kBuf = 16 * 68;
+  int l, k0;
+  __device__ explicit WaveFrame(int lane) : l(lane), k0(lane >> 4) {}
+  __device__ int ix() const { return l & 15; }
+  __device__ int iy(int j) const { return j; }
+  __device__ int ky() const { return l; }
+  __device__ int kx(int m, int c) const { return 4 * m + c; }
+  __device__ int wr(int k1) const { return (l & 15) * 68 + 4 * k1 + k0; }
+  __device__ int rd(int i) const { return i * 68 + l; }
+  // tw[m] = exp(-2 pi i m / 64)
+  static __device__ __forceinline__ float2 mul(float2 x, double2 w) {
+    return cmul(x, make_float2((float)w.x, (float)w.y));
+  }
+  static __device__ __forceinline__ double2 mul(double2 x, double2 w) {
+    return make_double2(x.x * w.x - x.y * w.y, x.x * w.y + x.y * w.x);
+  }
+  static __device__ __forceinline__ float2 mulc(float2 x, double2 w) {
+    return cmulc(x, make_float2((float)w.x, (float)w.y));
+  }
+  __device__ float2 twist(float2 x, int j, const double2* tw) const {
+    return mul(x, tw[(j * k0) & 63]);
+  }
+  // FP32 rows take inputs whose probe carries the twist, FP64 rows twist here
+  __device__ __forceinline__ void rows(float2 (&v)[16], float* T, const double2*) const {
+    reg_fft<16, -1>(v);
+    wave_exchange(v, T, [&](int j) { return wr(j); }, [&](int j) { return rd(j); });
+  }
+  __device__ __forceinline__ void rows(double2 (&v)[16], float* T, const double2* tw) const {
+#pragma unroll
+    for (int j = 1; j < 16; ++j) v[j] = mul(v[j], tw[(j * k0) & 63]);
+    reg_fft<16, -1>(v);
+    wave_exchange(v, T, [&](int j) { return wr(j); }, [&](int j) { return rd(j); });
+  }
+  template <typename C>
+  __device__ __forceinline__ void cols(const C (&x)[16], C (&y)[16], int c,
+                                       const double2* tw) const {
+    y[0] = x[0];
+#pragma unroll
+    for (int j = 1; j < 16; ++j) y[j] = mul(x[j], tw[(j * c) & 63]);
+    reg_fft<16, -1>(y);
+  }
+  __device__ __forceinline__ void cols_inv(float2 (&y)[16], float2 (&z)[16], int c,
+                                           const double2* tw) const {
+    reg_fft<16, 1>(y);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float2 t = mulc(y[j], tw[(j * c) & 63]);
+      z[j] = c ? cadd(z[j], t) : t;
+    }
+  }
+  __device__ __forceinline__ void rows_inv(float2 (&z)[16], float* T, const double2* tw) const {
+    wave_exchange(z, T, [&](int j) { return rd(j); }, [&](int j) { return wr(j); });
+    reg_fft<16, 1>(z);
+#pragma unroll
+    for (int j = 1; j < 16; ++j) z[j] = mulc(z[j], tw[(j * k0) & 63]);
+  }
+  // sum over the four lanes of a row: lane k0 keeps elements 4 k0 .. 4 k0 + 3
+  static constexpr int kOut = 4;
+  __device__ int out_iy(int j) const { return 4 * k0 + j; }
+  __device__ float2 out(const float2 (&z)[16], int j) const { return z[j]; }
+  __device__ __forceinline__ void combine(float2 (&z)[16]) const {
+    half_sum<8>(z, k0 >> 1, 32);
+    half_sum<4>(z, k0 & 1, 16);
+  }
+  template <int H>
+  __device__ __forceinline__ void half_sum(float2 (&z)[16], int up, int mask) const {
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const float2 keep = make_float2(up ? z[H + i].x : z[i].x, up ? z[H + i].y : z[i].y);
+      const float2 give = make_float2(up ? z[i].x : z[H + i].x, up ? z[i].y : z[H + i].y);
+      z[i] = make_float2(keep.x + __shfl_xor(give.x, mask, 64),
+                         keep.y + __shfl_xor(give.y, mask, 64));
+    }
+  }
+};
+
+// exp(-2 pi i m / 64) into LDS (64 x 64 frames)
+template <int D>
+__device__ __forceinline__ void stage_tw64(double2* tw) {
+  if constexpr (D == 64)
+    if (threadIdx.x < 64) tw[threadIdx.x] = make_double2(cospi(threadIdx.x / 32.0), -sinpi(threadIdx.x / 32.0));
+}
+
+// Line-search sums of k_minf (lagr = 0) for 32 x 32 frames and for 64 x 64
+// frames with probes up to 16 pixels: one wave per patch, kMinfWWaves waves per
+// workgroup, one partial per (chunk, workgroup).  A workgroup takes a
+// contiguous range of patches and the workgroups run in XCD-contiguous order,
+// since neighbouring patches read overlapping object rows.  The probe, scaled
+// to the far field and twisted, is staged in LDS in lane order.
+// Bound: vector issue and the LDS exchanges, two waves per SIMD (221 registers;
+// held to three waves it spills 47 and measured 8 % slower).  Four CG steps'
+// sweeps: 119 k frames of 32 x 32 8.9 -> 3.6 ms, 14.4 k frames of 64 x 64 with a
+// 16 x 16 probe 40 -> 1.25 ms (a lane per frame row before).
+constexpr int kMinfWWaves = 4;
+template <int D, int MODEL>
+__global__ __launch_bounds__(WAVE * kMinfWWaves, 2)
+void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
+                 const float2* __restrict__ dir, const float* __restrict__ data,
+                 const float2* __restrict__ prb, const int2* __restrict__ pos,
+                 const double* __restrict__ gammas, int ngam, int chunk, int nz, int n, int S,
+                 int P, int ox, float scale, float cd, const double* __restrict__ skip) {
+  using F = WaveFrame<D>;
+  __shared__ float2 prl[16 * WAVE];
+  __shared__ float Tb[kMinfWWaves][F::kBuf];
+  __shared__ double2 tw[D == 64 ? 64 : 1];
+  __shared__ float gsh[PT_MAX_GAM];
+  __shared__ double red[kMinfWWaves][PT_MAX_GAM];
+  const int c = blockIdx.y;
+  if (skip && skip[2 * c + 1] != 0.0) return;
+  const int wave = threadIdx.x / WAVE, lane = lane_id();
+  const F fr(lane);
+  const int o = D == 32 ? ox : 0;           // frame offset of the probe window
+  const int px = fr.ix() - o;
+  const bool colin = px >= 0 && px < P;
+  stage_tw64<D>(tw);
+  if (threadIdx.x < PT_MAX_GAM)
+    gsh[threadIdx.x] = threadIdx.x < ngam ? (float)gammas[(long)c * ngam + threadIdx.x] : 0.f;
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int py = fr.iy(j) - o;
+      float2 q = make_float2(0.f, 0.f);
+      if (colin && py >= 0 && py < P) q = fr.twist(cscale(prb[(long)px * P + py], scale), j, tw);
+      prl[j * WAVE + lane] = q;
+    }
+  }
+  __syncthreads();
+  float* T = Tb[wave];
+  double acc[PT_MAX_GAM];
+#pragma unroll
+  for (int j = 0; j < PT_MAX_GAM; ++j) acc[j] = 0.0;
+  const long npatch = (long)chunk * S, base = (long)c * npatch;
+  const long per = (npatch + gridDim.x - 1) / gridDim.x;
+  const long b0 = (long)xcd_contig(blockIdx.x, gridDim.x) * per;
+  const long b1 = min(b0 + per, npatch);
+  for (long pl = b0 + wave; pl < b1; pl += kMinfWWaves) {
+    const long p = base + pl;
+    const int2 ps = pos[p];
+    if (ps.x < 0) continue;  // a skipped patch has no far field: its sums do not change
+    const int t = (int)(p / S);
+    const long at = ((long)t * nz + ps.y) * n + ps.x;
+    float2 a[16], b[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int py = fr.iy(j) - o;
+      const bool in = colin && py >= 0 && py < P;
+      const long off = in ? at + (long)py * n + px : at;
+      a[j] = f[off];
+      b[j] = dir[off];
+      if (!in) a[j] = b[j] = make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float2 q = prl[j * WAVE + lane];
+      a[j] = cmul(q, a[j]);
+      b[j] = cmul(q, b[j]);
+    }
+    fr.rows(a, T, tw);
+    fr.rows(b, T, tw);
+    const float* dp = data + p * D * D + fr.ky();
+#pragma unroll 1
+    for (int sub = 0; sub < F::kSub; ++sub) {
+      float d[16], w[16];
+#pragma unroll
+      for (int m = 0; m < 16; ++m) d[m] = dp[fr.kx(m, sub) * D];
+      float2 ya[16], yb[16];
+      fr.cols(a, ya, sub, tw);
+      fr.cols(b, yb, sub, tw);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        d[m] *= cd;
+        if (MODEL == PT_MODEL_GAUSSIAN) d[m] = sqrtf(d[m]);
+      }
+      delta_prep<16, MODEL>(ya, w);
+#pragma unroll 1
+      for (int j = 0; j < PT_MAX_GAM; ++j) {
+        if (j < ngam && gsh[j] != 0.f) acc[0] += (double)delta_part<16, MODEL>(ya, yb, d, w, gsh[j]);
+        const double t0 = acc[0];
+#pragma unroll
+        for (int q = 0; q < PT_MAX_GAM - 1; ++q) acc[q] = acc[q + 1];
+        acc[PT_MAX_GAM - 1] = t0;
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < PT_MAX_GAM; ++j) {
+    const double v = wave_sum(acc[j]);
+    if (lane == 0) red[wave][j] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < ngam) {
+    double v = 0.0;
+    for (int w = 0; w < kMinfWWaves; ++w) v += red[w][threadIdx.x];
+    partial[((long)c * gridDim.x + blockIdx.x) * ngam + threadIdx.x] = v;
+  }
+}
+
 // Line-search sums of k_minf (lagr = 0), organised by the overlap-add
 // tiles: a workgroup of kMinfWaves waves takes one tile, stages the psi and
 // d pixels of its EB x EB extended region once in LDS as (psi, d) pairs
@@ -1002,6 +1332,176 @@ __global__ __launch_bounds__(WAVE * tile_waves<D>()) void k_tile_group(Group<Til
   tile_body<D, MODE>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
 }
 
+// tile_body for 32 x 32 frames and for 64 x 64 frames with probes up to 16
+// pixels (WaveFrame): kTileW waves per tile, each taking every kTileW-th of the
+// tile's patches, adding to the shared LDS tile in turn (a barrier between
+// turns), so the order of the sums is the list's.  With one wave per tile the 30
+// KB tiles left one wave per SIMD.  Bound: the FP64 transform's issue (0.44 ms of
+// 1.10 at 119 k frames of 32 x 32) and the LDS exchanges at two waves per SIMD.
+// Gradient of 14.4 k frames of 64 x 64 1.18 -> 0.44 ms, of 119 k of 32 x 32 1.04 ->
+// 1.10 ms (its FP64 values spill 30 registers; the per-row form is gone all the
+// same: adjoint of 20 k frames of 32 x 32 150 -> 72 us).
+constexpr int kTileW = 4;
+template <int D, int MODE>
+__device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
+  using F = WaveFrame<D>;
+  const int EB = A.EB, n = A.n, P = A.P;
+  extern __shared__ float lds_f[];
+  float2* acc = reinterpret_cast<float2*>(lds_f);
+  double2* tw = reinterpret_cast<double2*>(lds_f + ((2 * EB * EB + 3) & ~3) + 2 * WAVE);
+  const int wave = threadIdx.x / WAVE, lane = lane_id();
+  float* T = reinterpret_cast<float*>(tw + (D == 64 ? 64 : 0)) + wave * F::kBuf;
+  const long tile = xcd_contig(b, nb);
+  const int slotid = A.tile_slot[tile];
+  if (slotid < 0) return;
+  const int tpa = A.nty * A.ntx;
+  const int t = (int)(tile / tpa), rem = (int)(tile - (long)t * tpa);
+  const int y0 = (rem / A.ntx) * A.B, x0 = (rem % A.ntx) * A.B;
+  for (int i = threadIdx.x; i < EB * EB; i += kTileW * WAVE) acc[i] = make_float2(0.f, 0.f);
+  stage_tw64<D>(tw);
+  __syncthreads();
+  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
+  const F fr(lane);
+  const int o = D == 32 ? A.ox : 0;
+  const int px = fr.ix() - o;
+  const bool colin = px >= 0 && px < P;
+  for (int i0 = beg; i0 < end; i0 += kTileW) {
+    const int ii = i0 + wave;
+    const bool active = ii < end;
+    int2 ps = make_int2(0, 0);
+    float2 z[16];
+    if (active) {
+      const long p = A.tile_patch[ii];
+      ps = A.pos[p];
+      const float2 sh = A.shift[p];
+      double2 x[MODE == TILE_GRAD ? 16 : 1];
+      if constexpr (MODE == TILE_GRAD) {
+        // a = coefptycho * F(c * prb * psi), rounded once after an FP64 transform
+        const long at = ((long)t * A.nz + ps.y) * n + ps.x;
+        float2 v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int py = fr.iy(j) - o;
+          const bool in = colin && py >= 0 && py < P;
+          v[j] = A.f[in ? at + (long)py * n + px : at];
+          const float2 q = A.prb[in ? (long)px * P + py : 0];
+          v[j] = in ? cscale(cmul(q, v[j]), A.cs) : make_float2(0.f, 0.f);
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = make_double2((double)v[j].x, (double)v[j].y);
+        fr.rows(x, T, tw);
+      }
+#pragma unroll 1
+      for (int sub = 0; sub < F::kSub; ++sub) {
+        float2 y[16];
+        const long e0 = p * D * D + fr.ky();
+        if constexpr (MODE == TILE_ADJ) {
+          // the per-patch phase removed; at D = 64 also the factor W^(o k) of the
+          // probe's offset, which the sub-transforms leave out
+#pragma unroll
+          for (int m = 0; m < 16; ++m) y[m] = cmulc(A.gin[e0 + fr.kx(m, sub) * D], sh);
+          if constexpr (D == 64) {
+#pragma unroll
+            for (int m = 0; m < 16; ++m)
+              y[m] = F::mulc(y[m], tw[(A.ox * (fr.kx(m, sub) + fr.ky())) & 63]);
+          }
+        } else {
+          {
+            double2 yd[16];
+            fr.cols(x, yd, sub, tw);
+            const double sd = (double)A.cp;
+#pragma unroll
+            for (int m = 0; m < 16; ++m)
+              y[m] = make_float2((float)(yd[m].x * sd), (float)(yd[m].y * sd));
+          }
+          __builtin_amdgcn_sched_barrier(0);  // the data after the FP64 transform: registers
+          float dv[16];
+#pragma unroll
+          for (int m = 0; m < 16; ++m) dv[m] = A.data[e0 + fr.kx(m, sub) * D];
+          // residual as in tile_body
+#pragma unroll
+          for (int m = 0; m < 16; ++m) {
+            const float d = dv[m] * A.cd;
+            const float2 a = y[m];
+            const float aa = a.x * a.x + a.y * a.y;
+            float2 res;
+            if (A.model == PT_MODEL_POISSON) {
+              const float q = d / (aa + 1e-32f);
+              res = make_float2(a.x - q * a.x, a.y - q * a.y);
+            } else {
+              const float mo = sqrtf(aa);
+              const float sd = sqrtf(d);
+              if (mo > 0.f) {
+                const float q = sd / mo;
+                res = make_float2(a.x - q * a.x, a.y - q * a.y);
+              } else {
+                // angle(0) = 0 in the shifted frame
+                res = make_float2(-sd * sh.x, sd * sh.y);
+                if constexpr (D == 64)
+                  res = F::mulc(res, tw[(A.ox * (fr.kx(m, sub) + fr.ky())) & 63]);
+              }
+            }
+            y[m] = res;
+          }
+        }
+        fr.cols_inv(y, z, sub, tw);
+      }
+      fr.rows_inv(z, T, tw);
+      fr.combine(z);
+#pragma unroll
+      for (int j = 0; j < F::kOut; ++j) {
+        const int py = fr.out_iy(j) - o;
+        const bool in = colin && py >= 0 && py < P;
+        const float2 q = A.prb[in ? (long)px * P + py : 0];
+        z[j] = cscale(cmulc(z[j], q), A.out_scale);
+      }
+    }
+    // tile index of each kept value; values outside the probe go to a slot of
+    // the lane's own behind the tile, so that the additions need no branches
+    int at[F::kOut];
+#pragma unroll
+    for (int j = 0; j < F::kOut; ++j) {
+      const int fy = fr.out_iy(j), py = fy - o;
+      at[j] = colin && py >= 0 && py < P ? (ps.y + py - y0) * EB + ps.x + px - x0
+                                         : EB * EB + lane;
+    }
+#pragma unroll 1
+    for (int w = 0; w < kTileW; ++w) {
+      if (w == wave && active) {
+        // all reads, then all writes: the lane's pixels are distinct
+        float2 cur[F::kOut];
+#pragma unroll
+        for (int j = 0; j < F::kOut; ++j) cur[j] = acc[at[j]];
+#pragma unroll
+        for (int j = 0; j < F::kOut; ++j) acc[at[j]] = cadd(cur[j], z[j]);
+      }
+      __syncthreads();
+    }
+  }
+  float2* out = A.scratch + (long)slotid * EB * EB;
+  for (int i = threadIdx.x; i < EB * EB; i += kTileW * WAVE) out[i] = acc[i];
+}
+template <int D, int MODE>
+__global__ __launch_bounds__(WAVE * kTileW, 2) void k_tile_w(TileArgs A) {
+  tile_body_w<D, MODE>(A, blockIdx.x, gridDim.x);
+}
+template <int D, int MODE>
+__global__ __launch_bounds__(WAVE * kTileW, 2) void k_tile_w_group(Group<TileArgs> g) {
+  const int i = group_find(g, blockIdx.x);
+  tile_body_w<D, MODE>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
+}
+// LDS bytes of a k_tile_w workgroup
+template <int D>
+inline size_t tile_w_lds_bytes(int EB) {
+  return sizeof(float) * (size_t)(((2 * EB * EB + 3) & ~3) + 2 * WAVE) +
+         (D == 64 ? 64 * sizeof(double2) : 0) +
+         sizeof(float) * (size_t)kTileW * WaveFrame<D>::kBuf;
+}
+// whether a handle's frames run one wave per frame (WaveFrame)
+inline bool wave_frames(const pt_ptycho* h) {
+  return h->D == 32 || (h->D == 64 && h->P <= 16);
+}
+
 // LDS bytes of a k_tile workgroup
 inline size_t tile_lds_bytes(int D, int EB) {
   const int W = 1, G = 64 / D;
@@ -1081,7 +1581,9 @@ __global__ void k_setup_pos(int2* __restrict__ pos, float2* __restrict__ shift,
   if (i >= np) return;
   const float sx = scan[i], sy = scan[np + i];
   const float rx = roundf(sx), ry = roundf(sy);
-  pos[i] = make_int2((int)rx, (int)ry);
+  // a negative rounded coordinate marks the patch as skipped (x = -1), in y too:
+  // the kernels test x
+  pos[i] = rx < 0.f || ry < 0.f ? make_int2(-1, -1) : make_int2((int)rx, (int)ry);
   // takeshifts (kernels.cuh:306-317): e^{2 pi i frac(x)} * e^{2 pi i frac(y)}
   double ax = 2.0 * kPi * (double)(sx - rx), ay = 2.0 * kPi * (double)(sy - ry);
   double cx = cos(ax), sxn = sin(ax), cy = cos(ay), syn = sin(ay);
@@ -1122,10 +1624,19 @@ inline TileArgs tile_args(const pt_ptycho* h, const float2* gin, const float2* f
 template <int D, int MODE>
 int run_tiles(pt_ptycho* h, const float2* gin, const float2* f, const float* data, float cp,
               float cd, float out_scale, int model, hipStream_t st) {
-  const size_t lds = tile_lds_bytes(D, h->EB);
+  const TileArgs A = tile_args(h, gin, f, data, cp, cd, out_scale, model);
   ProfScope prof(MODE == TILE_GRAD ? "ptycho_grad_tile" : "ptycho_adj_tile", st);
-  hipLaunchKernelGGL((k_tile<D, MODE>), dim3((unsigned)h->ntiles), dim3(WAVE * tile_waves<D>()),
-                     lds, st, tile_args(h, gin, f, data, cp, cd, out_scale, model));
+  if constexpr (D >= 32) {
+    if (wave_frames(h)) {
+      hipLaunchKernelGGL((k_tile_w<D, MODE>), dim3((unsigned)h->ntiles), dim3(WAVE * kTileW),
+                         tile_w_lds_bytes<D>(h->EB), st, A);
+      PT_LAUNCH_CHECK();
+      return PT_OK;
+    }
+  }
+  if constexpr (D != 32)
+    hipLaunchKernelGGL((k_tile<D, MODE>), dim3((unsigned)h->ntiles), dim3(WAVE * tile_waves<D>()),
+                       tile_lds_bytes(D, h->EB), st, A);
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
@@ -1261,12 +1772,27 @@ int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, con
   }
   long np = (long)chunk * h->S;
   int nb = launch_blocks(np, 4 * G, std::max(1, 20480 / nchunk));
+  bool wave = false;
+  if constexpr (D >= 32) {
+    wave = wave_frames(h) && !lagr && dir;
+    if (wave) nb = std::max(1, nb / kMinfWWaves);
+  }
   double* part;
   int rc = minf_partials(h, (size_t)nchunk * nb * ngam, fixed, fixed_cap, &part);
   if (rc) return rc;
   {
   ProfScope prof(lagr ? "ptycho_lagr" : "ptycho_minf", st);
-  if (model == PT_MODEL_POISSON)
+  if constexpr (D >= 32) {
+    if (wave) {
+      auto kern = model == PT_MODEL_POISSON ? k_minf_wave<D, PT_MODEL_POISSON>
+                                            : k_minf_wave<D, PT_MODEL_GAUSSIAN>;
+      hipLaunchKernelGGL(kern, dim3(nb, nchunk), dim3(WAVE * kMinfWWaves), 0, st, part, f, dir,
+                         data, h->prb, h->pos, gammas, ngam, chunk, h->nz, h->n, h->S, h->P,
+                         h->ox, h->c * cp, cd, skip);
+    }
+  }
+  if (wave) {
+  } else if (model == PT_MODEL_POISSON)
     hipLaunchKernelGGL((k_minf<D, PT_MODEL_POISSON>), dim3(nb, nchunk), dim3(WAVE), 0, st,
                        part, f, dir, data, h->prb, h->pos, gammas, ngam, chunk, h->nz, h->n,
                        h->S, h->P, h->ox, h->oy, h->c, cp, cd, model, lagr, skip);
@@ -1520,8 +2046,9 @@ static bool distinct_handles(const A* a, int n) {
 }
 
 // One k_tile_group and one k_fold_group launch (the gradient of
-// pt_ptycho_grad) for the instances idx (at most kGroupMax, detector D)
-template <int D>
+// pt_ptycho_grad) for the instances idx (at most kGroupMax, detector D, all or
+// none with one wave per frame)
+template <int D, bool WF>
 static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, int model,
                           hipStream_t st) {
   Group<TileArgs> g;
@@ -1541,15 +2068,19 @@ static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, i
     fg.gx[k] = fold_blocks(h);
     fg.start[k] = totf;
     totf += fg.gx[k];
-    lds = std::max(lds, tile_lds_bytes(D, h->EB));
+    if constexpr (WF) lds = std::max(lds, tile_w_lds_bytes<D>(h->EB));
+    else lds = std::max(lds, tile_lds_bytes(D, h->EB));
   }
   g.start[n] = tot;
   fg.start[n] = totf;
   g.n = fg.n = n;
   {
     ProfScope prof("ptycho_grad_tile", st);
-    hipLaunchKernelGGL((k_tile_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * tile_waves<D>()), lds,
-                       st, g);
+    if constexpr (WF)
+      hipLaunchKernelGGL((k_tile_w_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * kTileW), lds, st, g);
+    else
+      hipLaunchKernelGGL((k_tile_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * tile_waves<D>()),
+                         lds, st, g);
   }
   PT_LAUNCH_CHECK();
   {
@@ -1565,7 +2096,7 @@ extern "C" int pt_ptycho_grad_group(const pt_ptycho_grad_args* a, int n, int mod
   PT_REQUIRE(n >= 0 && (a || n == 0), PT_ERR_ARG, "pt_ptycho_grad_group: bad argument");
   PT_REQUIRE(model == PT_MODEL_POISSON || model == PT_MODEL_GAUSSIAN, PT_ERR_ARG,
              "pt_ptycho_grad_group: bad model");
-  std::vector<int> bins[4];  // D = 8, 16, 32, 64
+  std::vector<int> bins[5];  // D = 8, 16, 32, 64 (one wave per frame), 64
   for (int i = 0; i < n; ++i) {
     const pt_ptycho_grad_args& x = a[i];
     PT_REQUIRE(x.h && x.grad && x.psi && x.data && x.hh && x.lamd, PT_ERR_ARG,
@@ -1576,21 +2107,22 @@ extern "C" int pt_ptycho_grad_group(const pt_ptycho_grad_args* a, int n, int mod
     PT_REQUIRE(x.rho_dev || x.rho > 0, PT_ERR_ARG,
                "pt_ptycho_grad_group: rho must be positive (instance " + std::to_string(i) + ")");
     const int D = x.h->D;
-    bins[D == 8 ? 0 : D == 16 ? 1 : D == 32 ? 2 : 3].push_back(i);
+    bins[D == 8 ? 0 : D == 16 ? 1 : D == 32 ? 2 : wave_frames(x.h) ? 3 : 4].push_back(i);
   }
   PT_REQUIRE(distinct_handles(a, n), PT_ERR_ARG,
              "pt_ptycho_grad_group: a handle appears twice (its tile scratch would be shared)");
   hipStream_t st = (hipStream_t)stream;
-  for (int b = 0; b < 4; ++b) {
+  for (int b = 0; b < 5; ++b) {
     for (size_t k0 = 0; k0 < bins[b].size(); k0 += kGroupMax) {
       const int m = (int)std::min<size_t>(kGroupMax, bins[b].size() - k0);
       const int* idx = bins[b].data() + k0;
       int rc;
       switch (b) {
-        case 0: rc = run_grad_group<8>(a, idx, m, model, st); break;
-        case 1: rc = run_grad_group<16>(a, idx, m, model, st); break;
-        case 2: rc = run_grad_group<32>(a, idx, m, model, st); break;
-        default: rc = run_grad_group<64>(a, idx, m, model, st); break;
+        case 0: rc = run_grad_group<8, false>(a, idx, m, model, st); break;
+        case 1: rc = run_grad_group<16, false>(a, idx, m, model, st); break;
+        case 2: rc = run_grad_group<32, true>(a, idx, m, model, st); break;
+        case 3: rc = run_grad_group<64, true>(a, idx, m, model, st); break;
+        default: rc = run_grad_group<64, false>(a, idx, m, model, st); break;
       }
       if (rc) return rc;
     }

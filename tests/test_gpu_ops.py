@@ -397,3 +397,67 @@ def test_ptycho_minf_candidate_cancelling_the_far_field():
     for j, g in enumerate(gam):
         ref = f(g) - f0
         assert abs(s[j] - ref) <= 1e-5 * abs(f0) + 1e-4 * abs(ref), (g, s[j], ref)
+
+
+@pytest.mark.parametrize("det,P,n,nz,step", [(32, 32, 64, 64, 8), (32, 20, 70, 61, 5),
+                                             (64, 16, 80, 72, 8), (64, 11, 71, 66, 7)])
+@pytest.mark.parametrize("model", ["poisson", "gaussian"])
+def test_ptycho_large_frames_vs_fp64(det, P, n, nz, step, model):
+    """Fused gradient, line-search sums and adjoint of 32 x 32 and 64 x 64
+    frames against FP64: probes that fill the frame, smaller ones (with an odd
+    size, so an uneven offset), the largest that takes one wave per frame at 64
+    (16); a skipped position in x and one in y, frames of an
+    object that is zero there (|a| = 0).  Tolerances: the FP64 forward's final
+    rounding and an FP32 inverse transform (1e-7 each, 12 passes) in the
+    gradient, FP32 terms summed in FP64 in the functional: under 1e-5."""
+    from ptychotomo_amd import _lib, objects
+    from ptychotomo_amd._dev import ptr, stream
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"large frames det={det} P={P} n={n} nz={nz} {model}", flush=True)
+    rng = np.random.default_rng(det + P)
+    nt, chunk, cp, cd, rho = 4, 2, 1.1, 0.9, 0.7
+    scan = objects.jittered_raster(nt, nz, n, P, step, 1.0, rng)
+    scan[0, 0, 1], scan[1, 1, 2] = -0.8, -0.9
+    prb = crandn(rng, (P, P))
+    op = ptychofft(nt, nz, n, nt, scan.shape[2], det, det, P)
+    sc, pr = dev(scan), dev(prb)
+    op.setobj(sc.data_ptr(), pr.data_ptr())
+    sh = (nt, nz, n)
+    psi = np.exp(1j * 0.3 * rng.standard_normal(sh)).astype(np.complex64)
+    psi[2] = 0
+    d = crandn(rng, sh) * np.float32(0.05)
+    h, lamd = crandn(rng, sh), crandn(rng, sh) * np.float32(0.1)
+    data = rng.poisson(4.0, (nt, scan.shape[2], det, det)).astype(np.float32)
+    far = lambda x: cp * optycho.fwd(x, prb, scan, det, det, np.complex128)  # noqa: E731
+    a, b, q = far(psi), far(d), np.float64(np.float32(cd)) * data
+    if model == "poisson":
+        r = a - q * a / (np.abs(a) ** 2 + 1e-32)
+    else:
+        r = a - np.sqrt(q) * np.exp(1j * np.angle(np.where(a == 0, 0, a)))  # angle(0) = 0
+    ref = cp * optycho.adj(r, prb, scan, nz, n, np.complex128) - rho * (h - psi + lamd / rho)
+    mdl = _lib.PT_MODEL[model]
+    t = {k: dev(v) for k, v in dict(psi=psi, d=d, h=h, lamd=lamd, data=data).items()}
+    out = torch.zeros(sh, dtype=torch.complex64, device="cuda")
+    _lib.call("pt_ptycho_grad", op._h, ptr(out), ptr(t["psi"]), ptr(t["data"]), ptr(t["h"]),
+              ptr(t["lamd"]), rho, None, cp, cd, mdl, stream())
+    eg = rel(out.cpu().numpy(), ref)
+    gam = np.array([0.0, 1.0, 0.25, 2.0 ** -9], np.float64)
+    g = dev(np.tile(gam, nt // chunk))
+    f1 = torch.zeros(nt // chunk * 4, dtype=torch.float64, device="cuda")
+    _lib.call("pt_ptycho_minf", op._h, ptr(f1), ptr(t["psi"]), ptr(t["d"]), ptr(t["data"]),
+              ptr(g), 4, chunk, cp, cd, mdl, 0, None, stream())
+    mlog = lambda x: np.log(np.maximum(x, 1e-32))  # noqa: E731
+    m0, es = np.abs(a), []
+    for c in range(nt // chunk):
+        s = slice(c * chunk, (c + 1) * chunk)
+        for j, gj in enumerate(gam):
+            m = np.abs(a + gj * b)
+            e = m ** 2 - m0 ** 2 - 2 * q * (mlog(m) - mlog(m0)) if model == "poisson" else \
+                (m - np.sqrt(q)) ** 2 - (m0 - np.sqrt(q)) ** 2
+            es.append(abs(float(f1[c * 4 + j]) - e[s].sum()) / max(np.abs(e[s]).sum(), 1e-30))
+    gin = crandn(rng, data.shape)
+    gd = dev(gin)
+    op.adj(out.data_ptr(), gd.data_ptr())
+    ea = rel(out.cpu().numpy(), optycho.adj(gin, prb, scan, nz, n, np.complex128))
+    print(f"grad {eg:.2e} sums {max(es):.2e} adj {ea:.2e}")
+    assert eg < 1e-5 and max(es) < 1e-5 and ea < 1e-5, (eg, es, ea)
