@@ -140,6 +140,10 @@ int pt_ptycho_adj(pt_ptycho* h, void* f, const void* g, pt_stream stream);
 /* Same with the output multiplied by `scale` (coefptycho, solver.py:104,124). */
 int pt_ptycho_fwd_scaled(pt_ptycho* h, void* g, const void* f, float scale, pt_stream stream);
 int pt_ptycho_adj_scaled(pt_ptycho* h, void* f, const void* g, float scale, pt_stream stream);
+/* Far-field intensities (solver.py:115) without the far field: out =
+ * iscale * |scale * F f|^2, out: [ptheta, nscan, detx, dety] float32. */
+int pt_ptycho_intensity(pt_ptycho* h, float* out, const void* f, float scale, float iscale,
+                        pt_stream stream);
 
 /* Fused ptychography gradient of cg_ptycho (solver.py:219-225):
  *   fpsi = coefptycho * F(psi)

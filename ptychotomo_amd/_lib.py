@@ -89,6 +89,7 @@ _SIGS = {
     "pt_ptycho_adj": (c_int, [vp, vp, vp, vp]),
     "pt_ptycho_fwd_scaled": (c_int, [vp, vp, vp, c_float, vp]),
     "pt_ptycho_adj_scaled": (c_int, [vp, vp, vp, c_float, vp]),
+    "pt_ptycho_intensity": (c_int, [vp, vp, vp, c_float, c_float, vp]),
     "pt_ptycho_grad": (c_int, [vp, vp, vp, vp, vp, vp, c_double, vp, c_float, c_float, c_int,
                                vp]),
     "pt_ptycho_minf": (c_int, [vp, vp, vp, vp, vp, vp, c_int, c_int, c_float, c_float, c_int,

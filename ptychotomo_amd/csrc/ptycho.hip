@@ -227,19 +227,25 @@ __device__ __forceinline__ void apply_probe(float2 (&v)[D], const float2* __rest
 }
 
 // ------------------------------------------------------------------ fwd
-template <int D>
-__global__ __launch_bounds__(WAVE) void k_fwd(float2* __restrict__ g, const float2* __restrict__ f,
+// INT = false: the far field with the per-patch phase (g); INT = true: only its
+// intensity scaled by isc (out), in which the phase has no part: 165 MB written
+// at 128^2, 192 angles, 16 x 16 frames instead of the far field written, read
+// and squared in a second pass (98 + 96 -> 59 us).  Bound: the far field or
+// intensity written.
+template <int D, bool INT>
+__global__ __launch_bounds__(WAVE) void k_fwd(float2* __restrict__ g, float* __restrict__ out,
+                                              const float2* __restrict__ f,
                                               const float2* __restrict__ prb,
                                               const int2* __restrict__ pos,
                                               const float2* __restrict__ shift, int pt, int nz, int n,
-                                              int S, int P, int ox, int oy, float cs) {
+                                              int S, int P, int ox, int oy, float cs, float isc) {
   constexpr int G = WAVE / D;
-  // frames up to 32 x 32 transpose one float component at a time (half the
-  // LDS of a complex buffer; at 64 x 64 that form spills registers); frames
-  // up to 16 x 16 read the probe from LDS (a lane's probe column is P-strided
-  // in memory: one cache line per lane and row)
-  __shared__ float Tf[D <= 32 ? G * D * (D + 1) : 1];
-  __shared__ float2 Tc[D <= 32 ? 1 : G * D * (D + 1)];
+  // frames up to 16 x 16 transpose one float component at a time (half the LDS
+  // of a complex buffer; at 64 x 64 that form spills registers) and read the
+  // probe from LDS (a lane's probe column is P-strided in memory: one cache
+  // line per lane and row)
+  __shared__ float Tf[D <= 16 ? G * D * (D + 1) : 1];
+  __shared__ float2 Tc[D <= 16 ? 1 : G * D * (D + 1)];
   __shared__ float2 prl[D <= 16 ? D * D : 1];
   const int lane = lane_id(), slot = lane / D, r = lane % D;
   if constexpr (D <= 16) {
@@ -256,13 +262,18 @@ __global__ __launch_bounds__(WAVE) void k_fwd(float2* __restrict__ g, const floa
     if constexpr (D <= 16) {
       load_rows<D>(v, f, ps, t, r, nz, n, P, ox, oy, active);
       apply_probe<D>(v, prl, r, P, ox, oy, cs);
+      frame_fwd_w<D>(v, Tf, slot, r);
     } else {
       load_frame_row<D>(v, f, prb, ps, t, r, nz, n, P, ox, oy, cs, active);
+      frame_fwd<D>(v, Tc, slot, r);
     }
-    if constexpr (D <= 32) frame_fwd_w<D>(v, Tf, slot, r);
-    else frame_fwd<D>(v, Tc, slot, r);
-    if (active) {
-      float2 sh = shift[p];
+    if (!active) continue;
+    if constexpr (INT) {
+      float* op = out + p * D * D + r;
+#pragma unroll
+      for (int k = 0; k < D; ++k) op[k * D] = (v[k].x * v[k].x + v[k].y * v[k].y) * isc;
+    } else {
+      const float2 sh = shift[p];
       float2* gp = g + p * D * D + r;
 #pragma unroll
       for (int k = 0; k < D; ++k) gp[k * D] = cmul(v[k], sh);
@@ -704,6 +715,36 @@ __device__ __forceinline__ void stage_tw64(double2* tw) {
     if (threadIdx.x < 64) tw[threadIdx.x] = make_double2(cospi(threadIdx.x / 32.0), -sinpi(threadIdx.x / 32.0));
 }
 
+// the probe, scaled and twisted, in lane order: prl[j * WAVE + lane] (one wave)
+template <int D>
+__device__ __forceinline__ void stage_probe(float2* prl, const float2* __restrict__ prb,
+                                            const WaveFrame<D>& fr, int lane, int P, int o,
+                                            float scale, const double2* tw) {
+  const int px = fr.ix() - o;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int py = fr.iy(j) - o;
+    float2 q = make_float2(0.f, 0.f);
+    if (px >= 0 && px < P && py >= 0 && py < P)
+      q = fr.twist(cscale(prb[(long)px * P + py], scale), j, tw);
+    prl[j * WAVE + lane] = q;
+  }
+}
+// a lane's 16 object values of the patch whose first pixel is f[at] (0 outside
+// the probe, read unconditionally)
+template <int D>
+__device__ __forceinline__ void load_frame(float2 (&a)[16], const float2* __restrict__ f,
+                                           const WaveFrame<D>& fr, long at, int n, int P, int o) {
+  const int px = fr.ix() - o;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int py = fr.iy(j) - o;
+    const bool in = px >= 0 && px < P && py >= 0 && py < P;
+    a[j] = f[in ? at + (long)py * n + px : at];
+    if (!in) a[j] = make_float2(0.f, 0.f);
+  }
+}
+
 // Line-search sums of k_minf (lagr = 0) for 32 x 32 frames and for 64 x 64
 // frames with probes up to 16 pixels: one wave per patch, kMinfWWaves waves per
 // workgroup, one partial per (chunk, workgroup).  A workgroup takes a
@@ -733,21 +774,11 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
   const int wave = threadIdx.x / WAVE, lane = lane_id();
   const F fr(lane);
   const int o = D == 32 ? ox : 0;           // frame offset of the probe window
-  const int px = fr.ix() - o;
-  const bool colin = px >= 0 && px < P;
   stage_tw64<D>(tw);
   if (threadIdx.x < PT_MAX_GAM)
     gsh[threadIdx.x] = threadIdx.x < ngam ? (float)gammas[(long)c * ngam + threadIdx.x] : 0.f;
   __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int py = fr.iy(j) - o;
-      float2 q = make_float2(0.f, 0.f);
-      if (colin && py >= 0 && py < P) q = fr.twist(cscale(prb[(long)px * P + py], scale), j, tw);
-      prl[j * WAVE + lane] = q;
-    }
-  }
+  if (wave == 0) stage_probe<D>(prl, prb, fr, lane, P, o, scale, tw);
   __syncthreads();
   float* T = Tb[wave];
   double acc[PT_MAX_GAM];
@@ -764,15 +795,8 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
     const int t = (int)(p / S);
     const long at = ((long)t * nz + ps.y) * n + ps.x;
     float2 a[16], b[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int py = fr.iy(j) - o;
-      const bool in = colin && py >= 0 && py < P;
-      const long off = in ? at + (long)py * n + px : at;
-      a[j] = f[off];
-      b[j] = dir[off];
-      if (!in) a[j] = b[j] = make_float2(0.f, 0.f);
-    }
+    load_frame<D>(a, f, fr, at, n, P, o);
+    load_frame<D>(b, dir, fr, at, n, P, o);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const float2 q = prl[j * WAVE + lane];
@@ -816,6 +840,58 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
     double v = 0.0;
     for (int w = 0; w < kMinfWWaves; ++w) v += red[w][threadIdx.x];
     partial[((long)c * gridDim.x + blockIdx.x) * ngam + threadIdx.x] = v;
+  }
+}
+
+// k_fwd for 32 x 32 frames and for 64 x 64 frames with probes up to 16 pixels
+template <int D, bool INT>
+__global__ __launch_bounds__(WAVE * kMinfWWaves, 3)
+void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* __restrict__ f,
+                const float2* __restrict__ prb, const int2* __restrict__ pos,
+                const float2* __restrict__ shift, long npatch, int nz, int n, int S, int P, int ox,
+                float cs, float isc) {
+  using F = WaveFrame<D>;
+  __shared__ float2 prl[16 * WAVE];
+  __shared__ float Tb[kMinfWWaves][F::kBuf];
+  __shared__ double2 tw[D == 64 ? 64 : 1];
+  const int wave = threadIdx.x / WAVE, lane = lane_id();
+  const F fr(lane);
+  const int o = D == 32 ? ox : 0;
+  stage_tw64<D>(tw);
+  __syncthreads();
+  if (wave == 0) stage_probe<D>(prl, prb, fr, lane, P, o, cs, tw);
+  __syncthreads();
+  const long per = (npatch + gridDim.x - 1) / gridDim.x;
+  const long b0 = (long)xcd_contig(blockIdx.x, gridDim.x) * per;
+  const long b1 = min(b0 + per, npatch);
+  for (long p = b0 + wave; p < b1; p += kMinfWWaves) {
+    const int2 ps = pos[p];
+    const long at = ((p / S) * nz + max(ps.y, 0)) * n + max(ps.x, 0);
+    float2 a[16];
+    load_frame<D>(a, f, fr, at, n, P, o);
+    // a skipped patch (x < 0) has a zero far field
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      a[j] = ps.x < 0 ? make_float2(0.f, 0.f) : cmul(prl[j * WAVE + lane], a[j]);
+    fr.rows(a, Tb[wave], tw);
+    const float2 sh = shift[p];
+    const long e0 = p * D * D + fr.ky();
+#pragma unroll 1
+    for (int sub = 0; sub < F::kSub; ++sub) {
+      float2 y[16];
+      fr.cols(a, y, sub, tw);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        const int kx = fr.kx(m, sub);
+        if constexpr (INT) {
+          out[e0 + kx * D] = (y[m].x * y[m].x + y[m].y * y[m].y) * isc;
+        } else {
+          float2 v = cmul(y[m], sh);
+          if constexpr (D == 64) v = F::mul(v, tw[(ox * (kx + fr.ky())) & 63]);
+          g[e0 + kx * D] = v;
+        }
+      }
+    }
   }
 }
 
@@ -1598,14 +1674,26 @@ int launch_blocks(long work, int per_block, int cap) {
   return (int)b;
 }
 
-template <int D>
-int run_fwd(pt_ptycho* h, float2* g, const float2* f, float scale, hipStream_t st) {
+template <int D, bool INT>
+int run_fwd(pt_ptycho* h, float2* g, float* out, const float2* f, float scale, float isc,
+            hipStream_t st) {
   constexpr int G = WAVE / D;
-  long np = (long)h->pt * h->S;
-  int nb = launch_blocks(np, G, 1 << 20);
+  const long np = (long)h->pt * h->S;
   ProfScope prof("ptycho_fwd", st);
-  hipLaunchKernelGGL(k_fwd<D>, dim3(nb), dim3(WAVE), 0, st, g, f, h->prb, h->pos, h->shift, h->pt,
-                     h->nz, h->n, h->S, h->P, h->ox, h->oy, h->c * scale);
+  if constexpr (D >= 32) {
+    if (wave_frames(h)) {
+      // 4 patches per wave where that leaves whole rounds of the chip
+      hipLaunchKernelGGL((k_fwd_wave<D, INT>), dim3(launch_blocks(np, 4 * kMinfWWaves, 1 << 20)),
+                         dim3(WAVE * kMinfWWaves), 0, st, g, out, f, h->prb, h->pos, h->shift, np,
+                         h->nz, h->n, h->S, h->P, h->ox, h->c * scale, isc);
+      PT_LAUNCH_CHECK();
+      return PT_OK;
+    }
+  }
+  if constexpr (D != 32)
+    hipLaunchKernelGGL((k_fwd<D, INT>), dim3(launch_blocks(np, G, 1 << 20)), dim3(WAVE), 0, st, g,
+                       out, f, h->prb, h->pos, h->shift, h->pt, h->nz, h->n, h->S, h->P, h->ox,
+                       h->oy, h->c * scale, isc);
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
@@ -1846,7 +1934,7 @@ int fwd_impl(pt_ptycho* h, void* g, const void* f, float scale, pt_stream stream
   PT_REQUIRE(h && g && f, PT_ERR_ARG, "pt_ptycho_fwd: null argument");
   PT_REQUIRE(h->ready, PT_ERR_STATE, "pt_ptycho_fwd: set_scan_probe not called");
   hipStream_t st = (hipStream_t)stream;
-  PT_DISPATCH_D(h->D, (run_fwd<DD>(h, (float2*)g, (const float2*)f, scale, st)));
+  PT_DISPATCH_D(h->D, (run_fwd<DD, false>(h, (float2*)g, nullptr, (const float2*)f, scale, 0.f, st)));
 }
 
 template <int MODE>
@@ -2005,6 +2093,14 @@ extern "C" int pt_ptycho_fwd(pt_ptycho* h, void* g, const void* f, pt_stream str
 extern "C" int pt_ptycho_fwd_scaled(pt_ptycho* h, void* g, const void* f, float scale,
                                     pt_stream stream) {
   return fwd_impl(h, g, f, scale, stream);
+}
+
+extern "C" int pt_ptycho_intensity(pt_ptycho* h, float* out, const void* f, float scale,
+                                   float iscale, pt_stream stream) {
+  PT_REQUIRE(h && out && f, PT_ERR_ARG, "pt_ptycho_intensity: null argument");
+  PT_REQUIRE(h->ready, PT_ERR_STATE, "pt_ptycho_intensity: set_scan_probe not called");
+  hipStream_t st = (hipStream_t)stream;
+  PT_DISPATCH_D(h->D, (run_fwd<DD, true>(h, nullptr, out, (const float2*)f, scale, iscale, st)));
 }
 
 static int adj_impl(pt_ptycho* h, void* f, const void* g, float scale, pt_stream stream) {

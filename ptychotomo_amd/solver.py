@@ -222,11 +222,9 @@ class Solver(object):
 
     def fwd_ptycho_batch_dev(self, psi):
         psi = to_dev(psi, c64)
-        far = empty((self.ntheta, self.nscan, self.ndety, self.ndetx))
-        self._ptycho.fwd_scaled(far.data_ptr(), psi.data_ptr(), float(self.coefptycho))
-        data = empty(far.shape, f32)
-        _call("pt_k_intensity", ptr(data), ptr(far), float(1.0 / self.coefdata), far.numel(),
-              stream())
+        data = empty((self.ntheta, self.nscan, self.ndety, self.ndetx), f32)
+        _call("pt_ptycho_intensity", self._ptycho._h, ptr(data), ptr(psi), float(self.coefptycho),
+              float(1.0 / self.coefdata), stream())
         return data
 
     def adj_ptycho(self, data):

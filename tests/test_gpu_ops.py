@@ -461,3 +461,29 @@ def test_ptycho_large_frames_vs_fp64(det, P, n, nz, step, model):
     ea = rel(out.cpu().numpy(), optycho.adj(gin, prb, scan, nz, n, np.complex128))
     print(f"grad {eg:.2e} sums {max(es):.2e} adj {ea:.2e}")
     assert eg < 1e-5 and max(es) < 1e-5 and ea < 1e-5, (eg, es, ea)
+
+
+@pytest.mark.parametrize("det,P", [(8, 5), (16, 16), (16, 11), (32, 32), (32, 17), (64, 16),
+                                   (64, 7), (64, 17)])
+def test_ptycho_intensity(det, P):
+    """Far-field intensities without the far field, one wave per frame or rows
+    per lane, with a skipped position, against FP64; tolerance an FP32
+    transform's (1e-7 per pass, 12 passes, squared): under 5e-6."""
+    from ptychotomo_amd import _lib, objects
+    from ptychotomo_amd._dev import ptr, stream
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"intensity det={det} P={P}", flush=True)
+    rng = np.random.default_rng(det + P)
+    nt, nz, n = 3, 70, 75
+    scan = objects.jittered_raster(nt, nz, n, P, 9, 1.0, rng)
+    scan[1, 0, 3] = -0.7
+    prb, psi = crandn(rng, (P, P)), crandn(rng, (nt, nz, n))
+    op = ptychofft(nt, nz, n, nt, scan.shape[2], det, det, P)
+    sc, pr, pd = dev(scan), dev(prb), dev(psi)
+    op.setobj(sc.data_ptr(), pr.data_ptr())
+    out = torch.full((nt, scan.shape[2], det, det), 7.0, device="cuda")
+    _lib.call("pt_ptycho_intensity", op._h, ptr(out), ptr(pd), 1.3, 0.4, stream())
+    ref = 0.4 * np.abs(1.3 * optycho.fwd(psi, prb, scan, det, det, np.complex128)) ** 2
+    err = rel(out.cpu().numpy(), ref)
+    print(f"rel {err:.2e}")
+    assert err < 5e-6, err
