@@ -239,3 +239,34 @@ def test_training_lowers_loss():
     losses = [float(net.train_step(xd, td, lr=3e-3).item()) for _ in range(40)]
     print("loss", losses[0], losses[-1])
     assert np.all(np.isfinite(losses)) and losses[-1] < 0.5 * losses[0]
+
+
+@pytest.mark.parametrize("D,H,W,cin,cout", [(3, 5, 7, 4, 16), (4, 4, 1, 16, 64), (2, 3, 5, 20, 32),
+                                            (4, 6, 9, 48, 16), (3, 4, 5, 96, 32), (4, 4, 5, 8, 48),
+                                            (8, 12, 20, 16, 16)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_conv_wgrad_edges(D, H, W, cin, cout, shift):
+    """Weight and bias gradients at the edges of the four-channel form: rows
+    shorter than a lane's four voxels, voxel counts that are no multiple of 16,
+    a last column group cut by 27 cin, an unaligned buffer and 48 channels
+    (two-byte form).  FP32 accumulation of bf16 products: 1e-5."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    rng = np.random.default_rng(D * H * W + cin + cout)
+    x = bf16_round(rng.standard_normal((D, H, W, cin)))
+    dy = bf16_round(rng.standard_normal((D, H, W, cout)))
+
+    def place(a):
+        buf = torch.zeros(a.size + 8, dtype=torch.int16, device="cuda")
+        buf[shift:shift + a.size] = dev(bf16_bits(a)).reshape(-1)
+        return buf[shift:shift + a.size]
+    xd, dyd = place(x), place(dy)
+    dw = torch.zeros(cout * 27 * cin, dtype=torch.float32, device="cuda")
+    db = torch.zeros(cout, dtype=torch.float32, device="cuda")
+    part = torch.zeros(1 << 20, dtype=torch.float32, device="cuda")
+    bpart = torch.zeros(256 * 64, dtype=torch.float64, device="cuda")
+    _lib.call("pt_nn_conv3d_wgrad", ptr(dw), ptr(db), ptr(part), part.numel(), ptr(bpart),
+              ptr(dyd), ptr(xd), D, H, W, cin, cout, stream())
+    rdw, rdb = on.conv3d_dw(dy, x)
+    assert relerr(dw.cpu().numpy().reshape(cout, 27, cin), rdw) < 1e-5
+    assert relerr(db.cpu().numpy(), rdb) < 1e-5
