@@ -393,6 +393,15 @@ int pt_k_ls_begin(double* state, double* cand, int nseg, int ngam, pt_stream str
 int pt_k_ls_select(double* state, double* cand, double* cand_next, double* step, const double* f1,
                    const double* f2, const double* w, int nseg, int ngam, int ngam_next, int last,
                    pt_stream stream);
+/* cg_tomo's whole line search (solver.py:171-183): the halving rule on
+ * w[0]*||K*(Ru + g Rd) - xi0||^2 + w[1]*||J(u + g d) - xi1||^2 from state[0]
+ * down to 1e-12, as pt_k_ls_begin and sweeps of pt_k_tomo_minf, pt_k_reg_minf
+ * and pt_k_ls_select give it; writes step = {gamma, 0}, state = {gamma, 1}.
+ * K, Ru, Rd, xi0 have len elements, u and d [nz,ny,nx], xi1 [3,nz,ny,nx]. */
+int pt_k_tomo_linesearch(double* state, double* step, const void* K, const void* Ru,
+                         const void* Rd, const void* xi0, const void* u, const void* d,
+                         const void* xi1, const double* w, long len, int nz, int ny, int nx,
+                         pt_stream stream);
 /* Residual balancing (solver.py:267-282): rho_tau = {rho, tau} updated in
  * place from norms = {||psi-h||^2, ||h-h0||^2, ||phi-e||^2, ||e-e0||^2}. */
 int pt_k_penalty(double* rho_tau, const double* norms, pt_stream stream);

@@ -135,6 +135,7 @@ _SIGS = {
     "pt_k_dai_yuan": (c_int, [vp, vp, c_int, vp]),
     "pt_k_ls_begin": (c_int, [vp, vp, c_int, c_int, vp]),
     "pt_k_ls_select": (c_int, [vp, vp, vp, vp, vp, vp, vp, c_int, c_int, c_int, c_int, vp]),
+    "pt_k_tomo_linesearch": (c_int, [vp] * 10 + [c_long, c_int, c_int, c_int, vp]),
     "pt_k_penalty": (c_int, [vp, vp, vp]),
     "pt_nn_conv3d": (c_int, [vp, vp, vp, vp, c_int, c_int, c_int, c_int, c_int, c_int, vp]),
     "pt_nn_conv3d_wflip": (c_int, [vp, vp, c_int, c_int, vp]),

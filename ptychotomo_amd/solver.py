@@ -44,16 +44,15 @@ PLANCK_CONSTANT = 6.58211928e-19  # [keV*s]   solver.py:15
 SPEED_OF_LIGHT = 299792458e+2     # [cm/s]    solver.py:16
 
 _MAXGAM = 8      # candidate slots of the line-search buffers (gamma = 0 + 7 halvings)
-# halvings per sweep of the device line searches; every schedule covers at least
-# 41 halvings (2 -> below 1e-12), so the halving rule is followed to its end.
-# cg_tomo's evaluations are cheap: 7 per sweep.  cg_ptycho's first CG step starts
+# halvings per sweep of cg_ptycho's device line searches; every schedule covers at
+# least 41 halvings (2 -> below 1e-12), so the halving rule is followed to its end
+# (cg_tomo's search is one call, pt_k_tomo_linesearch).  The first CG step starts
 # at gamma = 2 and usually accepts after 3-4 halvings (one sweep of 5); the later
 # steps start from the previous step, accept it about three times in four
 # (256^3: 212 of 288 chunk searches), and otherwise mostly within 5 more
 # halvings (sweeps of 1, 5, then 7).  A sweep costs the two far-field
 # transforms of every open chunk plus each candidate's sums (about a fifth of
 # the transforms' cost each)
-_TSCHED = (7,) * 6
 _PSCHED_FIRST = (5,) + (7,) * 6
 _PSCHED_LATER = (1, 5) + (7,) * 6
 # device scalar block (FP64): 1, rho, tau, takexi {pshift, cos, sin, kfac},
@@ -314,20 +313,15 @@ class Solver(object):
             gamma = 0
         return gamma
 
-    def _line_search_dev(self, w, nseg, evalf, weights, sched=_TSCHED):
+    def _line_search_gen(self, w, nseg, weights, sched):
         """The halving rule of line_search for nseg independent segments, on
         the device: sweeps of sched[i] halvings (plus gamma = 0) until every
-        segment has accepted a step (a schedule covers 2 -> 1e-12).
-        evalf(cand, ngam, state, f1, f2) enqueues the two functional terms
-        (their change from gamma = 0) at the ngam candidate slots per segment,
-        skipping finished segments; weights points to their two FP64 weights."""
-        for req in self._line_search_gen(w, nseg, weights, sched):
-            evalf(*req)
-
-    def _line_search_gen(self, w, nseg, weights, sched=_TSCHED):
-        """_line_search_dev as a generator: yields (cand, ngam, state, f1, f2)
-        where the evaluation is to be enqueued (by the caller, alone or in a
-        group of instances), then enqueues the sweep's selection.  Consecutive
+        segment has accepted a step (a schedule covers 2 -> 1e-12).  A
+        generator: yields (cand, ngam, state, f1, f2) where the two functional
+        terms (their change from gamma = 0) are to be evaluated at the ngam
+        candidate slots per segment, skipping finished segments (by the
+        caller, alone or in a group of instances), then enqueues the sweep's
+        selection; weights points to the terms' two FP64 weights.  Consecutive
         sweeps alternate between two candidate buffers."""
         st = stream()
         bufs = (w["cand"], w["cand2"])
@@ -392,14 +386,9 @@ class Solver(object):
             grad0 = grad
             self._tomo.fwd_scaled(Rd.data_ptr(), d.data_ptr(), ct)
 
-            def evalf(cand, ng, state, f1, f2):
-                _call("pt_k_tomo_minf", ptr(f1), ptr(K), ptr(Ru), ptr(Rd), ptr(xi0), ptr(cand),
-                      ng, lenp, ptr(state), st)
-                _call("pt_k_reg_minf", ptr(f2), ptr(u), ptr(d), ptr(xi1), ptr(cand), ng,
-                      nz, n, n, ptr(state), st)
-
             # minf = rho*|K R u - xi0|^2 + tau*|J u - xi1|^2 (solver.py:181-182)
-            self._line_search_dev(w, 1, evalf, _dp(blk, _RHO))
+            _call("pt_k_tomo_linesearch", ptr(w["state"]), ptr(w["step"]), ptr(K), ptr(Ru),
+                  ptr(Rd), ptr(xi0), ptr(u), ptr(d), ptr(xi1), _dp(blk, _RHO), lenp, nz, n, n, st)
             _call("pt_k_axpy_seg", ptr(u), ptr(w["step"]), ptr(d), lenu, 1, st)
             _call("pt_k_axpy_seg", ptr(Ru), ptr(w["step"]), ptr(Rd), lenp, 1, st)
             if hist is not None:

@@ -487,3 +487,48 @@ def test_ptycho_intensity(det, P):
     err = rel(out.cpu().numpy(), ref)
     print(f"rel {err:.2e}")
     assert err < 5e-6, err
+
+
+@pytest.mark.parametrize("nt,nz,n", [(1, 1, 4), (3, 5, 12), (24, 24, 36)])
+@pytest.mark.parametrize("fit", [1.0, 2.0 ** -7, 2.0 ** -8, 2.0 ** -23, -1.0])
+def test_tomo_linesearch_follows_the_sweeps(nt, nz, n, fit):
+    """pt_k_tomo_linesearch against the same search from its parts (sweeps of 7
+    candidates): accepted in the first group, in its last slot, in the next
+    groups, and never (an ascent direction: step 0).  The residual is the
+    direction's image times `fit`, so steps below 2 fit decrease the functional;
+    whole halvings, so the steps are equal."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    print(f"tomo line search nt={nt} nz={nz} n={n} fit={fit}", flush=True)
+    rng = np.random.default_rng(n)
+    K, Rd, Ru = (crandn(rng, (nt, nz, n)) for _ in range(3))
+    u, d = crandn(rng, (nz, n, n)), crandn(rng, (nz, n, n))
+    J = lambda v: np.stack([  # noqa: E731
+        np.pad(np.diff(v, axis=2), ((0, 0), (0, 0), (0, 1))),
+        np.pad(np.diff(v, axis=1), ((0, 0), (0, 1), (0, 0))),
+        np.pad(np.diff(v, axis=0), ((0, 1), (0, 0), (0, 0)))]) * (2 / np.sqrt(3))
+    # just below the crossing, away from ties
+    xi0 = K * (Ru + 0.9 * fit * Rd)
+    xi1 = J(u + 0.9 * fit * d)
+    t = {k: dev(np.ascontiguousarray(v, dtype=np.complex64)) for k, v in
+         dict(K=K, Ru=Ru, Rd=Rd, xi0=xi0, u=u, d=d, xi1=xi1).items()}
+    z = lambda *v: torch.tensor(v, dtype=torch.float64, device="cuda")  # noqa: E731
+    w, st = z(0.5, 0.25), stream()
+    state, step = z(2.0, 0.0), z(7.0, 7.0)
+    _lib.call("pt_k_tomo_linesearch", ptr(state), ptr(step), ptr(t["K"]), ptr(t["Ru"]),
+              ptr(t["Rd"]), ptr(t["xi0"]), ptr(t["u"]), ptr(t["d"]), ptr(t["xi1"]), ptr(w),
+              K.size, nz, n, n, st)
+    s2, p2, c, f1, f2 = z(2.0, 0.0), z(7.0, 7.0), z(*[0.0] * 8), z(*[0.0] * 8), z(*[0.0] * 8)
+    _lib.call("pt_k_ls_begin", ptr(s2), ptr(c), 1, 8, st)
+    for sw in range(6):
+        _lib.call("pt_k_tomo_minf", ptr(f1), ptr(t["K"]), ptr(t["Ru"]), ptr(t["Rd"]),
+                  ptr(t["xi0"]), ptr(c), 8, K.size, ptr(s2), st)
+        _lib.call("pt_k_reg_minf", ptr(f2), ptr(t["u"]), ptr(t["d"]), ptr(t["xi1"]), ptr(c), 8,
+                  nz, n, n, ptr(s2), st)
+        _lib.call("pt_k_ls_select", ptr(s2), ptr(c), ptr(c), ptr(p2), ptr(f1), ptr(f2), ptr(w),
+                  1, 8, 8, int(sw == 5), st)
+    got, ref = step.cpu().numpy(), p2.cpu().numpy()
+    print(got, ref)
+    assert np.array_equal(got, ref) and np.array_equal(state.cpu().numpy(), s2.cpu().numpy())
+    if fit > 2.0 ** -20:
+        assert 0.45 * fit < got[0] <= 1.8 * fit
