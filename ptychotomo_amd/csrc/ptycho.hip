@@ -148,13 +148,17 @@ __device__ __forceinline__ void transpose_w64(double2 (&w)[D], float* Ts, int r)
 // CG steps the FP32 trajectory then parts from the exact one by 3e-4 .. 1e-2
 // depending on the FFT's operation order.  The FP64 transform leaves only
 // the final rounding (relative, per entry).
-template <int D>
-__device__ __forceinline__ void frame_fwd64_w(float2 (&v)[D], float* T, int slot, int r, float s) {
+// mid() is called between the two passes (loads in flight during the second).
+template <int D, class F>
+__device__ __forceinline__ void frame_fwd64_w(float2 (&v)[D], float* T, int slot, int r, float s,
+                                              F mid) {
   double2 w[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) w[k] = make_double2((double)v[k].x, (double)v[k].y);
   reg_fft<D, -1>(w);
   transpose_w64<D, true>(w, T + slot * D * (D + 1), r);
+  __builtin_amdgcn_sched_barrier(0);
+  mid();
   reg_fft<D, -1>(w);
   const double sd = (double)s;
 #pragma unroll
@@ -1242,8 +1246,19 @@ struct TileArgs {
   float cs, cp, cd, out_scale;
 };
 
-// body of workgroup b of nb (one per tile)
-template <int D, int MODE>
+// body of workgroup b of nb (one per tile).  MODEL: the gradient's data model (any
+// value for the adjoint).  FULL: the probe covers the frame, so every frame
+// element is added without a bounds check.
+// The data column is loaded between the two passes of the FP64 transform: loaded
+// with the object rows it held D registers through the first pass, and with the
+// run-time model and bounds masks the 16 x 16 gradient took 256 registers and
+// spilled 31 of them.  Now 130, three waves per SIMD (the LDS tile's limit); at
+// 256^3, 384 angles, 1.43 M frames 1.54 -> 1.19 ms per launch.  Bound: vector issue
+// of the FP64 transform, residual and inverse (about 1700 instructions per four
+// frames, 1.0 ms).  The loads do not branch: a branch between the passes splits
+// the FP64 transform into two blocks, the compiler contracts its products
+// differently, and the gradient differs in the last bit.
+template <int D, int MODE, int MODEL, bool FULL>
 __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
   float2* __restrict__ scratch = A.scratch;
   const float2* __restrict__ gin = A.gin;
@@ -1255,8 +1270,8 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
   const int* __restrict__ tile_start = A.tile_start;
   const int* __restrict__ tile_patch = A.tile_patch;
   const int* __restrict__ tile_slot = A.tile_slot;
-  const int nty = A.nty, ntx = A.ntx, B = A.B, EB = A.EB, nz = A.nz, n = A.n, P = A.P;
-  const int ox = A.ox, oy = A.oy, model = A.model;
+  const int nty = A.nty, ntx = A.ntx, B = A.B, EB = A.EB, nz = A.nz, n = A.n;
+  const int P = FULL ? D : A.P, ox = FULL ? 0 : A.ox, oy = FULL ? 0 : A.oy;
   const float cs = A.cs, cp = A.cp, cd = A.cd, out_scale = A.out_scale;
   constexpr int G = WAVE / D;
   constexpr int W = tile_waves<D>();
@@ -1309,19 +1324,16 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
         for (int k = 0; k < D; ++k) v[k] = make_float2(0.f, 0.f);
       }
     } else {
-      // every global load of the group first (one memory round trip)
       load_rows<D>(v, f, ps, t, r, nz, n, P, ox, oy, active);
-      float dv[D];
-      {
-        const float* dp = data + p * D * D + r;
-#pragma unroll
-        for (int k = 0; k < D; ++k) dv[k] = active ? dp[k * D] : 0.f;
-      }
-      const float2 sh = active ? shift[p] : make_float2(1.f, 0.f);
 #pragma unroll
       for (int k = 0; k < D; ++k) v[k] = cscale(cmul(prv(k), v[k]), cs);
       // a = coefptycho * F(c * prb * psi), rounded once after an FP64 transform
-      frame_fwd64_w<D>(v, T, slot, r, cp);
+      float dv[D];
+      frame_fwd64_w<D>(v, T, slot, r, cp, [&]() {
+        const float* dp = data + p * D * D + r;
+#pragma unroll
+        for (int k = 0; k < D; ++k) dv[k] = dp[k * D];  // patch 0's where not active
+      });
       // residual in the unshifted frame (the per-patch unimodular factor of
       // kernels.cuh:319-355 cancels: r(s*a) = s*r(a), F* removes s again)
       if (active) {
@@ -1331,7 +1343,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
           const float2 a = v[k];
           const float aa = a.x * a.x + a.y * a.y;
           float2 res;
-          if (model == PT_MODEL_POISSON) {
+          if constexpr (MODEL == PT_MODEL_POISSON) {
             // IEEE division: where |a| is small the quotient's relative error
             // becomes a large absolute error of the residual, and a 1-ulp
             // reciprocal there moves a 36-step CG run 6x farther from FP64
@@ -1345,6 +1357,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
               res = make_float2(a.x - q * a.x, a.y - q * a.y);
             } else {
               // angle(0) = 0 in the shifted frame: r = -sqrt(d) there
+              const float2 sh = shift[p];
               res = make_float2(-sd * sh.x, sd * sh.y);
             }
           }
@@ -1397,15 +1410,16 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
   float2* out = scratch + (long)slotid * EB * EB;
   for (int i = threadIdx.x; i < EB * EB; i += W * WAVE) out[i] = acc[i];
 }
-template <int D, int MODE>
-__global__ __launch_bounds__(WAVE * tile_waves<D>()) void k_tile(TileArgs A) {
-  tile_body<D, MODE>(A, blockIdx.x, gridDim.x);
+template <int D, int MODE, int MODEL, bool FULL>
+__global__ __launch_bounds__(WAVE * tile_waves<D>()) __attribute__((amdgpu_waves_per_eu(D <= 16 ? 3 : 1))) void k_tile(TileArgs A) {
+  tile_body<D, MODE, MODEL, FULL>(A, blockIdx.x, gridDim.x);
 }
 // the same for a group of instances (their tile grids flattened)
-template <int D, int MODE>
-__global__ __launch_bounds__(WAVE * tile_waves<D>()) void k_tile_group(Group<TileArgs> g) {
+template <int D, int MODE, int MODEL, bool FULL>
+__global__ __launch_bounds__(WAVE * tile_waves<D>()) __attribute__((amdgpu_waves_per_eu(D <= 16 ? 3 : 1)))
+void k_tile_group(Group<TileArgs> g) {
   const int i = group_find(g, blockIdx.x);
-  tile_body<D, MODE>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
+  tile_body<D, MODE, MODEL, FULL>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
 }
 
 // tile_body for 32 x 32 frames and for 64 x 64 frames with probes up to 16
@@ -1698,6 +1712,30 @@ int run_fwd(pt_ptycho* h, float2* g, float* out, const float2* f, float scale, f
   return PT_OK;
 }
 
+// the probe covers the frame (no offset): the FULL kernels
+template <int D>
+inline bool minf_full(const pt_ptycho* h) {
+  return h->P == D && h->ox == 0 && h->oy == 0;
+}
+// fn(k_tile<...>, k_tile_group<...>) for the model and probe form (frames of 64
+// x 64 come here with a probe beyond 16 pixels, rarely the whole frame: one form)
+template <int D, int MODE, class F>
+inline void tile_dispatch(int model, bool full, F&& fn) {
+  auto by_full = [&](auto model_c) {
+    constexpr int M = decltype(model_c)::value;
+    if constexpr (D <= 16) {
+      if (full) {
+        fn(k_tile<D, MODE, M, true>, k_tile_group<D, MODE, M, true>);
+        return;
+      }
+    }
+    fn(k_tile<D, MODE, M, false>, k_tile_group<D, MODE, M, false>);
+  };
+  if constexpr (MODE == TILE_ADJ) by_full(std::integral_constant<int, PT_MODEL_POISSON>());
+  else if (model == PT_MODEL_POISSON) by_full(std::integral_constant<int, PT_MODEL_POISSON>());
+  else by_full(std::integral_constant<int, PT_MODEL_GAUSSIAN>());
+}
+
 inline TileArgs tile_args(const pt_ptycho* h, const float2* gin, const float2* f, const float* data,
                           float cp, float cd, float out_scale, int model) {
   TileArgs A;
@@ -1723,8 +1761,10 @@ int run_tiles(pt_ptycho* h, const float2* gin, const float2* f, const float* dat
     }
   }
   if constexpr (D != 32)
-    hipLaunchKernelGGL((k_tile<D, MODE>), dim3((unsigned)h->ntiles), dim3(WAVE * tile_waves<D>()),
-                       tile_lds_bytes(D, h->EB), st, A);
+    tile_dispatch<D, MODE>(model, minf_full<D>(h), [&](auto kern, auto) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)h->ntiles), dim3(WAVE * tile_waves<D>()),
+                         tile_lds_bytes(D, h->EB), st, A);
+    });
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
@@ -1762,11 +1802,6 @@ struct RhoTerm {
   double* f2 = nullptr;
 };
 
-// the probe covers the frame (no offset): k_minf_tile's FULL path
-template <int D>
-inline bool minf_full(const pt_ptycho* h) {
-  return h->P == D && h->ox == 0 && h->oy == 0;
-}
 // whether a line search of this handle runs on the overlap-add tiles: frames
 // up to 16 x 16 whose extended tile fits the staging, where a tile holds on
 // average at least one patch per slot of its workgroup (sparser tiles would
@@ -2143,10 +2178,10 @@ static bool distinct_handles(const A* a, int n) {
 
 // One k_tile_group and one k_fold_group launch (the gradient of
 // pt_ptycho_grad) for the instances idx (at most kGroupMax, detector D, all or
-// none with one wave per frame)
+// none with one wave per frame, all or none with a probe that covers the frame)
 template <int D, bool WF>
 static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, int model,
-                          hipStream_t st) {
+                          bool full, hipStream_t st) {
   Group<TileArgs> g;
   Group<FoldArgs> fg;
   size_t lds = 0;
@@ -2175,8 +2210,9 @@ static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, i
     if constexpr (WF)
       hipLaunchKernelGGL((k_tile_w_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * kTileW), lds, st, g);
     else
-      hipLaunchKernelGGL((k_tile_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * tile_waves<D>()),
-                         lds, st, g);
+      tile_dispatch<D, TILE_GRAD>(model, full, [&](auto, auto kern) {
+        hipLaunchKernelGGL(kern, dim3(tot), dim3(WAVE * tile_waves<D>()), lds, st, g);
+      });
   }
   PT_LAUNCH_CHECK();
   {
@@ -2192,7 +2228,8 @@ extern "C" int pt_ptycho_grad_group(const pt_ptycho_grad_args* a, int n, int mod
   PT_REQUIRE(n >= 0 && (a || n == 0), PT_ERR_ARG, "pt_ptycho_grad_group: bad argument");
   PT_REQUIRE(model == PT_MODEL_POISSON || model == PT_MODEL_GAUSSIAN, PT_ERR_ARG,
              "pt_ptycho_grad_group: bad model");
-  std::vector<int> bins[5];  // D = 8, 16, 32, 64 (one wave per frame), 64
+  // D = 8 and 16 (probe partial / full), 32, 64 (one wave per frame), 64
+  std::vector<int> bins[7];
   for (int i = 0; i < n; ++i) {
     const pt_ptycho_grad_args& x = a[i];
     PT_REQUIRE(x.h && x.grad && x.psi && x.data && x.hh && x.lamd, PT_ERR_ARG,
@@ -2203,22 +2240,28 @@ extern "C" int pt_ptycho_grad_group(const pt_ptycho_grad_args* a, int n, int mod
     PT_REQUIRE(x.rho_dev || x.rho > 0, PT_ERR_ARG,
                "pt_ptycho_grad_group: rho must be positive (instance " + std::to_string(i) + ")");
     const int D = x.h->D;
-    bins[D == 8 ? 0 : D == 16 ? 1 : D == 32 ? 2 : wave_frames(x.h) ? 3 : 4].push_back(i);
+    const int b = D == 8    ? (minf_full<8>(x.h) ? 1 : 0)
+                  : D == 16 ? 2 + (minf_full<16>(x.h) ? 1 : 0)
+                  : D == 32 ? 4
+                            : wave_frames(x.h) ? 5 : 6;
+    bins[b].push_back(i);
   }
   PT_REQUIRE(distinct_handles(a, n), PT_ERR_ARG,
              "pt_ptycho_grad_group: a handle appears twice (its tile scratch would be shared)");
   hipStream_t st = (hipStream_t)stream;
-  for (int b = 0; b < 5; ++b) {
+  for (int b = 0; b < 7; ++b) {
     for (size_t k0 = 0; k0 < bins[b].size(); k0 += kGroupMax) {
       const int m = (int)std::min<size_t>(kGroupMax, bins[b].size() - k0);
       const int* idx = bins[b].data() + k0;
       int rc;
       switch (b) {
-        case 0: rc = run_grad_group<8, false>(a, idx, m, model, st); break;
-        case 1: rc = run_grad_group<16, false>(a, idx, m, model, st); break;
-        case 2: rc = run_grad_group<32, true>(a, idx, m, model, st); break;
-        case 3: rc = run_grad_group<64, true>(a, idx, m, model, st); break;
-        default: rc = run_grad_group<64, false>(a, idx, m, model, st); break;
+        case 0:
+        case 1: rc = run_grad_group<8, false>(a, idx, m, model, b == 1, st); break;
+        case 2:
+        case 3: rc = run_grad_group<16, false>(a, idx, m, model, b == 3, st); break;
+        case 4: rc = run_grad_group<32, true>(a, idx, m, model, false, st); break;
+        case 5: rc = run_grad_group<64, true>(a, idx, m, model, false, st); break;
+        default: rc = run_grad_group<64, false>(a, idx, m, model, false, st); break;
       }
       if (rc) return rc;
     }
