@@ -734,19 +734,36 @@ __device__ __forceinline__ void stage_probe(float2* prl, const float2* __restric
     prl[j * WAVE + lane] = q;
   }
 }
-// a lane's 16 object values of the patch whose first pixel is f[at] (0 outside
-// the probe, read unconditionally)
+// a lane's 16 object values of the patch whose first pixel is f[0] (0 outside
+// the probe, read unconditionally).  f is uniform over the wave: the loads take
+// scalar bases and unsigned 32-bit byte offsets, one for all values of a lane
+// where the probe fills the transform's window.
+template <class V>
+__device__ __forceinline__ V load_at(const V* f, unsigned byte) {
+  return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(f) + byte);
+}
 template <int D>
 __device__ __forceinline__ void load_frame(float2 (&a)[16], const float2* __restrict__ f,
-                                           const WaveFrame<D>& fr, long at, int n, int P, int o) {
+                                           const WaveFrame<D>& fr, int n, int P, int o) {
   const int px = fr.ix() - o;
+  if (P == (D == 32 ? 32 : 16)) {
+    const unsigned off = (unsigned)(fr.iy(0) * n + px) * sizeof(float2);
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int py = fr.iy(j) - o;
-    const bool in = px >= 0 && px < P && py >= 0 && py < P;
-    a[j] = f[in ? at + (long)py * n + px : at];
-    if (!in) a[j] = make_float2(0.f, 0.f);
+    for (int j = 0; j < 16; ++j) a[j] = load_at(f + (D == 32 ? 2 : 1) * j * n, off);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int py = fr.iy(j) - o;
+      const bool in = px >= 0 && px < P && py >= 0 && py < P;
+      a[j] = load_at(f, in ? (unsigned)(py * n + px) * sizeof(float2) : 0u);
+      if (!in) a[j] = make_float2(0.f, 0.f);
+    }
   }
+}
+// the wave's number within the workgroup, as a scalar: what depends on it alone
+// (the patch, its position and addresses) is computed once per wave
+__device__ __forceinline__ int wave_uniform() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
 }
 
 // Line-search sums of k_minf (lagr = 0) for 32 x 32 frames and for 64 x 64
@@ -757,8 +774,8 @@ __device__ __forceinline__ void load_frame(float2 (&a)[16], const float2* __rest
 // to the far field and twisted, is staged in LDS in lane order.
 // Bound: vector issue and the LDS exchanges, two waves per SIMD (221 registers;
 // held to three waves it spills 47 and measured 8 % slower).  Four CG steps'
-// sweeps: 119 k frames of 32 x 32 8.9 -> 3.6 ms, 14.4 k frames of 64 x 64 with a
-// 16 x 16 probe 40 -> 1.25 ms (a lane per frame row before).
+// sweeps: 119 k frames of 32 x 32 8.9 -> 3.4 ms, 14.4 k frames of 64 x 64 with a
+// 16 x 16 probe 40 -> 1.26 ms (a lane per frame row before).
 constexpr int kMinfWWaves = 4;
 template <int D, int MODEL>
 __global__ __launch_bounds__(WAVE * kMinfWWaves, 2)
@@ -775,7 +792,7 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
   __shared__ double red[kMinfWWaves][PT_MAX_GAM];
   const int c = blockIdx.y;
   if (skip && skip[2 * c + 1] != 0.0) return;
-  const int wave = threadIdx.x / WAVE, lane = lane_id();
+  const int wave = wave_uniform(), lane = lane_id();
   const F fr(lane);
   const int o = D == 32 ? ox : 0;           // frame offset of the probe window
   stage_tw64<D>(tw);
@@ -799,8 +816,8 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
     const int t = (int)(p / S);
     const long at = ((long)t * nz + ps.y) * n + ps.x;
     float2 a[16], b[16];
-    load_frame<D>(a, f, fr, at, n, P, o);
-    load_frame<D>(b, dir, fr, at, n, P, o);
+    load_frame<D>(a, f + at, fr, n, P, o);
+    load_frame<D>(b, dir + at, fr, n, P, o);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const float2 q = prl[j * WAVE + lane];
@@ -809,12 +826,12 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
     }
     fr.rows(a, T, tw);
     fr.rows(b, T, tw);
-    const float* dp = data + p * D * D + fr.ky();
+    const float* dp = data + p * D * D;
 #pragma unroll 1
     for (int sub = 0; sub < F::kSub; ++sub) {
       float d[16], w[16];
 #pragma unroll
-      for (int m = 0; m < 16; ++m) d[m] = dp[fr.kx(m, sub) * D];
+      for (int m = 0; m < 16; ++m) d[m] = load_at(dp, (unsigned)(fr.kx(m, sub) * D + fr.ky()) * 4u);
       float2 ya[16], yb[16];
       fr.cols(a, ya, sub, tw);
       fr.cols(b, yb, sub, tw);
@@ -858,7 +875,7 @@ void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* _
   __shared__ float2 prl[16 * WAVE];
   __shared__ float Tb[kMinfWWaves][F::kBuf];
   __shared__ double2 tw[D == 64 ? 64 : 1];
-  const int wave = threadIdx.x / WAVE, lane = lane_id();
+  const int wave = wave_uniform(), lane = lane_id();
   const F fr(lane);
   const int o = D == 32 ? ox : 0;
   stage_tw64<D>(tw);
@@ -872,27 +889,27 @@ void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* _
     const int2 ps = pos[p];
     const long at = ((p / S) * nz + max(ps.y, 0)) * n + max(ps.x, 0);
     float2 a[16];
-    load_frame<D>(a, f, fr, at, n, P, o);
+    load_frame<D>(a, f + at, fr, n, P, o);
     // a skipped patch (x < 0) has a zero far field
 #pragma unroll
     for (int j = 0; j < 16; ++j)
       a[j] = ps.x < 0 ? make_float2(0.f, 0.f) : cmul(prl[j * WAVE + lane], a[j]);
     fr.rows(a, Tb[wave], tw);
     const float2 sh = shift[p];
-    const long e0 = p * D * D + fr.ky();
+    const long e0 = p * D * D;
 #pragma unroll 1
     for (int sub = 0; sub < F::kSub; ++sub) {
       float2 y[16];
       fr.cols(a, y, sub, tw);
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
-        const int kx = fr.kx(m, sub);
+        const int kx = fr.kx(m, sub), e = kx * D + fr.ky();
         if constexpr (INT) {
-          out[e0 + kx * D] = (y[m].x * y[m].x + y[m].y * y[m].y) * isc;
+          (out + e0)[e] = (y[m].x * y[m].x + y[m].y * y[m].y) * isc;
         } else {
           float2 v = cmul(y[m], sh);
           if constexpr (D == 64) v = F::mul(v, tw[(ox * (kx + fr.ky())) & 63]);
-          g[e0 + kx * D] = v;
+          (g + e0)[e] = v;
         }
       }
     }
@@ -1426,21 +1443,26 @@ void k_tile_group(Group<TileArgs> g) {
 // pixels (WaveFrame): kTileW waves per tile, each taking every kTileW-th of the
 // tile's patches, adding to the shared LDS tile in turn (a barrier between
 // turns), so the order of the sums is the list's.  With one wave per tile the 30
-// KB tiles left one wave per SIMD.  Bound: the FP64 transform's issue (0.44 ms of
-// 1.10 at 119 k frames of 32 x 32) and the LDS exchanges at two waves per SIMD.
-// Gradient of 14.4 k frames of 64 x 64 1.18 -> 0.44 ms, of 119 k of 32 x 32 1.04 ->
-// 1.10 ms (its FP64 values spill 30 registers; the per-row form is gone all the
-// same: adjoint of 20 k frames of 32 x 32 150 -> 72 us).
+// KB tiles left one wave per SIMD.  Bound: the FP64 transform's issue (0.44 of
+// 0.67 ms at 119 k frames of 32 x 32) and the LDS exchanges at two waves per SIMD.
+// What depends on the patch alone is scalar (wave_uniform, load_at), the data model
+// a template argument: gradient of 119 k frames of 32 x 32 1.09 -> 0.67 ms (with
+// 64-bit addresses per lane and value, and both models' code, it spilled 58
+// registers), of 14.4 k of 64 x 64 0.44 -> 0.35 ms; a lane per frame row took 1.04
+// and 1.18 ms.  Adjoint of 20 k frames of 32 x 32 72 us.
+// (Six waves for the 32 x 32 gradient, 160 registers and three waves per SIMD,
+// measured 1.01 ms against 0.67: more turns at the shared tile.)
 constexpr int kTileW = 4;
-template <int D, int MODE>
+template <int D, int MODE, int MODEL>
 __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
   using F = WaveFrame<D>;
   const int EB = A.EB, n = A.n, P = A.P;
   extern __shared__ float lds_f[];
   float2* acc = reinterpret_cast<float2*>(lds_f);
   double2* tw = reinterpret_cast<double2*>(lds_f + ((2 * EB * EB + 3) & ~3) + 2 * WAVE);
-  const int wave = threadIdx.x / WAVE, lane = lane_id();
-  float* T = reinterpret_cast<float*>(tw + (D == 64 ? 64 : 0)) + wave * F::kBuf;
+  const int wave = wave_uniform(), lane = lane_id();
+  float2* prl = reinterpret_cast<float2*>(tw + (D == 64 ? 64 : 0));
+  float* T = reinterpret_cast<float*>(prl + (MODE == TILE_GRAD ? 16 * WAVE : 0)) + wave * F::kBuf;
   const long tile = xcd_contig(b, nb);
   const int slotid = A.tile_slot[tile];
   if (slotid < 0) return;
@@ -1449,12 +1471,23 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
   const int y0 = (rem / A.ntx) * A.B, x0 = (rem % A.ntx) * A.B;
   for (int i = threadIdx.x; i < EB * EB; i += kTileW * WAVE) acc[i] = make_float2(0.f, 0.f);
   stage_tw64<D>(tw);
-  __syncthreads();
-  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
   const F fr(lane);
   const int o = D == 32 ? A.ox : 0;
   const int px = fr.ix() - o;
   const bool colin = px >= 0 && px < P;
+  // gradient: the probe times c = 1/D (exact) staged in lane order, untwisted.  The
+  // adjoint uses it once per patch and reads it from memory: 8 KB more would cost
+  // it a workgroup per CU (91 -> 99 us at 20 k frames of 32 x 32).
+  if constexpr (MODE == TILE_GRAD) {
+    for (int j = wave; j < 16; j += kTileW) {
+      const int py = fr.iy(j) - o;
+      const bool in = colin && py >= 0 && py < P;
+      prl[j * WAVE + lane] = in ? cscale(A.prb[(long)px * P + py], A.cs) : make_float2(0.f, 0.f);
+    }
+  }
+  const float oscale = MODE == TILE_GRAD ? A.out_scale / A.cs : A.out_scale;
+  __syncthreads();
+  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
   for (int i0 = beg; i0 < end; i0 += kTileW) {
     const int ii = i0 + wave;
     const bool active = ii < end;
@@ -1469,27 +1502,23 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
         // a = coefptycho * F(c * prb * psi), rounded once after an FP64 transform
         const long at = ((long)t * A.nz + ps.y) * n + ps.x;
         float2 v[16];
+        load_frame<D>(v, A.f + at, fr, n, P, o);
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const int py = fr.iy(j) - o;
-          const bool in = colin && py >= 0 && py < P;
-          v[j] = A.f[in ? at + (long)py * n + px : at];
-          const float2 q = A.prb[in ? (long)px * P + py : 0];
-          v[j] = in ? cscale(cmul(q, v[j]), A.cs) : make_float2(0.f, 0.f);
+          const float2 q = cmul(prl[j * WAVE + lane], v[j]);
+          x[j] = make_double2((double)q.x, (double)q.y);
         }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) x[j] = make_double2((double)v[j].x, (double)v[j].y);
         fr.rows(x, T, tw);
       }
 #pragma unroll 1
       for (int sub = 0; sub < F::kSub; ++sub) {
         float2 y[16];
-        const long e0 = p * D * D + fr.ky();
+        const long e0 = p * D * D;
         if constexpr (MODE == TILE_ADJ) {
           // the per-patch phase removed; at D = 64 also the factor W^(o k) of the
           // probe's offset, which the sub-transforms leave out
 #pragma unroll
-          for (int m = 0; m < 16; ++m) y[m] = cmulc(A.gin[e0 + fr.kx(m, sub) * D], sh);
+          for (int m = 0; m < 16; ++m) y[m] = cmulc(load_at(A.gin + e0, (unsigned)(fr.kx(m, sub) * D + fr.ky()) * 8u), sh);
           if constexpr (D == 64) {
 #pragma unroll
             for (int m = 0; m < 16; ++m)
@@ -1507,7 +1536,7 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
           __builtin_amdgcn_sched_barrier(0);  // the data after the FP64 transform: registers
           float dv[16];
 #pragma unroll
-          for (int m = 0; m < 16; ++m) dv[m] = A.data[e0 + fr.kx(m, sub) * D];
+          for (int m = 0; m < 16; ++m) dv[m] = load_at(A.data + e0, (unsigned)(fr.kx(m, sub) * D + fr.ky()) * 4u);
           // residual as in tile_body
 #pragma unroll
           for (int m = 0; m < 16; ++m) {
@@ -1515,16 +1544,15 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
             const float2 a = y[m];
             const float aa = a.x * a.x + a.y * a.y;
             float2 res;
-            if (A.model == PT_MODEL_POISSON) {
+            if constexpr (MODEL == PT_MODEL_POISSON) {
               const float q = d / (aa + 1e-32f);
               res = make_float2(a.x - q * a.x, a.y - q * a.y);
             } else {
               const float mo = sqrtf(aa);
               const float sd = sqrtf(d);
-              if (mo > 0.f) {
-                const float q = sd / mo;
-                res = make_float2(a.x - q * a.x, a.y - q * a.y);
-              } else {
+              const float q = sd / mo;
+              res = make_float2(a.x - q * a.x, a.y - q * a.y);
+              if (!(mo > 0.f)) {
                 // angle(0) = 0 in the shifted frame
                 res = make_float2(-sd * sh.x, sd * sh.y);
                 if constexpr (D == 64)
@@ -1540,10 +1568,14 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
       fr.combine(z);
 #pragma unroll
       for (int j = 0; j < F::kOut; ++j) {
-        const int py = fr.out_iy(j) - o;
-        const bool in = colin && py >= 0 && py < P;
-        const float2 q = A.prb[in ? (long)px * P + py : 0];
-        z[j] = cscale(cmulc(z[j], q), A.out_scale);
+        float2 q;
+        if constexpr (MODE == TILE_GRAD) {
+          q = prl[(D == 64 ? fr.out_iy(j) : j) * WAVE + lane];
+        } else {
+          const int py = fr.out_iy(j) - o;
+          q = A.prb[colin && py >= 0 && py < P ? (long)px * P + py : 0];
+        }
+        z[j] = cscale(cmulc(z[j], q), oscale);
       }
     }
     // tile index of each kept value; values outside the probe go to a slot of
@@ -1571,20 +1603,21 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
   float2* out = A.scratch + (long)slotid * EB * EB;
   for (int i = threadIdx.x; i < EB * EB; i += kTileW * WAVE) out[i] = acc[i];
 }
-template <int D, int MODE>
+template <int D, int MODE, int MODEL>
 __global__ __launch_bounds__(WAVE * kTileW, 2) void k_tile_w(TileArgs A) {
-  tile_body_w<D, MODE>(A, blockIdx.x, gridDim.x);
+  tile_body_w<D, MODE, MODEL>(A, blockIdx.x, gridDim.x);
 }
-template <int D, int MODE>
+template <int D, int MODE, int MODEL>
 __global__ __launch_bounds__(WAVE * kTileW, 2) void k_tile_w_group(Group<TileArgs> g) {
   const int i = group_find(g, blockIdx.x);
-  tile_body_w<D, MODE>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
+  tile_body_w<D, MODE, MODEL>(g.a[i], blockIdx.x - g.start[i], g.gx[i]);
 }
 // LDS bytes of a k_tile_w workgroup
-template <int D>
+template <int D, int MODE>
 inline size_t tile_w_lds_bytes(int EB) {
   return sizeof(float) * (size_t)(((2 * EB * EB + 3) & ~3) + 2 * WAVE) +
          (D == 64 ? 64 * sizeof(double2) : 0) +
+         (MODE == TILE_GRAD ? sizeof(float2) * (size_t)16 * WAVE : 0) +
          sizeof(float) * (size_t)kTileW * WaveFrame<D>::kBuf;
 }
 // whether a handle's frames run one wave per frame (WaveFrame)
@@ -1754,8 +1787,11 @@ int run_tiles(pt_ptycho* h, const float2* gin, const float2* f, const float* dat
   ProfScope prof(MODE == TILE_GRAD ? "ptycho_grad_tile" : "ptycho_adj_tile", st);
   if constexpr (D >= 32) {
     if (wave_frames(h)) {
-      hipLaunchKernelGGL((k_tile_w<D, MODE>), dim3((unsigned)h->ntiles), dim3(WAVE * kTileW),
-                         tile_w_lds_bytes<D>(h->EB), st, A);
+      auto kern = MODE == TILE_ADJ || model == PT_MODEL_POISSON
+                      ? k_tile_w<D, MODE, PT_MODEL_POISSON>
+                      : k_tile_w<D, MODE, MODE == TILE_ADJ ? PT_MODEL_POISSON : PT_MODEL_GAUSSIAN>;
+      const size_t lds = tile_w_lds_bytes<D, MODE>(h->EB);
+      hipLaunchKernelGGL(kern, dim3((unsigned)h->ntiles), dim3(WAVE * kTileW), lds, st, A);
       PT_LAUNCH_CHECK();
       return PT_OK;
     }
@@ -2199,7 +2235,7 @@ static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, i
     fg.gx[k] = fold_blocks(h);
     fg.start[k] = totf;
     totf += fg.gx[k];
-    if constexpr (WF) lds = std::max(lds, tile_w_lds_bytes<D>(h->EB));
+    if constexpr (WF) lds = std::max(lds, tile_w_lds_bytes<D, TILE_GRAD>(h->EB));
     else lds = std::max(lds, tile_lds_bytes(D, h->EB));
   }
   g.start[n] = tot;
@@ -2207,12 +2243,15 @@ static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, i
   g.n = fg.n = n;
   {
     ProfScope prof("ptycho_grad_tile", st);
-    if constexpr (WF)
-      hipLaunchKernelGGL((k_tile_w_group<D, TILE_GRAD>), dim3(tot), dim3(WAVE * kTileW), lds, st, g);
-    else
+    if constexpr (WF) {
+      auto kern = model == PT_MODEL_POISSON ? k_tile_w_group<D, TILE_GRAD, PT_MODEL_POISSON>
+                                            : k_tile_w_group<D, TILE_GRAD, PT_MODEL_GAUSSIAN>;
+      hipLaunchKernelGGL(kern, dim3(tot), dim3(WAVE * kTileW), lds, st, g);
+    } else {
       tile_dispatch<D, TILE_GRAD>(model, full, [&](auto, auto kern) {
         hipLaunchKernelGGL(kern, dim3(tot), dim3(WAVE * tile_waves<D>()), lds, st, g);
       });
+    }
   }
   PT_LAUNCH_CHECK();
   {
