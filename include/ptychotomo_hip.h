@@ -230,6 +230,14 @@ typedef struct pt_ptycho_linesearch_args {
   const double* skip;
 } pt_ptycho_linesearch_args;
 
+/* One sweep of cg_ptycho's line search: pt_ptycho_linesearch at the ngam
+ * candidates a->gammas of the chunks that the search state a->skip leaves
+ * open (updated in place), then pt_k_ls_select with the weights w; a->f1 and
+ * a->f2 are not used. */
+int pt_ptycho_linesearch_sweep(const pt_ptycho_linesearch_args* a, double* cand_next, double* step,
+                               const double* w, int ngam, int ngam_next, int last, int model,
+                               pt_stream stream);
+
 /* pt_ptycho_linesearch for n independent reconstructions at once (no
  * counterpart in the reference, which reconstructs one object per run: the
  * batched solver's multi-instance launch).  Instances that take the

@@ -96,6 +96,8 @@ _SIGS = {
                                c_int, vp, vp]),
     "pt_ptycho_minf_noalloc": (c_int, [vp, vp, vp, vp, vp, vp, c_int, c_int, c_float, c_float,
                                        c_int, c_int, vp, vp]),
+    "pt_ptycho_linesearch_sweep": (c_int, [ctypes.POINTER(LinesearchArgs), vp, vp, vp, c_int, c_int,
+                                           c_int, c_int, vp]),
     "pt_ptycho_linesearch": (c_int, [vp, vp, vp, vp, vp, vp, vp, vp, c_double, vp, vp, c_int,
                                      c_int, c_float, c_float, c_int, vp, vp]),
     "pt_ptycho_linesearch_group": (c_int, [ctypes.POINTER(LinesearchArgs), c_int, c_int, c_int,

@@ -18,7 +18,7 @@ import torch
 
 from . import _lib
 from ._dev import stream
-from .solver import Solver, run_ptycho_request
+from .solver import Solver, run_ptycho_request, select_request
 
 
 class BatchSolver:
@@ -156,6 +156,8 @@ class BatchSolver:
                 else:
                     arr = (_lib.LinesearchArgs * n)(*[r[1] for r in reqs])
                     _lib.call("pt_ptycho_linesearch_group", arr, n, ng, mdl, st)
+                    for r in reqs:
+                        select_request(r, st)
                 reqs = [next(g) for g in gens]
             if any(r[0] != "end" for r in reqs):
                 raise RuntimeError("BatchSolver: instances out of step")

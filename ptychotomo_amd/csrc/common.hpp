@@ -571,4 +571,45 @@ __device__ __forceinline__ int xcd_contig(int w, int total) {
   return x * q + min(x, r) + (w >> 3);
 }
 
+// ---------------------------------------------------------------- line search
+// One sweep's decision of a segment (solver.py:171-177): f_j = f1[j] + f2[j] already
+// weighted, candidates cand[j] (j = 0: gamma = 0).  Accepts the first candidate
+// that is not a strict ascent or is <= 1e-12 (then 0): step = {gamma, 0}, state =
+// {gamma, 1}; otherwise the next sweep (cand_next) continues from half the last
+// candidate, or, with `last`, the search ends at 0.  FP64, no contraction: the
+// host restatement of the rule gives the same bits.
+template <class F>
+__device__ inline void ls_decide(double* state, double* step, const double* cand,
+                                 double* cand_next, int ngam, int ngam_next, int last, F f) {
+#pragma clang fp contract(off)
+  const double fz = f(0);
+  for (int j = 1; j < ngam; ++j) {
+    const double g = cand[j];
+    if (fz - f(j) < 0.0 && g > 1e-12) continue;
+    const double out = g <= 1e-12 ? 0.0 : g;
+    step[0] = out;
+    step[1] = 0.0;
+    state[0] = out;
+    state[1] = 1.0;
+    return;
+  }
+  if (last) {
+    step[0] = step[1] = 0.0;
+    state[0] = 0.0;
+    state[1] = 1.0;
+    return;
+  }
+  const double cur = cand[ngam - 1] * 0.5;
+  state[0] = cur;
+  cand_next[0] = 0.0;
+  for (int j = 1; j < ngam_next; ++j) cand_next[j] = cur * ldexp(1.0, -(j - 1));
+}
+
+// Sums over pixels of the rho term's change at ngam candidates per segment, left
+// as partials [seg][block][8] in the stream's reduction scratch (pt_k_rho_minf
+// without its second pass): *part, *nblk.
+int rho_minf_partials(double** part, int* nblk, const void* h, const void* psi, const void* lamd,
+                      const void* d, double rho, const double* rho_dev, const double* gammas,
+                      int ngam, long len, int nseg, const double* skip, hipStream_t st);
+
 }  // namespace pt

@@ -926,8 +926,8 @@ void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* _
 // chunk (blockIdx.y), kMinfTiles of them: a sweep in which every chunk has
 // finished its search (skip) then costs a quarter of the workgroup launches,
 // and one in which a single chunk is open still fills the device.  Per-patch arithmetic is that of
-// k_minf; one partial per (chunk, tile, wave) in
-// partial[((c*tpc + tile)*kMinfWaves + w)*ngam + j].
+// k_minf.  The tiles' sums add up in LDS; one partial per workgroup in
+// partial[(c*ngam + j)*gx + workgroup].
 // FULL: the probe covers the frame (P = D, no offset): no bounds selects,
 // and the probe in LDS is pre-scaled by cs*cp (the far field is linear in
 // the probe), so the frames need no scaling after the transform.
@@ -1010,10 +1010,11 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
     else prl[i] = cscale(prb[i], pscale);
   }
   __shared__ float gsh[NG];
+  __shared__ double tot[2][kMinfWaves][NG];  // data term, rho term; each wave adds to its own
+  if (lane < NG) tot[0][wave][lane] = tot[1][wave][lane] = 0.0;
   const int tpa = nty * ntx, tpc = chunk * tpa;
   if (threadIdx.x < NG)
     gsh[threadIdx.x] = threadIdx.x < ngam ? (float)gammas[(long)c * ngam + threadIdx.x] : 0.f;
-  const long nbt = (long)tpc * kMinfWaves;
   const float rho = (float)(rho_dev ? rho_dev[0] : rho_host);
   const int ix = r - ox;
   for (int tb = bx; tb < tpc; tb += gxn) {
@@ -1119,12 +1120,11 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
         acc[NG - 1] = t0;
       }
     }
-    double* out = partial + (long)c * ngam * nbt + (long)tb * kMinfWaves + wave;
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
       if (j >= ngam) break;
       const double v = wave_sum(acc[j]);
-      if (lane == 0) out[j * nbt] = v;
+      if (lane == 0) tot[0][wave][j] += v;
     }
     if (!hh) continue;
     // The functional's rho term (solver.py:213), change of
@@ -1132,8 +1132,7 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
     // this tile owns: its B x B core, and for the last tile of a row or
     // column of tiles everything up to the object's edge (inside the
     // extended region), so the tiles of an angle partition it.  psi and d
-    // were just staged from the same lines (cached); partials in
-    // partial_rho, same layout as the data term's.
+    // were just staged from the same lines (cached).
     const int ty = rem / ntx, tx = rem % ntx;
     const int wy = (ty == nty - 1 ? nz : y0 + B) - y0, wx = (tx == ntx - 1 ? n : x0 + B) - x0;
 #pragma unroll
@@ -1154,14 +1153,18 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
         }
       }
     }
-    double* outr = partial_rho + (long)c * ngam * nbt + (long)tb * kMinfWaves + wave;
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
       if (j >= ngam) break;
       const double v = wave_sum(acc[j]);
-      if (lane == 0) outr[j * nbt] = v;
+      if (lane == 0) tot[1][wave][j] += v;
     }
   }
+  __syncthreads();
+  const int term = wave, j = lane;  // two waves: wave 0 the data term, wave 1 the rho term
+  static_assert(kMinfWaves == 2, "one wave per term");
+  if (j < ngam && (term == 0 || hh))
+    (term ? partial_rho : partial)[((long)c * ngam + j) * gxn + bx] = tot[term][0][j] + tot[term][1][j];
 }
 
 template <int D, int MODEL, int NG, bool FULL>
@@ -1215,6 +1218,50 @@ __global__ __launch_bounds__(256) void k_reduce_partials_group(Group<ReduceArgs>
   for (long b = threadIdx.x; b < A.nblk; b += blockDim.x) v[0] += src[b];
   block_sum<1>(v, sm);
   if (threadIdx.x == 0) A.out[c * ngam + j] = v[0];
+}
+
+// Sums of a sweep's partials of both terms and its decision, one workgroup per
+// chunk: a wave per (term, candidate) adds the partials in a fixed order, then one
+// lane applies the halving rule.  The two reductions and the selection this
+// replaces (and, off the tile path, the rho term's second pass) were 62 of some 330
+// launches of an ADMM iteration, each 3.5 us in small problems: iteration at 64^3
+// 1.99 -> 1.87 ms, 4 CG steps at 128^2, 64 angles, 64 x 64 frames 3.13 -> 3.02 ms.
+// The line search on tiles writes a partial per workgroup (an eighth of one per
+// wave and tile), since one workgroup per chunk reads them: 7 us at 256^3.
+struct LsFinishArgs {
+  double* state;
+  const double* cand;
+  double* cand_next;
+  double* step;
+  const double* w;       // weights of the two terms
+  const double* p[2];    // partials of chunk c, candidate j, block b:
+  long cs[2], js[2], bs[2];  // p[c*cs + j*js + b*bs]
+  int nb[2];
+  int ngam, ngam_next, last;
+};
+__global__ __launch_bounds__(1024) void k_ls_finish(LsFinishArgs A) {
+  __shared__ double f[2][PT_MAX_GAM];
+  const int c = blockIdx.x, wid = threadIdx.x / WAVE, lane = lane_id();
+  if (A.state[2 * c + 1] != 0.0) return;
+  const int term = wid / PT_MAX_GAM, j = wid % PT_MAX_GAM;
+  if (j < A.ngam) {
+    const double* src = A.p[term] + c * A.cs[term] + j * A.js[term];
+    const long bs = A.bs[term];
+    const int nb = A.nb[term];
+    double s = 0.0;
+#pragma unroll 8
+    for (int b = lane; b < nb; b += WAVE) s += src[b * bs];
+    s = wave_sum(s);
+    if (lane == 0) f[term][j] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  const double w0 = A.w[0], w1 = A.w[1];
+  ls_decide(A.state + 2 * c, A.step + 2 * c, A.cand + c * A.ngam, A.cand_next + c * A.ngam_next,
+            A.ngam, A.ngam_next, A.last, [&](int k) {
+#pragma clang fp contract(off)
+              return w0 * f[0][k] + w1 * f[1][k];
+            });
 }
 
 // LDS bytes of a k_minf_tile workgroup
@@ -1836,6 +1883,7 @@ struct RhoTerm {
   double rho = 0.0;
   const double* rho_dev = nullptr;
   double* f2 = nullptr;
+  LsFinishArgs* fin = nullptr;  // set: finish the sweep with k_ls_finish instead of sums and f2
 };
 
 // whether a line search of this handle runs on the overlap-add tiles: frames
@@ -1902,23 +1950,33 @@ int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, con
   // line-search sums over the overlap-add tiles (frames read from LDS)
   const size_t tl = minf_tile_lds_bytes(D, h->EB, h->P);
   if constexpr (D <= 16) if (!lagr && dir && minf_tile_path<D>(h)) {
-    const int tpc = chunk * h->nty * h->ntx;
-    const int nbt = tpc * kMinfWaves;
+    const int nbt = minf_tile_gx(h, chunk);
     const size_t nper = (size_t)nchunk * nbt * ngam;
+    // a fixed buffer has to hold one partial per wave and tile (the interface's bound)
+    const size_t need = fixed ? (size_t)nchunk * chunk * h->nty * h->ntx * kMinfWaves * ngam : nper;
     double* part;
-    int rc = minf_partials(h, rt.hh ? 2 * nper : nper, fixed, fixed_cap, &part);
+    int rc = minf_partials(h, rt.hh ? 2 * need : need, fixed, fixed_cap, &part);
     if (rc) return rc;
     double* part_rho = rt.hh ? part + nper : nullptr;
     {
       ProfScope prof("ptycho_minf", st);
       const MinfTileArgs A = minf_tile_args(h, part, part_rho, f, dir, data, gammas, ngam, chunk,
                                             cp, cd, skip, rt);
-      const int gx = minf_tile_gx(h, chunk);
       minf_dispatch<D>(model, minf_full<D>(h), ngam, [&](auto kern, auto) {
-        hipLaunchKernelGGL(kern, dim3(gx, nchunk), dim3(WAVE * kMinfWaves), tl, st, A);
+        hipLaunchKernelGGL(kern, dim3(nbt, nchunk), dim3(WAVE * kMinfWaves), tl, st, A);
       });
     }
     PT_LAUNCH_CHECK();
+    if (rt.fin) {
+      LsFinishArgs& F = *rt.fin;
+      for (int t = 0; t < 2; ++t) {
+        F.p[t] = t ? part_rho : part;
+        F.cs[t] = (long)ngam * nbt; F.js[t] = nbt; F.bs[t] = 1; F.nb[t] = nbt;
+      }
+      hipLaunchKernelGGL(k_ls_finish, dim3(nchunk), dim3(1024), 0, st, F);
+      PT_LAUNCH_CHECK();
+      return PT_OK;
+    }
     hipLaunchKernelGGL(k_reduce_partials_t, dim3(nchunk, ngam), dim3(256), 0, st, sums, part,
                        (long)nbt, ngam, skip);
     PT_LAUNCH_CHECK();
@@ -1961,6 +2019,19 @@ int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, con
                        h->S, h->P, h->ox, h->oy, h->c, cp, cd, model, lagr, skip);
   }
   PT_LAUNCH_CHECK();
+  if (rt.fin) {
+    LsFinishArgs& F = *rt.fin;
+    double* pr;
+    int nbr;
+    rc = rho_minf_partials(&pr, &nbr, rt.hh, f, rt.lamd, dir, rt.rho, rt.rho_dev, gammas, ngam,
+                           (long)h->pt * h->nz * h->n, nchunk, skip, st);
+    if (rc) return rc;
+    F.p[0] = part; F.cs[0] = (long)nb * ngam; F.js[0] = 1; F.bs[0] = ngam; F.nb[0] = nb;
+    F.p[1] = pr; F.cs[1] = (long)nbr * 8; F.js[1] = 1; F.bs[1] = 8; F.nb[1] = nbr;
+    hipLaunchKernelGGL(k_ls_finish, dim3(nchunk), dim3(1024), 0, st, F);
+    PT_LAUNCH_CHECK();
+    return PT_OK;
+  }
   hipLaunchKernelGGL(k_reduce_partials, dim3(nchunk, ngam), dim3(64), 0, st, sums, part, nb,
                      ngam, skip);
   PT_LAUNCH_CHECK();
@@ -2352,6 +2423,40 @@ extern "C" int pt_ptycho_linesearch(pt_ptycho* h, double* f1, double* f2, const 
                                      nullptr, 0, rt)));
 }
 
+extern "C" int pt_ptycho_linesearch_sweep(const pt_ptycho_linesearch_args* a, double* cand_next,
+                                          double* step, const double* w, int ngam, int ngam_next,
+                                          int last, int model, pt_stream stream) {
+  PT_REQUIRE(a && a->h && a->psi && a->dir && a->data && a->hh && a->lamd && a->gammas &&
+                 a->skip && cand_next && step && w,
+             PT_ERR_ARG, "pt_ptycho_linesearch_sweep: null argument");
+  pt_ptycho* h = a->h;
+  PT_REQUIRE(h->ready, PT_ERR_STATE, "pt_ptycho_linesearch_sweep: set_scan_probe not called");
+  PT_REQUIRE(ngam >= 2 && ngam <= PT_MAX_GAM && ngam_next >= 2 && ngam_next <= PT_MAX_GAM,
+             PT_ERR_ARG, "pt_ptycho_linesearch_sweep: 2 <= ngam, ngam_next <= 8");
+  PT_REQUIRE(a->chunk > 0 && h->pt % a->chunk == 0, PT_ERR_SIZE,
+             "pt_ptycho_linesearch_sweep: chunk must divide the number of angles");
+  PT_REQUIRE(model == PT_MODEL_POISSON || model == PT_MODEL_GAUSSIAN, PT_ERR_ARG,
+             "pt_ptycho_linesearch_sweep: bad model");
+  PT_REQUIRE(a->rho_dev || a->rho > 0, PT_ERR_ARG,
+             "pt_ptycho_linesearch_sweep: rho must be positive");
+  PT_REQUIRE(cand_next != a->gammas || ngam_next == ngam || h->pt == a->chunk, PT_ERR_ARG,
+             "pt_ptycho_linesearch_sweep: a sweep of another width needs its own candidate buffer");
+  LsFinishArgs F = {};
+  F.state = const_cast<double*>(a->skip);
+  F.cand = a->gammas; F.cand_next = cand_next; F.step = step; F.w = w;
+  F.ngam = ngam; F.ngam_next = ngam_next; F.last = last;
+  RhoTerm rt;
+  rt.hh = (const float2*)a->hh;
+  rt.lamd = (const float2*)a->lamd;
+  rt.rho = a->rho;
+  rt.rho_dev = a->rho_dev;
+  rt.fin = &F;
+  hipStream_t st = (hipStream_t)stream;
+  PT_DISPATCH_D(h->D, (run_minf<DD>(h, nullptr, (const float2*)a->psi, (const float2*)a->dir,
+                                    a->data, a->gammas, ngam, a->chunk, a->coefptycho,
+                                    a->coefdata, model, 0, a->skip, st, nullptr, 0, rt)));
+}
+
 // One launch of k_minf_tile_group (and the two grouped reductions) for the
 // instances idx (at most kGroupMax, all on the tile path with detector D and
 // the same probe form)
@@ -2366,7 +2471,7 @@ static int run_minf_group(const pt_ptycho_linesearch_args* a, const int* idx, in
     const pt_ptycho_linesearch_args& x = a[idx[k]];
     pt_ptycho* h = x.h;
     const int nchunk = h->pt / x.chunk;
-    const int nbt = x.chunk * h->nty * h->ntx * kMinfWaves;
+    const int nbt = minf_tile_gx(h, x.chunk);
     const size_t nper = (size_t)nchunk * nbt * ngam;
     double* part;
     int rc = minf_partials(h, 2 * nper, nullptr, 0, &part);
@@ -2379,7 +2484,7 @@ static int run_minf_group(const pt_ptycho_linesearch_args* a, const int* idx, in
     rt.f2 = x.f2;
     g.a[k] = minf_tile_args(h, part, part + nper, (const float2*)x.psi, (const float2*)x.dir,
                             x.data, x.gammas, ngam, x.chunk, x.coefptycho, x.coefdata, x.skip, rt);
-    g.gx[k] = minf_tile_gx(h, x.chunk);
+    g.gx[k] = nbt;
     g.start[k] = tot;
     tot += g.gx[k] * nchunk;
     r1.a[k] = ReduceArgs{x.f1, part, x.skip, (long)nbt};

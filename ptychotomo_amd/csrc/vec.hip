@@ -134,20 +134,27 @@ int seg_reduce(double* out, long len, int nseg, F f, hipStream_t st) {
 // as seg_reduce with NV = PT_MAX_CAND accumulators, of which the first
 // `nout` are written per segment
 template <typename F>
-int seg_reduce_n(double* out, long len, int nseg, int nout, F f, hipStream_t st,
-                 const double* skip = nullptr) {
+int seg_partials_n(double** part, int* nblk, long len, int nseg, F f, hipStream_t st,
+                   const double* skip) {
   constexpr int NV = 8;
   PT_REQUIRE(nseg > 0 && len % nseg == 0, PT_ERR_SIZE, "reduction: nseg must divide len");
   const long seglen = len / nseg;
-  int nblk = (int)std::min<long>(RMAXBLK, std::max<long>(1, (seglen + RB * 4 - 1) / (RB * 4)));
-  nblk = std::max(1, std::min(nblk, std::max(1, (nseg == 1 ? RMAXBLK : RMAXTOT) / nseg)));
-  double* part;
-  int rc = partial_buf((size_t)nseg * nblk * NV, &part, st);
+  *nblk = (int)std::min<long>(RMAXBLK, std::max<long>(1, (seglen + RB * 4 - 1) / (RB * 4)));
+  *nblk = std::max(1, std::min(*nblk, std::max(1, (nseg == 1 ? RMAXBLK : RMAXTOT) / nseg)));
+  int rc = partial_buf((size_t)nseg * *nblk * NV, part, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((k_seg_reduce<NV, F>), dim3(nblk, nseg), dim3(RB), 0, st, part, seglen, f,
+  hipLaunchKernelGGL((k_seg_reduce<NV, F>), dim3(*nblk, nseg), dim3(RB), 0, st, *part, seglen, f,
                      skip);
   PT_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_finish_n, dim3(nseg, nout), dim3(RB), 0, st, out, part, nblk, NV, nout,
+  return PT_OK;
+}
+template <typename F>
+int seg_reduce_n(double* out, long len, int nseg, int nout, F f, hipStream_t st,
+                 const double* skip = nullptr) {
+  double* part;
+  int nblk, rc = seg_partials_n(&part, &nblk, len, nseg, f, st, skip);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_finish_n, dim3(nseg, nout), dim3(RB), 0, st, out, part, nblk, 8, nout,
                      skip);
   PT_LAUNCH_CHECK();
   return PT_OK;
@@ -914,6 +921,15 @@ extern "C" int pt_k_rho_minf(double* out, const void* h, const void* psi, const 
                                (const float2*)d, SV{rho, rho_dev}, gammas, ngam, len / nseg},
                       (hipStream_t)stream, skip);
 }
+int pt::rho_minf_partials(double** part, int* nblk, const void* h, const void* psi,
+                          const void* lamd, const void* d, double rho, const double* rho_dev,
+                          const double* gammas, int ngam, long len, int nseg, const double* skip,
+                          hipStream_t st) {
+  return seg_partials_n(part, nblk, len, nseg,
+                        FRhoMinf{(const float2*)h, (const float2*)psi, (const float2*)lamd,
+                                 (const float2*)d, SV{rho, rho_dev}, gammas, ngam, len / nseg},
+                        st, skip);
+}
 extern "C" int pt_k_tomo_minf(double* out, const void* K, const void* Ru, const void* Rd,
                               const void* xi0, const double* gammas, int ngam, long len,
                               const double* skip, pt_stream stream) {
@@ -989,28 +1005,8 @@ __global__ void k_ls_select(double* __restrict__ state, const double* cand, doub
   const double w0 = w[0], w1 = f2 ? w[1] : 0.0;
   const double* a = f1 + s * ngam;
   const double* b = f2 ? f2 + s * ngam : nullptr;
-  const double fz = w0 * a[0] + (b ? w1 * b[0] : 0.0);
-  for (int j = 1; j < ngam; ++j) {
-    const double g = cand[s * ngam + j];
-    const double fj = w0 * a[j] + (b ? w1 * b[j] : 0.0);
-    if (fz - fj < 0.0 && g > 1e-12) continue;
-    const double out = g <= 1e-12 ? 0.0 : g;
-    step[2 * s] = out;
-    step[2 * s + 1] = 0.0;
-    state[2 * s] = out;
-    state[2 * s + 1] = 1.0;
-    return;
-  }
-  const double cur = cand[s * ngam + ngam - 1] * 0.5;
-  if (last) {
-    step[2 * s] = step[2 * s + 1] = 0.0;
-    state[2 * s] = 0.0;
-    state[2 * s + 1] = 1.0;
-    return;
-  }
-  state[2 * s] = cur;
-  cand_next[s * ngam_next] = 0.0;
-  for (int j = 1; j < ngam_next; ++j) cand_next[s * ngam_next + j] = cur * ldexp(1.0, -(j - 1));
+  ls_decide(state + 2 * s, step + 2 * s, cand + s * ngam, cand_next + s * ngam_next, ngam,
+            ngam_next, last, [&](int j) { return w0 * a[j] + (b ? w1 * b[j] : 0.0); });
 }
 
 // cg_tomo's whole halving search (solver.py:171-183) in two sweeps: the first

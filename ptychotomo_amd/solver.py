@@ -317,12 +317,13 @@ class Solver(object):
         """The halving rule of line_search for nseg independent segments, on
         the device: sweeps of sched[i] halvings (plus gamma = 0) until every
         segment has accepted a step (a schedule covers 2 -> 1e-12).  A
-        generator: yields (cand, ngam, state, f1, f2) where the two functional
-        terms (their change from gamma = 0) are to be evaluated at the ngam
-        candidate slots per segment, skipping finished segments (by the
-        caller, alone or in a group of instances), then enqueues the sweep's
-        selection; weights points to the terms' two FP64 weights.  Consecutive
-        sweeps alternate between two candidate buffers."""
+        generator: yields (cand, ngam, state, f1, f2, select) where the two
+        functional terms (their change from gamma = 0) are to be evaluated at
+        the ngam candidate slots per segment, skipping finished segments, and
+        the sweep's selection is to be made with the arguments `select` (by the
+        caller, alone or in a group of instances); weights points to the terms'
+        two FP64 weights.  Consecutive sweeps alternate between two candidate
+        buffers."""
         st = stream()
         bufs = (w["cand"], w["cand2"])
         ng = sched[0] + 1
@@ -331,9 +332,8 @@ class Solver(object):
             last = sw == len(sched) - 1
             ng_next = ng if last else sched[sw + 1] + 1
             cur, nxt = bufs[sw % 2], bufs[(sw + 1) % 2]
-            yield cur, ng, w["state"], w["f1"], w["f2"]
-            _call("pt_k_ls_select", ptr(w["state"]), ptr(cur), ptr(nxt), ptr(w["step"]),
-                  ptr(w["f1"]), ptr(w["f2"]), weights, nseg, ng, ng_next, int(last), st)
+            yield cur, ng, w["state"], w["f1"], w["f2"], (ptr(nxt), ptr(w["step"]), weights, nseg,
+                                                          ng_next, int(last))
             ng = ng_next
 
     def _dai_yuan_dev(self, w, i, grad, grad0, L, nseg):
@@ -432,9 +432,10 @@ class Solver(object):
     def _cg_ptycho_gen(self, op, nseg, data, psi, h, lamd, blk, piter, coefdata, hist=None):
         """_cg_ptycho_dev as a generator: its two heavy launches -- the fused
         gradient and each line-search sweep -- are yielded as requests
-        ("grad", GradArgs) and ("ls", LinesearchArgs, ngam) for the caller to
-        make (run_ptycho_request, or one grouped call for many instances in
-        lock-step); everything else is enqueued here on the current stream."""
+        ("grad", GradArgs) and ("ls", LinesearchArgs, ngam, select) for the caller
+        to make (run_ptycho_request, or one grouped call for many instances in
+        lock-step, then select_request); everything else is enqueued here on the
+        current stream."""
         st = stream()
         L = psi.numel()
         w = self._work(("ptycho", id(op)), nseg, psi.shape)
@@ -452,12 +453,12 @@ class Solver(object):
             grad0 = grad
             # minf = data term + rho*|h - psi + lamd/rho|^2 (solver.py:208-213): the
             # two terms in one pass over the overlap-add tiles
-            for cand, ng, state, f1, f2 in self._line_search_gen(
+            for cand, ng, state, f1, f2, sel in self._line_search_gen(
                     w, nseg, _dp(blk, _ONE), _PSCHED_FIRST if i == 0 else _PSCHED_LATER):
                 yield ("ls", _lib.LinesearchArgs(
                     op._h, f1.data_ptr(), f2.data_ptr(), psi.data_ptr(), d.data_ptr(),
                     data.data_ptr(), h.data_ptr(), lamd.data_ptr(), 0.0, rho_dev,
-                    cand.data_ptr(), chunk, cp, cd, state.data_ptr()), ng)
+                    cand.data_ptr(), chunk, cp, cd, state.data_ptr()), ng, sel)
             _call("pt_k_axpy_seg", ptr(psi), ptr(w["step"]), ptr(d), L, nseg, st)
             if hist is not None:
                 hist[i].copy_(w["step"][0::2])
@@ -688,8 +689,15 @@ def run_ptycho_request(req, mdl, st):
         _call("pt_ptycho_grad", a.h, a.grad, a.psi, a.data, a.hh, a.lamd, a.rho, a.rho_dev,
               a.coefptycho, a.coefdata, mdl, st)
     else:
-        _call("pt_ptycho_linesearch", a.h, a.f1, a.f2, a.psi, a.dir, a.data, a.hh, a.lamd, a.rho,
-              a.rho_dev, a.gammas, req[2], a.chunk, a.coefptycho, a.coefdata, mdl, a.skip, st)
+        nxt, step, weights, _, ng_next, last = req[3]
+        _call("pt_ptycho_linesearch_sweep", a, nxt, step, weights, req[2], ng_next, last, mdl, st)
+
+
+def select_request(req, st):
+    """The selection of a ("ls", ...) request whose two terms are evaluated."""
+    a, (nxt, step, weights, nseg, ng_next, last) = req[1], req[3]
+    _call("pt_k_ls_select", a.skip, a.gammas, nxt, step, a.f1, a.f2, weights, nseg, req[2],
+          ng_next, last, st)
 
 
 def _dp(t, k=0):

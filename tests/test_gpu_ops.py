@@ -532,3 +532,151 @@ def test_tomo_linesearch_follows_the_sweeps(nt, nz, n, fit):
     assert np.array_equal(got, ref) and np.array_equal(state.cpu().numpy(), s2.cpu().numpy())
     if fit > 2.0 ** -20:
         assert 0.45 * fit < got[0] <= 1.8 * fit
+
+
+@pytest.mark.parametrize("det,P,n,nz,step", [(8, 8, 40, 33, 3), (8, 5, 33, 40, 2),
+                                             (16, 16, 64, 49, 4), (16, 11, 50, 61, 3)])
+@pytest.mark.parametrize("model", ["poisson", "gaussian"])
+def test_ptycho_grad_small_frames_vs_fp64(det, P, n, nz, step, model):
+    """Fused gradient of 8 x 8 and 16 x 16 frames, probes that fill the frame and
+    smaller odd ones, against FP64; a skipped position, frames of an object that
+    is zero there, a last group of patches that does not fill a wave, and the
+    grouped call of the same.  Tolerance: the FP64 forward's final rounding and
+    an FP32 inverse transform (1e-7 each, 8 passes): under 1e-5."""
+    from ptychotomo_amd import _lib, objects
+    from ptychotomo_amd._dev import ptr, stream
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"small frames det={det} P={P} n={n} nz={nz} {model}", flush=True)
+    rng = np.random.default_rng(det + P)
+    nt, cp, cd, rho = 3, 1.1, 0.9, 0.7
+    scan = objects.jittered_raster(nt, nz, n, P, step, 1.0, rng)
+    scan[0, 0, 1] = -0.8
+    prb = crandn(rng, (P, P))
+    op = ptychofft(nt, nz, n, nt, scan.shape[2], det, det, P)
+    sc, pr = dev(scan), dev(prb)
+    op.setobj(sc.data_ptr(), pr.data_ptr())
+    sh = (nt, nz, n)
+    psi = np.exp(1j * 0.3 * rng.standard_normal(sh)).astype(np.complex64)
+    psi[2] = 0
+    h, lamd = crandn(rng, sh), crandn(rng, sh) * np.float32(0.1)
+    data = rng.poisson(4.0, (nt, scan.shape[2], det, det)).astype(np.float32)
+    a = cp * optycho.fwd(psi, prb, scan, det, det, np.complex128)
+    q = np.float64(np.float32(cd)) * data
+    if model == "poisson":
+        r = a - q * a / (np.abs(a) ** 2 + 1e-32)
+    else:
+        r = a - np.sqrt(q) * np.exp(1j * np.angle(np.where(a == 0, 0, a)))  # angle(0) = 0
+    ref = cp * optycho.adj(r, prb, scan, nz, n, np.complex128) - rho * (h - psi + lamd / rho)
+    mdl = _lib.PT_MODEL[model]
+    t = {k: dev(v) for k, v in dict(psi=psi, h=h, lamd=lamd, data=data).items()}
+    out, out2 = (torch.zeros(sh, dtype=torch.complex64, device="cuda") for _ in range(2))
+    _lib.call("pt_ptycho_grad", op._h, ptr(out), ptr(t["psi"]), ptr(t["data"]), ptr(t["h"]),
+              ptr(t["lamd"]), rho, None, cp, cd, mdl, stream())
+    arr = (_lib.GradArgs * 1)(_lib.GradArgs(op._h, out2.data_ptr(), t["psi"].data_ptr(),
+                                            t["data"].data_ptr(), t["h"].data_ptr(),
+                                            t["lamd"].data_ptr(), rho, None, cp, cd))
+    _lib.call("pt_ptycho_grad_group", arr, 1, mdl, stream())
+    e = rel(out.cpu().numpy(), ref)
+    print(f"grad {e:.2e}")
+    assert e < 1e-5, e
+    assert torch.equal(torch.view_as_real(out), torch.view_as_real(out2))
+
+
+@pytest.mark.parametrize("n,pz,ntheta", [(20, 3, 11), (64, 3, 20), (36, 9, 14)])
+def test_tomo_grid_corners_are_not_read(n, pz, ntheta):
+    """The grid's corners beyond the samples' disc are neither written nor read:
+    after a pass over NaN in each direction the results equal a fresh handle's
+    (generic and register line passes, an odd slice count)."""
+    from ptychotomo_amd.radonusfft import radonusfft
+    print(f"grid corners n={n} pz={pz} ntheta={ntheta}", flush=True)
+    rng = np.random.default_rng(n)
+    th = dev(np.linspace(0, np.pi, ntheta, endpoint=False).astype(np.float32))
+    u, g = dev(crandn(rng, (pz, n, n))), dev(crandn(rng, (ntheta, pz, n)))
+    un, gn = torch.full_like(u, float("nan")), torch.full_like(g, float("nan"))
+    res = []
+    for stale in (False, True):
+        op = radonusfft(ntheta, pz, n)
+        op.setobj(th.data_ptr())
+        f, b = torch.zeros_like(g), torch.zeros_like(u)
+        if stale:
+            op.fwd(f.data_ptr(), un.data_ptr())
+            op.adj(b.data_ptr(), gn.data_ptr())
+            op.fwd(f.data_ptr(), un.data_ptr())
+        op.adj(b.data_ptr(), g.data_ptr())
+        if stale:
+            op.adj(un.data_ptr(), gn.data_ptr())
+        op.fwd(f.data_ptr(), u.data_ptr())
+        torch.cuda.synchronize()
+        res.append((f.cpu().numpy(), b.cpu().numpy()))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("det,P,n,nz,step", [(16, 16, 72, 56, 4), (8, 8, 40, 40, 8),
+                                             (32, 32, 64, 64, 8), (64, 20, 90, 80, 9)])
+@pytest.mark.parametrize("model", ["poisson", "gaussian"])
+def test_ptycho_linesearch_sweep_is_its_parts(det, P, n, nz, step, model):
+    """pt_ptycho_linesearch_sweep against pt_ptycho_linesearch and
+    pt_k_ls_select over a whole search: the same state, step and candidates
+    after every sweep (the sums differ in FP64 order only), for frames on the
+    overlap-add tiles, sparse ones, 32 x 32 ones and 64 x 64 ones with a large
+    probe; chunks that accept early, later and not before the step is below FP32
+    resolution (an ascent direction)."""
+    import ctypes
+    from ptychotomo_amd import _lib, objects
+    from ptychotomo_amd._dev import ptr, stream
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"sweep det={det} P={P} {model}", flush=True)
+    rng = np.random.default_rng(n + det)
+    nt, chunk, cp, cd = 6, 2, 1.1, 0.9
+    nc, mdl = nt // chunk, _lib.PT_MODEL[model]
+    scan = objects.jittered_raster(nt, nz, n, P, step, 1.0, rng)
+    op = ptychofft(nt, nz, n, nt, scan.shape[2], det, det, P)
+    sc, pr = dev(scan), dev(objects.gaussian_probe(P, P / 4) * np.float32(3))
+    op.setobj(sc.data_ptr(), pr.data_ptr())
+    sh = (nt, nz, n)
+    t = dict(psi=np.exp(1j * 0.3 * rng.standard_normal(sh)), h=crandn(rng, sh),
+             lamd=crandn(rng, sh) * 0.1,
+             data=rng.poisson(4.0, (nt, scan.shape[2], det, det)).astype(np.float32))
+    t = {k: dev(v if k == "data" else v.astype(np.complex64)) for k, v in t.items()}
+    d = torch.zeros(sh, dtype=torch.complex64, device="cuda")
+    _lib.call("pt_ptycho_grad", op._h, ptr(d), ptr(t["psi"]), ptr(t["data"]), ptr(t["h"]),
+              ptr(t["lamd"]), 0.7, None, cp, cd, mdl, stream())
+    d *= -0.2
+    d[chunk:2 * chunk] *= 30.0
+    d[2 * chunk:] *= -1.0
+    w = torch.tensor([1.0, 0.7], dtype=torch.float64, device="cuda")
+    z = lambda k: torch.zeros(k, dtype=torch.float64, device="cuda")  # noqa: E731
+    sched = (2, 5) + (7,) * 5 + (3,)
+    runs = []
+    for fused in (False, True):
+        state, stp, f1, f2 = z(2 * nc), z(2 * nc), z(8 * nc), z(8 * nc)
+        bufs = [z(8 * nc), z(8 * nc)]
+        state[0::2] = 2.0
+        _lib.call("pt_k_ls_begin", ptr(state), ptr(bufs[0]), nc, sched[0] + 1, stream())
+        trace = []
+        for s, k in enumerate(sched):
+            last = int(s == len(sched) - 1)
+            ng, nx = k + 1, (sched[s] if last else sched[s + 1]) + 1
+            cur, nxt = bufs[s % 2], bufs[(s + 1) % 2]
+            a = _lib.LinesearchArgs(op._h, f1.data_ptr(), f2.data_ptr(), t["psi"].data_ptr(),
+                                    d.data_ptr(), t["data"].data_ptr(), t["h"].data_ptr(),
+                                    t["lamd"].data_ptr(), 0.7, None, cur.data_ptr(), chunk, cp, cd,
+                                    state.data_ptr())
+            if fused:
+                _lib.call("pt_ptycho_linesearch_sweep", ctypes.byref(a), ptr(nxt), ptr(stp), ptr(w),
+                          ng, nx, last, mdl, stream())
+            else:
+                _lib.call("pt_ptycho_linesearch", op._h, ptr(f1), ptr(f2), ptr(t["psi"]), ptr(d),
+                          ptr(t["data"]), ptr(t["h"]), ptr(t["lamd"]), 0.7, None, ptr(cur), ng,
+                          chunk, cp, cd, mdl, ptr(state), stream())
+                _lib.call("pt_k_ls_select", ptr(state), ptr(cur), ptr(nxt), ptr(stp), ptr(f1),
+                          ptr(f2), ptr(w), nc, ng, nx, last, stream())
+            trace.append([x.cpu().numpy().copy() for x in (state, stp, nxt)])
+        runs.append(trace)
+    print("steps", runs[1][-1][1][0::2])
+    for a, b in zip(*runs):
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x, y)
+    assert np.all(runs[1][-1][0][1::2] == 1.0)
+    assert runs[1][-1][1][0] > 1e-3 > 1e-5 > runs[1][-1][1][4]
