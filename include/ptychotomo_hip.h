@@ -410,6 +410,17 @@ int pt_k_tomo_linesearch(double* state, double* step, const void* K, const void*
                          const void* Rd, const void* xi0, const void* u, const void* d,
                          const void* xi1, const double* w, long len, int nz, int ny, int nx,
                          pt_stream stream);
+/* The end of an ADMM iteration (solver.py:322-330), in place, with device FP64
+ * scalars.  split: e_new = J u, phi = soft threshold of e_new + mu/tau at
+ * alpha/tau, mu += tau (e_new - phi); norms = {||phi - e_new||^2,
+ * ||e_new - e||^2}; e = e_new.  object: h_new = exp(i c Ru) exp(i pshift)
+ * (pshift = {phase, cos, sin} as pt_k_takexi_dev leaves it), lamd += rho
+ * (h_new - psi); norms = {||psi - h_new||^2, ||h_new - h||^2}; h = h_new. */
+int pt_k_split_update(double* norms, void* phi, void* e, void* mu, const void* u,
+                      const double* tau, double alpha, int nz, int ny, int nx, pt_stream stream);
+int pt_k_object_update(double* norms, void* h, void* lamd, const void* psi, const void* Ru,
+                       double c, const double* pshift, const double* rho, long len,
+                       pt_stream stream);
 /* Residual balancing (solver.py:267-282): rho_tau = {rho, tau} updated in
  * place from norms = {||psi-h||^2, ||h-h0||^2, ||phi-e||^2, ||e-e0||^2}. */
 int pt_k_penalty(double* rho_tau, const double* norms, pt_stream stream);

@@ -135,6 +135,8 @@ _SIGS = {
     "pt_k_intensity": (c_int, [vp, vp, c_float, c_long, vp]),
     "pt_k_dual": (c_int, [vp, vp, vp, vp, c_double, vp, c_int, c_long, vp]),
     "pt_k_dai_yuan": (c_int, [vp, vp, c_int, vp]),
+    "pt_k_split_update": (c_int, [vp] * 6 + [c_double, c_int, c_int, c_int, vp]),
+    "pt_k_object_update": (c_int, [vp] * 5 + [c_double, vp, vp, c_long, vp]),
     "pt_k_ls_begin": (c_int, [vp, vp, c_int, c_int, vp]),
     "pt_k_ls_select": (c_int, [vp, vp, vp, vp, vp, vp, vp, c_int, c_int, c_int, c_int, vp]),
     "pt_k_tomo_linesearch": (c_int, [vp] * 10 + [c_long, c_int, c_int, c_int, vp]),

@@ -345,6 +345,66 @@ struct FExpTomo {
   }
 };
 
+// The end of an ADMM iteration as two passes over its states (solver.py:257-264,
+// 322-330).  Element-wise the formulas of FRegSolve, FRegFwd, FExpTomo, FDual and
+// FNorm2Lin; v[0], v[1] = the primal and dual residual sums of the penalty update.
+// Bound: memory.  As separate kernels with copies of the new h and e they moved 13
+// and 12 arrays' worth where these read and write 6 and 5 (e, phi, mu: 403 MB each
+// at 256^3; h, lamd, psi, Ru: 201 MB at 384 angles): 1.5 -> 0.64 ms there.
+struct FSplitTail {  // phi, mu and e from u: v = |phi - e|^2, |e - e_old|^2
+  float2* phi; float2* e; float2* mu; const float2* u; SV tau; double alpha; int nz, ny, nx;
+  __device__ void operator()(long i, double (&v)[2]) const {
+    const double t = tau.get();
+    const float itau = (float)(1.0 / t), thr = (float)(alpha / t), tf = (float)t;
+    const long plane = (long)nz * ny * nx;
+    const int x = (int)(i % nx);
+    const long r = i / nx;
+    const int y = (int)(r % ny);
+    const int z = (int)(r / ny);
+    const float c = 1.15470053837925152902f;  // 2/sqrt(3)
+    const float2 w = u[i];
+    float2 g[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)}, q[3], m[3];
+    if (x < nx - 1) { float2 s = u[i + 1]; g[0] = make_float2((s.x - w.x) * c, (s.y - w.y) * c); }
+    if (y < ny - 1) { float2 s = u[i + nx]; g[1] = make_float2((s.x - w.x) * c, (s.y - w.y) * c); }
+    if (z < nz - 1) { float2 s = u[i + (long)ny * nx]; g[2] = make_float2((s.x - w.x) * c, (s.y - w.y) * c); }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      m[k] = mu[k * plane + i];
+      q[k] = make_float2(g[k].x + m[k].x * itau, g[k].y + m[k].y * itau);
+      ss += q[k].x * q[k].x + q[k].y * q[k].y;
+    }
+    const float za = sqrtf(ss), sh = thr / za;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const long j = k * plane + i;
+      const float2 p = za <= thr ? make_float2(0.f, 0.f)
+                                 : make_float2(q[k].x - sh * q[k].x, q[k].y - sh * q[k].y);
+      const float2 d = csub(g[k], p), o = csub(g[k], e[j]);
+      phi[j] = p;
+      mu[j] = make_float2(m[k].x + tf * d.x, m[k].y + tf * d.y);
+      e[j] = g[k];
+      v[0] += (double)d.x * d.x + (double)d.y * d.y;
+      v[1] += (double)o.x * o.x + (double)o.y * o.y;
+    }
+  }
+};
+struct FObjectTail {  // h and lamd from Ru: v = |psi - h|^2, |h - h_old|^2
+  float2* h; float2* lamd; const float2* psi; const float2* Ru; float c; const double* ph; SV rho;
+  __device__ void operator()(long i, double (&v)[2]) const {
+    const float2 p = Ru[i];
+    const float a = expf(-c * p.y), rf = (float)rho.get();
+    float sn, cs;
+    sincosf(c * p.x, &sn, &cs);
+    const float2 hn = cmul(make_float2(a * cs, a * sn), make_float2((float)ph[1], (float)ph[2]));
+    const float2 l = lamd[i], d = csub(hn, psi[i]), o = csub(hn, h[i]);
+    lamd[i] = make_float2(l.x + rf * d.x, l.y + rf * d.y);
+    h[i] = hn;
+    v[0] += (double)d.x * d.x + (double)d.y * d.y;
+    v[1] += (double)o.x * o.x + (double)o.y * o.y;
+  }
+};
+
 __device__ __forceinline__ float2 mlog_c(float2 x) {
   const float m = hypotf(x.x, x.y);
   if (m < 1e-32f) return make_float2(logf(1e-32f), 0.f);
@@ -1154,6 +1214,27 @@ extern "C" int pt_k_tomo_linesearch(double* state, double* step, const void* K, 
     PT_LAUNCH_CHECK();
   }
   return PT_OK;
+}
+extern "C" int pt_k_split_update(double* norms, void* phi, void* e, void* mu, const void* u,
+                                 const double* tau, double alpha, int nz, int ny, int nx,
+                                 pt_stream stream) {
+  PT_REQUIRE(norms && phi && e && mu && u && tau, PT_ERR_ARG, "pt_k_split_update: null argument");
+  PT_REQUIRE(nz > 0 && ny > 0 && nx > 0, PT_ERR_SIZE, "pt_k_split_update: sizes must be positive");
+  return seg_reduce<2>(norms, (long)nz * ny * nx, 1,
+                       FSplitTail{(float2*)phi, (float2*)e, (float2*)mu, (const float2*)u,
+                                  SV{0.0, tau}, alpha, nz, ny, nx},
+                       (hipStream_t)stream);
+}
+extern "C" int pt_k_object_update(double* norms, void* h, void* lamd, const void* psi,
+                                  const void* Ru, double c, const double* pshift,
+                                  const double* rho, long len, pt_stream stream) {
+  PT_REQUIRE(norms && h && lamd && psi && Ru && pshift && rho, PT_ERR_ARG,
+             "pt_k_object_update: null argument");
+  PT_REQUIRE(len > 0, PT_ERR_SIZE, "pt_k_object_update: len must be positive");
+  return seg_reduce<2>(norms, len, 1,
+                       FObjectTail{(float2*)h, (float2*)lamd, (const float2*)psi,
+                                   (const float2*)Ru, (float)c, pshift, SV{0.0, rho}},
+                       (hipStream_t)stream);
 }
 extern "C" int pt_k_ls_begin(double* state, double* cand, int nseg, int ngam, pt_stream stream) {
   PT_REQUIRE(state && cand && nseg > 0, PT_ERR_ARG, "pt_k_ls_begin: bad argument");

