@@ -410,6 +410,14 @@ int pt_k_tomo_linesearch(double* state, double* step, const void* K, const void*
                          const void* Rd, const void* xi0, const void* u, const void* d,
                          const void* xi1, const double* w, long len, int nz, int ny, int nx,
                          pt_stream stream);
+/* A CG step of cg_tomo (solver.py:186-191): Ru += step[0] Rd (Rd NULL: as it
+ * is), r = scale * conj(K) (K Ru - xi0), and grad += tau * J*(J u - xi1); as
+ * pt_k_axpy_seg, pt_k_tomo_resid and pt_k_reg_grad without the sums.  step,
+ * scale and tau: device FP64. */
+int pt_k_cg_resid(void* r, void* Ru, const void* Rd, const double* step, const void* K,
+                  const void* xi0, const double* scale, long len, pt_stream stream);
+int pt_k_cg_reg_grad(void* grad, const void* u, const void* xi1, const double* tau, int nz, int ny,
+                     int nx, pt_stream stream);
 /* The end of an ADMM iteration (solver.py:322-330), in place, with device FP64
  * scalars.  split: e_new = J u, phi = soft threshold of e_new + mu/tau at
  * alpha/tau, mu += tau (e_new - phi); norms = {||phi - e_new||^2,

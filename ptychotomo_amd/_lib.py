@@ -135,6 +135,8 @@ _SIGS = {
     "pt_k_intensity": (c_int, [vp, vp, c_float, c_long, vp]),
     "pt_k_dual": (c_int, [vp, vp, vp, vp, c_double, vp, c_int, c_long, vp]),
     "pt_k_dai_yuan": (c_int, [vp, vp, c_int, vp]),
+    "pt_k_cg_resid": (c_int, [vp] * 7 + [c_long, vp]),
+    "pt_k_cg_reg_grad": (c_int, [vp] * 4 + [c_int, c_int, c_int, vp]),
     "pt_k_split_update": (c_int, [vp] * 6 + [c_double, c_int, c_int, c_int, vp]),
     "pt_k_object_update": (c_int, [vp] * 5 + [c_double, vp, vp, c_long, vp]),
     "pt_k_ls_begin": (c_int, [vp, vp, c_int, c_int, vp]),

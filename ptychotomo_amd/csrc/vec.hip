@@ -478,11 +478,14 @@ __device__ __forceinline__ void grad3(const float2* __restrict__ u, long i, int 
 struct FRegGrad {
   float2* grad; const float2* u; const float2* xi1; SV tau; int nz, ny, nx;
   __device__ void operator()(long i, double (&v)[1]) const {
-    const long plane = (long)nz * ny * nx;
     const int x = (int)(i % nx);
     const long r = i / nx;
     const int y = (int)(r % ny);
     const int z = (int)(r / ny);
+    at(i, x, y, z, v);
+  }
+  __device__ __forceinline__ void at(long i, int x, int y, int z, double (&v)[1]) const {
+    const long plane = (long)nz * ny * nx;
     float2 g[3];
     grad3(u, i, x, y, z, nz, ny, nx, g);
     float2 w[3];
@@ -511,6 +514,35 @@ struct FRegGrad {
     grad[i] = make_float2(gv.x + c * s.x, gv.y + c * s.y);
   }
 };
+// A CG step's two element-wise passes of cg_tomo (FTomoResid and FRegGrad without
+// their sums, which the solver does not use: no second pass).  The residual pass
+// first makes the previous step's Ru += step Rd, whose result only it reads
+// (TAIL5).  The gradient pass runs over planes (blockIdx.y = z), one 32-bit
+// division per voxel instead of 64-bit ones: REGG.
+struct FCgResid {
+  float2* r; float2* Ru; const float2* Rd; const double* step; const float2* K; const float2* xi0;
+  SV scale;
+  __device__ void operator()(long i) const {
+    float2 ru = Ru[i];
+    if (Rd) {
+      ru = cadd(ru, cmul(make_float2((float)step[0], (float)step[1]), Rd[i]));
+      Ru[i] = ru;
+    }
+    const float2 k = K[i];
+    const float2 e = csub(cmul(k, ru), xi0[i]);
+    r[i] = cscale(cmul(cconj(k), e), (float)scale.get());
+  }
+};
+__global__ __launch_bounds__(256) void k_cg_reg_grad(FRegGrad f) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= f.ny * f.nx) return;
+  const int y = (int)((unsigned)p / (unsigned)f.nx), x = p - y * f.nx;
+  for (int z = blockIdx.y; z < f.nz; z += gridDim.y) {
+    double v[1];
+    f.at((long)z * f.ny * f.nx + p, x, y, z, v);
+  }
+}
+
 // Line-search candidates, formed as the reference forms them: the stepped
 // quantity x + gamma*dx element-wise in FP32 (a step below FP32 resolution
 // gives exactly the gamma = 0 value).  What is summed (in FP64) is the change
@@ -1213,6 +1245,25 @@ extern "C" int pt_k_tomo_linesearch(double* state, double* step, const void* K, 
                        g0, g1);
     PT_LAUNCH_CHECK();
   }
+  return PT_OK;
+}
+extern "C" int pt_k_cg_resid(void* r, void* Ru, const void* Rd, const double* step, const void* K,
+                             const void* xi0, const double* scale, long len, pt_stream stream) {
+  PT_REQUIRE(r && Ru && K && xi0 && scale && (!Rd || step), PT_ERR_ARG,
+             "pt_k_cg_resid: null argument");
+  return map(len, FCgResid{(float2*)r, (float2*)Ru, (const float2*)Rd, step, (const float2*)K,
+                           (const float2*)xi0, SV{0.0, scale}}, (hipStream_t)stream);
+}
+extern "C" int pt_k_cg_reg_grad(void* grad, const void* u, const void* xi1, const double* tau,
+                                int nz, int ny, int nx, pt_stream stream) {
+  PT_REQUIRE(grad && u && xi1 && tau, PT_ERR_ARG, "pt_k_cg_reg_grad: null argument");
+  PT_REQUIRE(nz > 0 && ny > 0 && nx > 0 && (long)ny * nx <= 0x7fffff00L, PT_ERR_SIZE,
+             "pt_k_cg_reg_grad: bad size");
+  hipLaunchKernelGGL(k_cg_reg_grad, dim3((unsigned)((ny * nx + 255) / 256), std::min(nz, 65535)),
+                     dim3(256), 0, (hipStream_t)stream,
+                     FRegGrad{(float2*)grad, (const float2*)u, (const float2*)xi1, SV{0.0, tau},
+                              nz, ny, nx});
+  PT_LAUNCH_CHECK();
   return PT_OK;
 }
 extern "C" int pt_k_split_update(double* norms, void* phi, void* e, void* mu, const void* u,

@@ -362,7 +362,8 @@ class Solver(object):
     def _cg_tomo_dev(self, xi0, xi1, K, u, Ru, blk, titer, hist=None):
         """cg_tomo on u in place; Ru = R u is carried by linearity
         (R(u + g d) = R u + g R d), so a CG iteration costs one adjoint and one
-        forward USFFT."""
+        forward USFFT.  Ru is left as before the last step (nothing needs it
+        then)."""
         nz, n = self.nz, self.n
         lenp, lenu = Ru.numel(), u.numel()
         st = stream()
@@ -370,18 +371,17 @@ class Solver(object):
         if "r_t" not in w or w["r_t"].shape != Ru.shape:
             w["r_t"], w["Rd"] = empty(Ru.shape), empty(Ru.shape)
         r_t, Rd, d = w["r_t"], w["Rd"], w["d"]
-        sc = w["sc"]
         w["state"].copy_(w["state0"])             # gamma = 2 (solver.py:184)
         ct = float(self.coeftomo)
         grad0 = None
         for i in range(titer):
             grad = w["grad"][i % 2]
-            # grad = rho*R*(conj(K)(K Ru - xi0)) + tau*J*(J u - xi1)
-            _call("pt_k_tomo_resid", ptr(r_t), _dp(sc, 0), ptr(K), ptr(Ru), ptr(xi0), 0.0,
-                  _dp(blk, _RHO), lenp, st)
+            # grad = rho*R*(conj(K)(K Ru - xi0)) + tau*J*(J u - xi1); the previous
+            # step's Ru += g R d on the way
+            _call("pt_k_cg_resid", ptr(r_t), ptr(Ru), ptr(Rd) if i else None, ptr(w["step"]),
+                  ptr(K), ptr(xi0), _dp(blk, _RHO), lenp, st)
             self._tomo.adj_scaled(grad.data_ptr(), r_t.data_ptr(), ct)
-            _call("pt_k_reg_grad", ptr(grad), _dp(sc, 1), ptr(u), ptr(xi1), 0.0, _dp(blk, _TAU),
-                  nz, n, n, st)
+            _call("pt_k_cg_reg_grad", ptr(grad), ptr(u), ptr(xi1), _dp(blk, _TAU), nz, n, n, st)
             self._dai_yuan_dev(w, i, grad, grad0, lenu, 1)
             grad0 = grad
             self._tomo.fwd_scaled(Rd.data_ptr(), d.data_ptr(), ct)
@@ -390,7 +390,6 @@ class Solver(object):
             _call("pt_k_tomo_linesearch", ptr(w["state"]), ptr(w["step"]), ptr(K), ptr(Ru),
                   ptr(Rd), ptr(xi0), ptr(u), ptr(d), ptr(xi1), _dp(blk, _RHO), lenp, nz, n, n, st)
             _call("pt_k_axpy_seg", ptr(u), ptr(w["step"]), ptr(d), lenu, 1, st)
-            _call("pt_k_axpy_seg", ptr(Ru), ptr(w["step"]), ptr(Rd), lenp, 1, st)
             if hist is not None:
                 hist[i:i + 1].copy_(w["step"][0:1])
 
