@@ -719,14 +719,15 @@ __device__ __forceinline__ void stage_tw64(double2* tw) {
     if (threadIdx.x < 64) tw[threadIdx.x] = make_double2(cospi(threadIdx.x / 32.0), -sinpi(threadIdx.x / 32.0));
 }
 
-// the probe, scaled and twisted, in lane order: prl[j * WAVE + lane] (one wave)
-template <int D>
+// the probe, scaled and twisted, in lane order: prl[j * WAVE + lane] (all W waves)
+template <int W, int D>
 __device__ __forceinline__ void stage_probe(float2* prl, const float2* __restrict__ prb,
-                                            const WaveFrame<D>& fr, int lane, int P, int o,
+                                            const WaveFrame<D>& fr, int wave, int lane, int P, int o,
                                             float scale, const double2* tw) {
   const int px = fr.ix() - o;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int k = 0; k < 16 / W; ++k) {
+    const int j = wave + W * k;
     const int py = fr.iy(j) - o;
     float2 q = make_float2(0.f, 0.f);
     if (px >= 0 && px < P && py >= 0 && py < P)
@@ -799,7 +800,7 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
   if (threadIdx.x < PT_MAX_GAM)
     gsh[threadIdx.x] = threadIdx.x < ngam ? (float)gammas[(long)c * ngam + threadIdx.x] : 0.f;
   __syncthreads();
-  if (wave == 0) stage_probe<D>(prl, prb, fr, lane, P, o, scale, tw);
+  stage_probe<kMinfWWaves>(prl, prb, fr, wave, lane, P, o, scale, tw);
   __syncthreads();
   float* T = Tb[wave];
   double acc[PT_MAX_GAM];
@@ -864,7 +865,13 @@ void k_minf_wave(double* __restrict__ partial, const float2* __restrict__ f,
   }
 }
 
-// k_fwd for 32 x 32 frames and for 64 x 64 frames with probes up to 16 pixels
+// k_fwd for 32 x 32 frames and for 64 x 64 frames with probes up to 16 pixels.  A
+// wave takes one patch while that needs at most kFwdWBlocks workgroups (four per
+// CU), beyond that up to four, which share the staged probe.  Four in a row from the
+// first patch on left few frames to a fraction of the CUs: 968 frames of 32 x 32 19
+// -> 7.8 us, 392 of 64 x 64 42 -> 12 us; at 26912 frames of 32 x 32 four per wave
+// take 59 us.  Bound there: the far field written (3.7 TB/s).
+constexpr int kFwdWBlocks = 1024;
 template <int D, bool INT>
 __global__ __launch_bounds__(WAVE * kMinfWWaves, 3)
 void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* __restrict__ f,
@@ -880,7 +887,7 @@ void k_fwd_wave(float2* __restrict__ g, float* __restrict__ out, const float2* _
   const int o = D == 32 ? ox : 0;
   stage_tw64<D>(tw);
   __syncthreads();
-  if (wave == 0) stage_probe<D>(prl, prb, fr, lane, P, o, cs, tw);
+  stage_probe<kMinfWWaves>(prl, prb, fr, wave, lane, P, o, cs, tw);
   __syncthreads();
   const long per = (npatch + gridDim.x - 1) / gridDim.x;
   const long b0 = (long)xcd_contig(blockIdx.x, gridDim.x) * per;
@@ -1776,9 +1783,10 @@ int run_fwd(pt_ptycho* h, float2* g, float* out, const float2* f, float scale, f
   ProfScope prof("ptycho_fwd", st);
   if constexpr (D >= 32) {
     if (wave_frames(h)) {
-      // 4 patches per wave where that leaves whole rounds of the chip
-      hipLaunchKernelGGL((k_fwd_wave<D, INT>), dim3(launch_blocks(np, 4 * kMinfWWaves, 1 << 20)),
-                         dim3(WAVE * kMinfWWaves), 0, st, g, out, f, h->prb, h->pos, h->shift, np,
+      const int nw = (int)std::min<long>(4, 1 + (np - 1) / (kMinfWWaves * kFwdWBlocks));
+      const int nb = launch_blocks(np, nw * kMinfWWaves, 1 << 20);
+      hipLaunchKernelGGL((k_fwd_wave<D, INT>), dim3(nb), dim3(WAVE * kMinfWWaves), 0, st, g, out, f,
+                         h->prb, h->pos, h->shift, np,
                          h->nz, h->n, h->S, h->P, h->ox, h->c * scale, isc);
       PT_LAUNCH_CHECK();
       return PT_OK;

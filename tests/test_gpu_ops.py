@@ -743,3 +743,60 @@ def test_admm_tail_passes_vs_fp64(nz, ny, nx, nt):
     n = blk.cpu().numpy()[5:]
     sq = lambda x: (np.abs(x) ** 2).sum()  # noqa: E731
     np.testing.assert_allclose(n, [sq(phi - g), sq(g - e0), sq(psi - hn), sq(hn - h)], rtol=2e-6)
+
+
+def _device_us(f, reps=20, rounds=7):
+    """device time of one call among `reps` back to back: the least of `rounds`"""
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    f()
+    best = np.inf
+    for _ in range(rounds):
+        a.record()
+        for _ in range(reps):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / reps)
+    return best
+
+
+@pytest.mark.parametrize("det,P,n,step", [(32, 32, 128, 16), (64, 16, 128, 16), (64, 9, 90, 10)])
+def test_ptycho_fwd_patches_per_wave(det, P, n, step):
+    """Large frames' far fields with one to four patches per wave (the counts
+    around the rule's steps, 4096 patches per step): each angle's as the
+    operator of a few angles gives it, bit for bit.  And a few hundred patches,
+    which fit the device at once, take no longer than 1.8 times what four take
+    (four patches in a row on a quarter of the waves took 2.3 to 3.3 times)."""
+    from ptychotomo_amd import objects
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"fwd patches per wave det={det} P={P}", flush=True)
+    S = objects.jittered_raster(1, n, n, P, step, 1.0, np.random.default_rng(0)).shape[2]
+    nt = 4 * 4096 // S + 2
+    rng = np.random.default_rng(det + P)
+    scan = objects.jittered_raster(nt, n, n, P, step, 1.0, rng)
+    psi = dev(np.exp(1j * 0.3 * rng.standard_normal((nt, n, n))).astype(np.complex64))
+    pr = dev(objects.gaussian_probe(P, P / 4))
+
+    def op_of(nta, nscan):
+        op = ptychofft(nta, n, n, nta, nscan, det, det, P)
+        sc = dev(np.ascontiguousarray(scan[:, :nta, :nscan]))
+        op.setobj(sc.data_ptr(), pr.data_ptr())
+        return op, torch.empty((nta, nscan, det, det), dtype=torch.complex64, device="cuda")
+    one, ref = op_of(1, S)
+    one.fwd(ref.data_ptr(), psi.data_ptr())
+    for k in range(1, 5):
+        for nta in (k * 4096 // S, k * 4096 // S + 1):
+            op, far = op_of(nta, S)
+            op.fwd(far.data_ptr(), psi.data_ptr())
+            assert torch.equal(far[0], ref[0]), (k, nta)
+            few, last = op_of(1, S)
+            sc = dev(np.ascontiguousarray(scan[:, nta - 1:nta]))
+            few.setobj(sc.data_ptr(), pr.data_ptr())
+            few.fwd(last.data_ptr(), psi[nta - 1].data_ptr())
+            assert torch.equal(far[-1], last[0]), (k, nta)
+    four, f4 = op_of(1, 4)
+    many, fm = op_of(max(1, 256 // S), S)
+    t4 = _device_us(lambda: four.fwd(f4.data_ptr(), psi.data_ptr()))
+    tm = _device_us(lambda: many.fwd(fm.data_ptr(), psi.data_ptr()))
+    print(f"4 patches {t4:.1f} us, {fm.shape[0] * S} patches {tm:.1f} us")
+    assert tm < 1.8 * t4, (t4, tm)
