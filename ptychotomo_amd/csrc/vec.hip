@@ -1101,17 +1101,26 @@ __global__ void k_ls_select(double* __restrict__ state, const double* cand, doub
             ngam_next, last, [&](int j) { return w0 * a[j] + (b ? w1 * b[j] : 0.0); });
 }
 
-// cg_tomo's whole halving search (solver.py:171-183) in two sweeps: the first
-// kTLFirst halvings, which the solver's searches rarely pass, then all that are
-// left down to 1e-12 in groups of kTLFirst.  Each sweep is an evaluation (both
-// functional terms, blockIdx.y) and a one-workgroup kernel that sums the partials
-// in a fixed order and applies the halving rule; the second pair exits at once
-// when the first accepted a step.  4 launches instead of the 31 of six sweeps of
-// two reductions, their finishing passes and a selection: latency-bound in small
-// problems (cg_tomo at 128^3, 4 steps: 2.34 -> 2.16 ms).
+// cg_tomo's whole halving search (solver.py:171-183) in groups of kTLFirst
+// halvings.  A sweep takes one or several groups: an evaluation (both functional
+// terms, blockIdx.y) and a one-workgroup kernel that sums the partials in a fixed
+// order and applies the halving rule; a sweep after the accepted step exits at once.
+// 4 to 12 launches instead of the 31 of six sweeps of two reductions, their finishing
+// passes and a selection.
+// Which groups share a sweep: a sweep that exits costs 3.4 us, a group that need not
+// have been evaluated 10 us at 96 x 64^2, 48 us at 192 x 128^2, 400 us at 384 x 256^2
+// (bound: K, Ru, Rd, xi0, u, d, xi1 read once per group).  Up to kTLSmall blocks of
+// 1024 elements the first group has a sweep and all others share one; up to kTLLarge
+// the first three have one each; beyond that every group has.  Step accepted in the
+// first / second / third group: 23 / 75 / 77 us (96 x 64^2), 70 / 125 / 179 us
+// (192 x 128^2), 430 / 850 / 1260 us (384 x 256^2); with all groups after the first in
+// one sweep the latter took 70 / 295 / 304 and 418 / 2420 / 2430 us.  Half the blocks
+// up to kTLLarge: the selection then reads half the partials (at 192 x 128^2 75 -> 70
+// us; at 384 x 256^2 435 -> 454).
 constexpr int kTLFirst = 7;    // halvings per group (slot 0 is gamma = 0)
 constexpr int kTLGroups = 6;   // groups in all: 42 halvings, 2 -> below 1e-12
 constexpr int kTLBlocks = 2048;  // per term: 8 per CU
+constexpr long kTLSmall = 1024, kTLLarge = 8192;
 __global__ __launch_bounds__(RB) void k_tomo_ls_eval(double* __restrict__ partial, FTomoMinf ft,
                                                      long lenp, FRegMinf fr, long lenu,
                                                      const double* __restrict__ state, int g0,
@@ -1228,7 +1237,8 @@ extern "C" int pt_k_tomo_linesearch(double* state, double* step, const void* K, 
              "pt_k_tomo_linesearch: sizes must be positive");
   hipStream_t st = (hipStream_t)stream;
   const long lenu = (long)nz * ny * nx;
-  const int nblk = (int)std::min<long>(kTLBlocks, (std::max(len, lenu) + RB * 4 - 1) / (RB * 4));
+  const long nb = (std::max(len, lenu) + RB * 4 - 1) / (RB * 4);
+  const int nblk = (int)std::min<long>(nb <= kTLLarge ? kTLBlocks / 2 : kTLBlocks, nb);
   double* part;
   const int rc = partial_buf((size_t)kTLGroups * 2 * nblk * PT_MAX_CAND, &part, st);
   if (rc) return rc;
@@ -1236,8 +1246,12 @@ extern "C" int pt_k_tomo_linesearch(double* state, double* step, const void* K, 
                      nullptr, kTLFirst + 1};
   const FRegMinf fr{(const float2*)u, (const float2*)d, (const float2*)xi1, nullptr, kTLFirst + 1,
                     nz, ny, nx};
-  for (int sw = 0; sw < 2; ++sw) {
-    const int g0 = sw, g1 = sw ? kTLGroups : 1;
+  // the first group of each sweep
+  static constexpr int few[] = {0, 1, kTLGroups}, some[] = {0, 1, 2, 3, kTLGroups},
+                       all[] = {0, 1, 2, 3, 4, 5, kTLGroups};
+  const int* at = nb <= kTLSmall ? few : nb <= kTLLarge ? some : all;
+  for (; at[0] < kTLGroups; ++at) {
+    const int g0 = at[0], g1 = at[1];
     hipLaunchKernelGGL(k_tomo_ls_eval, dim3(nblk, 2), dim3(RB), 0, st, part, ft, len, fr, lenu,
                        state, g0, g1);
     PT_LAUNCH_CHECK();

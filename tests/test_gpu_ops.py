@@ -800,3 +800,66 @@ def test_ptycho_fwd_patches_per_wave(det, P, n, step):
     tm = _device_us(lambda: many.fwd(fm.data_ptr(), psi.data_ptr()))
     print(f"4 patches {t4:.1f} us, {fm.shape[0] * S} patches {tm:.1f} us")
     assert tm < 1.8 * t4, (t4, tm)
+
+
+@pytest.mark.parametrize("nt,nz,n", [(8, 32, 180), (130, 64, 128), (16, 208, 204)])
+def test_tomo_linesearch_groups_of_halvings(nt, nz, n):
+    """pt_k_tomo_linesearch where all later groups of halvings share a sweep,
+    where the first three have their own and where every group has: the steps of
+    the search made from its parts, accepted in each group and never.  And a step
+    accepted at the tenth halving (second group) of a problem that memory bounds
+    takes no longer than 2.8 times one accepted at the second (reading everything
+    once more is 1.6 times; evaluating all later groups for it took 3.5)."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    print(f"tomo line search groups nt={nt} nz={nz} n={n}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    cr = lambda *sh: torch.view_as_complex(  # noqa: E731
+        torch.randn((*sh, 2), generator=gen, device="cuda"))
+
+    def J(v):
+        o = torch.zeros((3, *v.shape), dtype=v.dtype, device="cuda")
+        o[0, :, :, :-1], o[1, :, :-1], o[2, :-1] = (v.diff(dim=k) for k in (2, 1, 0))
+        return o * (2 / 3 ** 0.5)
+
+    z = lambda *v: torch.tensor(v, dtype=torch.float64, device="cuda")  # noqa: E731
+    w = z(0.5, 0.25)
+
+    def search(nt, nz, n, fits):
+        K, Ru, Rd = (cr(nt, nz, n) for _ in range(3))
+        u, d = cr(nz, n, n), cr(nz, n, n)
+        for fit in fits:
+            xi0, xi1 = K * (Ru + 0.9 * fit * Rd), J(u + 0.9 * fit * d)
+            state, step = z(2.0, 0.0), z(7.0, 7.0)
+
+            def run():
+                state[0] = 2.0
+                _lib.call("pt_k_tomo_linesearch", ptr(state), ptr(step), ptr(K), ptr(Ru), ptr(Rd),
+                          ptr(xi0), ptr(u), ptr(d), ptr(xi1), ptr(w), K.numel(), nz, n, n,
+                          stream())
+
+            def parts():
+                s2, p2 = z(2.0, 0.0), z(7.0, 7.0)
+                c, f1, f2 = (torch.zeros(8, dtype=torch.float64, device="cuda") for _ in range(3))
+                _lib.call("pt_k_ls_begin", ptr(s2), ptr(c), 1, 8, stream())
+                for sw in range(6):
+                    _lib.call("pt_k_tomo_minf", ptr(f1), ptr(K), ptr(Ru), ptr(Rd), ptr(xi0), ptr(c),
+                              8, K.numel(), ptr(s2), stream())
+                    _lib.call("pt_k_reg_minf", ptr(f2), ptr(u), ptr(d), ptr(xi1), ptr(c), 8, nz, n,
+                              n, ptr(s2), stream())
+                    _lib.call("pt_k_ls_select", ptr(s2), ptr(c), ptr(c), ptr(p2), ptr(f1), ptr(f2),
+                              ptr(w), 1, 8, 8, int(sw == 5), stream())
+                return s2, p2
+            run()
+            yield fit, run, step, state, parts
+
+    for fit, _, step, state, parts in search(nt, nz, n, [1.0, 2.0 ** -8, 2.0 ** -15, 2.0 ** -22, -1.0]):
+        s2, p2 = parts()
+        print(fit, step.tolist(), p2.tolist())
+        assert torch.equal(step, p2) and torch.equal(state, s2), fit
+        if fit > 0:
+            assert 0.45 * fit < step[0].item() <= 1.8 * fit
+    if nt == 130:
+        us = [_device_us(run, 5) for _, run, *_ in search(192, 128, 128, [1.0, 2.0 ** -9])]
+        print("accepted in the first, second group:", us)
+        assert us[1] < 2.8 * us[0], us
