@@ -249,6 +249,19 @@ int pt_ptycho_linesearch_sweep(const pt_ptycho_linesearch_args* a, double* cand_
  * instances use ngam candidates and the given model. */
 int pt_ptycho_linesearch_group(const pt_ptycho_linesearch_args* a, int n, int ngam, int model,
                                pt_stream stream);
+/* One sweep of the line search of n independent reconstructions (the arguments
+ * of pt_ptycho_linesearch_sweep that differ between them in s): grouped as
+ * pt_ptycho_linesearch_group, with the decisions of a group in one launch.
+ * Sums, their order and decisions are those of n calls of
+ * pt_ptycho_linesearch_sweep, bit for bit. */
+typedef struct pt_ptycho_sweep_args {
+  double* cand_next;
+  double* step;
+  const double* w;
+} pt_ptycho_sweep_args;
+int pt_ptycho_linesearch_sweep_group(const pt_ptycho_linesearch_args* a,
+                                     const pt_ptycho_sweep_args* s, int n, int ngam, int ngam_next,
+                                     int last, int model, pt_stream stream);
 
 /* pt_ptycho_minf for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc).  No

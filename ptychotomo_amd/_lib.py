@@ -56,6 +56,11 @@ class LinesearchArgs(ctypes.Structure):
                 ("chunk", c_int), ("coefptycho", c_float), ("coefdata", c_float), ("skip", vp)]
 
 
+class SweepArgs(ctypes.Structure):
+    """pt_ptycho_sweep_args (one instance of pt_ptycho_linesearch_sweep_group)"""
+    _fields_ = [("cand_next", vp), ("step", vp), ("w", vp)]
+
+
 class GradArgs(ctypes.Structure):
     """pt_ptycho_grad_args (one instance of pt_ptycho_grad_group)"""
     _fields_ = [("h", vp), ("grad", vp), ("psi", vp), ("data", vp), ("hh", vp), ("lamd", vp),
@@ -98,6 +103,8 @@ _SIGS = {
                                        c_int, c_int, vp, vp]),
     "pt_ptycho_linesearch_sweep": (c_int, [ctypes.POINTER(LinesearchArgs), vp, vp, vp, c_int, c_int,
                                            c_int, c_int, vp]),
+    "pt_ptycho_linesearch_sweep_group": (c_int, [ctypes.POINTER(LinesearchArgs),
+                                                 ctypes.POINTER(SweepArgs)] + [c_int] * 5 + [vp]),
     "pt_ptycho_linesearch": (c_int, [vp, vp, vp, vp, vp, vp, vp, vp, c_double, vp, vp, c_int,
                                      c_int, c_float, c_float, c_int, vp, vp]),
     "pt_ptycho_linesearch_group": (c_int, [ctypes.POINTER(LinesearchArgs), c_int, c_int, c_int,

@@ -5,7 +5,7 @@ Each instance keeps its own ``Solver`` (operators sized for it) and its own
 stream.  An ADMM iteration advances every instance in lock-step: the
 ptychography CG's heavy launches -- the fused gradient and each line-search
 sweep -- are made as one grouped launch for all instances
-(``pt_ptycho_grad_group`` / ``pt_ptycho_linesearch_group``: every instance's
+(``pt_ptycho_grad_group`` / ``pt_ptycho_linesearch_sweep_group``: every instance's
 overlap-add tiles in one grid), and the rest of each instance's iteration
 runs on its own stream, so small instances overlap on the device.  Without
 grouping, the iteration can also be captured as one HIP graph per iteration
@@ -18,7 +18,7 @@ import torch
 
 from . import _lib
 from ._dev import stream
-from .solver import Solver, run_ptycho_request, select_request
+from .solver import Solver, run_ptycho_request
 
 
 class BatchSolver:
@@ -155,9 +155,9 @@ class BatchSolver:
                     _lib.call("pt_ptycho_grad_group", arr, n, mdl, st)
                 else:
                     arr = (_lib.LinesearchArgs * n)(*[r[1] for r in reqs])
-                    _lib.call("pt_ptycho_linesearch_group", arr, n, ng, mdl, st)
-                    for r in reqs:
-                        select_request(r, st)
+                    sw = (_lib.SweepArgs * n)(*[r[3][:3] for r in reqs])
+                    _lib.call("pt_ptycho_linesearch_sweep_group", arr, sw, n, ng, *reqs[0][3][3:],
+                              mdl, st)
                 reqs = [next(g) for g in gens]
             if any(r[0] != "end" for r in reqs):
                 raise RuntimeError("BatchSolver: instances out of step")

@@ -1246,9 +1246,9 @@ struct LsFinishArgs {
   int nb[2];
   int ngam, ngam_next, last;
 };
-__global__ __launch_bounds__(1024) void k_ls_finish(LsFinishArgs A) {
+__device__ __forceinline__ void ls_finish_body(const LsFinishArgs& A, int c) {
   __shared__ double f[2][PT_MAX_GAM];
-  const int c = blockIdx.x, wid = threadIdx.x / WAVE, lane = lane_id();
+  const int wid = threadIdx.x / WAVE, lane = lane_id();
   if (A.state[2 * c + 1] != 0.0) return;
   const int term = wid / PT_MAX_GAM, j = wid % PT_MAX_GAM;
   if (j < A.ngam) {
@@ -1269,6 +1269,15 @@ __global__ __launch_bounds__(1024) void k_ls_finish(LsFinishArgs A) {
 #pragma clang fp contract(off)
               return w0 * f[0][k] + w1 * f[1][k];
             });
+}
+__global__ __launch_bounds__(1024) void k_ls_finish(LsFinishArgs A) {
+  ls_finish_body(A, blockIdx.x);
+}
+// the same for a group of instances (their chunks flattened): the same sums in the
+// same order, so that a grouped sweep decides as the instance's own would
+__global__ __launch_bounds__(1024) void k_ls_finish_group(Group<LsFinishArgs> g) {
+  const int i = group_find(g, blockIdx.x);
+  ls_finish_body(g.a[i], blockIdx.x - g.start[i]);
 }
 
 // LDS bytes of a k_minf_tile workgroup
@@ -1948,6 +1957,14 @@ inline void minf_dispatch(int model, bool full, int ngam, F&& fn) {
   }
 }
 
+// the partials of a line search on tiles, as k_ls_finish reads them
+inline void ls_tile_partials(LsFinishArgs* F, const double* part, const double* part_rho, int nbt) {
+  for (int t = 0; t < 2; ++t) {
+    F->p[t] = t ? part_rho : part;
+    F->cs[t] = (long)F->ngam * nbt; F->js[t] = nbt; F->bs[t] = 1; F->nb[t] = nbt;
+  }
+}
+
 template <int D>
 int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, const float* data,
              const double* gammas, int ngam, int chunk, float cp, float cd, int model, int lagr,
@@ -1976,12 +1993,8 @@ int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, con
     }
     PT_LAUNCH_CHECK();
     if (rt.fin) {
-      LsFinishArgs& F = *rt.fin;
-      for (int t = 0; t < 2; ++t) {
-        F.p[t] = t ? part_rho : part;
-        F.cs[t] = (long)ngam * nbt; F.js[t] = nbt; F.bs[t] = 1; F.nb[t] = nbt;
-      }
-      hipLaunchKernelGGL(k_ls_finish, dim3(nchunk), dim3(1024), 0, st, F);
+      ls_tile_partials(rt.fin, part, part_rho, nbt);
+      hipLaunchKernelGGL(k_ls_finish, dim3(nchunk), dim3(1024), 0, st, *rt.fin);
       PT_LAUNCH_CHECK();
       return PT_OK;
     }
@@ -2431,48 +2444,71 @@ extern "C" int pt_ptycho_linesearch(pt_ptycho* h, double* f1, double* f2, const 
                                      nullptr, 0, rt)));
 }
 
+// the sweep's arguments checked (of instance inst of a group, or inst = -1); its
+// decision's arguments
+static int sweep_args(const pt_ptycho_linesearch_args& a, const pt_ptycho_sweep_args& s, int ngam,
+                      int ngam_next, int last, int model, int inst, LsFinishArgs* F) {
+  auto err = [&](const char* msg) {
+    return inst < 0 ? std::string("pt_ptycho_linesearch_sweep: ") + msg
+                    : std::string("pt_ptycho_linesearch_sweep_group: ") + msg + " (instance " +
+                          std::to_string(inst) + ")";
+  };
+  PT_REQUIRE(a.h && a.psi && a.dir && a.data && a.hh && a.lamd && a.gammas && a.skip &&
+                 s.cand_next && s.step && s.w,
+             PT_ERR_ARG, err("null argument"));
+  const pt_ptycho* h = a.h;
+  PT_REQUIRE(h->ready, PT_ERR_STATE, err("set_scan_probe not called"));
+  PT_REQUIRE(ngam >= 2 && ngam <= PT_MAX_GAM && ngam_next >= 2 && ngam_next <= PT_MAX_GAM,
+             PT_ERR_ARG, err("2 <= ngam, ngam_next <= 8"));
+  PT_REQUIRE(a.chunk > 0 && h->pt % a.chunk == 0, PT_ERR_SIZE,
+             err("chunk must divide the number of angles"));
+  PT_REQUIRE(model == PT_MODEL_POISSON || model == PT_MODEL_GAUSSIAN, PT_ERR_ARG,
+             err("bad model"));
+  PT_REQUIRE(a.rho_dev || a.rho > 0, PT_ERR_ARG, err("rho must be positive"));
+  PT_REQUIRE(s.cand_next != a.gammas || ngam_next == ngam || h->pt == a.chunk, PT_ERR_ARG,
+             err("a sweep of another width needs its own candidate buffer"));
+  *F = LsFinishArgs{};
+  F->state = const_cast<double*>(a.skip);
+  F->cand = a.gammas; F->cand_next = s.cand_next; F->step = s.step; F->w = s.w;
+  F->ngam = ngam; F->ngam_next = ngam_next; F->last = last;
+  return PT_OK;
+}
+
+static RhoTerm rho_term(const pt_ptycho_linesearch_args& a, LsFinishArgs* fin) {
+  RhoTerm rt;
+  rt.hh = (const float2*)a.hh;
+  rt.lamd = (const float2*)a.lamd;
+  rt.rho = a.rho;
+  rt.rho_dev = a.rho_dev;
+  rt.f2 = a.f2;
+  rt.fin = fin;
+  return rt;
+}
+
 extern "C" int pt_ptycho_linesearch_sweep(const pt_ptycho_linesearch_args* a, double* cand_next,
                                           double* step, const double* w, int ngam, int ngam_next,
                                           int last, int model, pt_stream stream) {
-  PT_REQUIRE(a && a->h && a->psi && a->dir && a->data && a->hh && a->lamd && a->gammas &&
-                 a->skip && cand_next && step && w,
-             PT_ERR_ARG, "pt_ptycho_linesearch_sweep: null argument");
+  PT_REQUIRE(a, PT_ERR_ARG, "pt_ptycho_linesearch_sweep: null argument");
+  LsFinishArgs F;
+  const int rc = sweep_args(*a, {cand_next, step, w}, ngam, ngam_next, last, model, -1, &F);
+  if (rc) return rc;
   pt_ptycho* h = a->h;
-  PT_REQUIRE(h->ready, PT_ERR_STATE, "pt_ptycho_linesearch_sweep: set_scan_probe not called");
-  PT_REQUIRE(ngam >= 2 && ngam <= PT_MAX_GAM && ngam_next >= 2 && ngam_next <= PT_MAX_GAM,
-             PT_ERR_ARG, "pt_ptycho_linesearch_sweep: 2 <= ngam, ngam_next <= 8");
-  PT_REQUIRE(a->chunk > 0 && h->pt % a->chunk == 0, PT_ERR_SIZE,
-             "pt_ptycho_linesearch_sweep: chunk must divide the number of angles");
-  PT_REQUIRE(model == PT_MODEL_POISSON || model == PT_MODEL_GAUSSIAN, PT_ERR_ARG,
-             "pt_ptycho_linesearch_sweep: bad model");
-  PT_REQUIRE(a->rho_dev || a->rho > 0, PT_ERR_ARG,
-             "pt_ptycho_linesearch_sweep: rho must be positive");
-  PT_REQUIRE(cand_next != a->gammas || ngam_next == ngam || h->pt == a->chunk, PT_ERR_ARG,
-             "pt_ptycho_linesearch_sweep: a sweep of another width needs its own candidate buffer");
-  LsFinishArgs F = {};
-  F.state = const_cast<double*>(a->skip);
-  F.cand = a->gammas; F.cand_next = cand_next; F.step = step; F.w = w;
-  F.ngam = ngam; F.ngam_next = ngam_next; F.last = last;
-  RhoTerm rt;
-  rt.hh = (const float2*)a->hh;
-  rt.lamd = (const float2*)a->lamd;
-  rt.rho = a->rho;
-  rt.rho_dev = a->rho_dev;
-  rt.fin = &F;
+  const RhoTerm rt = rho_term(*a, &F);
   hipStream_t st = (hipStream_t)stream;
   PT_DISPATCH_D(h->D, (run_minf<DD>(h, nullptr, (const float2*)a->psi, (const float2*)a->dir,
                                     a->data, a->gammas, ngam, a->chunk, a->coefptycho,
                                     a->coefdata, model, 0, a->skip, st, nullptr, 0, rt)));
 }
 
-// One launch of k_minf_tile_group (and the two grouped reductions) for the
-// instances idx (at most kGroupMax, all on the tile path with detector D and
-// the same probe form)
+// One launch of k_minf_tile_group and the two grouped reductions, or the grouped
+// decisions (fin, by instance), for the instances idx (at most kGroupMax, all on the
+// tile path with detector D and the same probe form)
 template <int D>
-static int run_minf_group(const pt_ptycho_linesearch_args* a, const int* idx, int n, int ngam,
-                          int model, bool full, hipStream_t st) {
+static int run_minf_group(const pt_ptycho_linesearch_args* a, LsFinishArgs* fin, const int* idx,
+                          int n, int ngam, int model, bool full, hipStream_t st) {
   Group<MinfTileArgs> g;
   Group<ReduceArgs> r1, r2;
+  Group<LsFinishArgs> gf;
   size_t lds = 0;
   int tot = 0, totc = 0;
   for (int k = 0; k < n; ++k) {
@@ -2484,27 +2520,26 @@ static int run_minf_group(const pt_ptycho_linesearch_args* a, const int* idx, in
     double* part;
     int rc = minf_partials(h, 2 * nper, nullptr, 0, &part);
     if (rc) return rc;
-    RhoTerm rt;
-    rt.hh = (const float2*)x.hh;
-    rt.lamd = (const float2*)x.lamd;
-    rt.rho = x.rho;
-    rt.rho_dev = x.rho_dev;
-    rt.f2 = x.f2;
     g.a[k] = minf_tile_args(h, part, part + nper, (const float2*)x.psi, (const float2*)x.dir,
-                            x.data, x.gammas, ngam, x.chunk, x.coefptycho, x.coefdata, x.skip, rt);
+                            x.data, x.gammas, ngam, x.chunk, x.coefptycho, x.coefdata, x.skip,
+                            rho_term(x, nullptr));
     g.gx[k] = nbt;
     g.start[k] = tot;
     tot += g.gx[k] * nchunk;
     r1.a[k] = ReduceArgs{x.f1, part, x.skip, (long)nbt};
     r2.a[k] = ReduceArgs{x.f2, part + nper, x.skip, (long)nbt};
-    r1.gx[k] = r2.gx[k] = nchunk;
-    r1.start[k] = r2.start[k] = totc;
+    if (fin) {
+      ls_tile_partials(&fin[idx[k]], part, part + nper, nbt);
+      gf.a[k] = fin[idx[k]];
+    }
+    r1.gx[k] = r2.gx[k] = gf.gx[k] = nchunk;
+    r1.start[k] = r2.start[k] = gf.start[k] = totc;
     totc += nchunk;
     lds = std::max(lds, minf_tile_lds_bytes(D, h->EB, h->P));
   }
   g.start[n] = tot;
-  r1.start[n] = r2.start[n] = totc;
-  g.n = r1.n = r2.n = n;
+  r1.start[n] = r2.start[n] = gf.start[n] = totc;
+  g.n = r1.n = r2.n = gf.n = n;
   {
     ProfScope prof("ptycho_minf", st);
     minf_dispatch<D>(model, full, ngam, [&](auto, auto kern) {
@@ -2512,10 +2547,45 @@ static int run_minf_group(const pt_ptycho_linesearch_args* a, const int* idx, in
     });
   }
   PT_LAUNCH_CHECK();
+  if (fin) {
+    hipLaunchKernelGGL(k_ls_finish_group, dim3(totc), dim3(1024), 0, st, gf);
+    PT_LAUNCH_CHECK();
+    return PT_OK;
+  }
   hipLaunchKernelGGL(k_reduce_partials_group, dim3(totc, ngam), dim3(256), 0, st, r1, ngam);
   PT_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_reduce_partials_group, dim3(totc, ngam), dim3(256), 0, st, r2, ngam);
   PT_LAUNCH_CHECK();
+  return PT_OK;
+}
+
+// groups of (detector size, probe form) on the tile path, kGroupMax at a time; every
+// other instance by single(i)
+template <class F>
+static int minf_groups(const pt_ptycho_linesearch_args* a, LsFinishArgs* fin, int n, int ngam,
+                       int model, hipStream_t st, F single) {
+  std::vector<int> bins[4];  // D = 8 / 16, probe partial / full
+  for (int i = 0; i < n; ++i) {
+    const pt_ptycho* h = a[i].h;
+    int b = -1;
+    if (h->D == 8 && minf_tile_path<8>(h)) b = minf_full<8>(h) ? 1 : 0;
+    if (h->D == 16 && minf_tile_path<16>(h)) b = 2 + (minf_full<16>(h) ? 1 : 0);
+    if (b >= 0) {
+      bins[b].push_back(i);
+      continue;
+    }
+    const int rc = single(i);
+    if (rc) return rc;
+  }
+  for (int b = 0; b < 4; ++b) {
+    for (size_t k0 = 0; k0 < bins[b].size(); k0 += kGroupMax) {
+      const int m = (int)std::min<size_t>(kGroupMax, bins[b].size() - k0);
+      const int* idx = bins[b].data() + k0;
+      const int rc = b < 2 ? run_minf_group<8>(a, fin, idx, m, ngam, model, b == 1, st)
+                           : run_minf_group<16>(a, fin, idx, m, ngam, model, b == 3, st);
+      if (rc) return rc;
+    }
+  }
   return PT_OK;
 }
 
@@ -2544,35 +2614,32 @@ extern "C" int pt_ptycho_linesearch_group(const pt_ptycho_linesearch_args* a, in
   PT_REQUIRE(distinct_handles(a, n), PT_ERR_ARG,
              "pt_ptycho_linesearch_group: a handle appears twice (its partial sums would be "
              "shared)");
-  hipStream_t st = (hipStream_t)stream;
-  // groups of (detector size, probe form) on the tile path, kGroupMax at a time;
-  // every other instance as pt_ptycho_linesearch
-  std::vector<int> bins[4];  // D = 8 / 16, probe partial / full
-  for (int i = 0; i < n; ++i) {
-    const pt_ptycho* h = a[i].h;
-    int b = -1;
-    if (h->D == 8 && minf_tile_path<8>(h)) b = minf_full<8>(h) ? 1 : 0;
-    if (h->D == 16 && minf_tile_path<16>(h)) b = 2 + (minf_full<16>(h) ? 1 : 0);
-    if (b >= 0) {
-      bins[b].push_back(i);
-      continue;
-    }
+  return minf_groups(a, nullptr, n, ngam, model, (hipStream_t)stream, [&](int i) {
     const pt_ptycho_linesearch_args& x = a[i];
-    int rc = pt_ptycho_linesearch(x.h, x.f1, x.f2, x.psi, x.dir, x.data, x.hh, x.lamd, x.rho,
-                                  x.rho_dev, x.gammas, ngam, x.chunk, x.coefptycho, x.coefdata,
-                                  model, x.skip, stream);
+    return pt_ptycho_linesearch(x.h, x.f1, x.f2, x.psi, x.dir, x.data, x.hh, x.lamd, x.rho,
+                                x.rho_dev, x.gammas, ngam, x.chunk, x.coefptycho, x.coefdata,
+                                model, x.skip, stream);
+  });
+}
+
+extern "C" int pt_ptycho_linesearch_sweep_group(const pt_ptycho_linesearch_args* a,
+                                                const pt_ptycho_sweep_args* s, int n, int ngam,
+                                                int ngam_next, int last, int model,
+                                                pt_stream stream) {
+  PT_REQUIRE(n >= 0 && ((a && s) || n == 0), PT_ERR_ARG,
+             "pt_ptycho_linesearch_sweep_group: bad argument");
+  std::vector<LsFinishArgs> fin(n);
+  for (int i = 0; i < n; ++i) {
+    const int rc = sweep_args(a[i], s[i], ngam, ngam_next, last, model, i, &fin[i]);
     if (rc) return rc;
   }
-  for (int b = 0; b < 4; ++b) {
-    for (size_t k0 = 0; k0 < bins[b].size(); k0 += kGroupMax) {
-      const int m = (int)std::min<size_t>(kGroupMax, bins[b].size() - k0);
-      const int* idx = bins[b].data() + k0;
-      const int rc = b < 2 ? run_minf_group<8>(a, idx, m, ngam, model, b == 1, st)
-                           : run_minf_group<16>(a, idx, m, ngam, model, b == 3, st);
-      if (rc) return rc;
-    }
-  }
-  return PT_OK;
+  PT_REQUIRE(distinct_handles(a, n), PT_ERR_ARG,
+             "pt_ptycho_linesearch_sweep_group: a handle appears twice (its partial sums would "
+             "be shared)");
+  return minf_groups(a, fin.data(), n, ngam, model, (hipStream_t)stream, [&](int i) {
+    return pt_ptycho_linesearch_sweep(&a[i], s[i].cand_next, s[i].step, s[i].w, ngam, ngam_next,
+                                      last, model, stream);
+  });
 }
 
 extern "C" int pt_ptycho_minf(pt_ptycho* h, double* sums, const void* psi, const void* dir,

@@ -320,10 +320,10 @@ class Solver(object):
         generator: yields (cand, ngam, state, f1, f2, select) where the two
         functional terms (their change from gamma = 0) are to be evaluated at
         the ngam candidate slots per segment, skipping finished segments, and
-        the sweep's selection is to be made with the arguments `select` (by the
-        caller, alone or in a group of instances); weights points to the terms'
-        two FP64 weights.  Consecutive sweeps alternate between two candidate
-        buffers."""
+        the sweep's selection is to be made with the arguments `select` (next
+        candidates, steps, weights, ngam of the next sweep, last; by the caller,
+        alone or in a group of instances); weights points to the terms' two FP64
+        weights.  Consecutive sweeps alternate between two candidate buffers."""
         st = stream()
         bufs = (w["cand"], w["cand2"])
         ng = sched[0] + 1
@@ -332,8 +332,8 @@ class Solver(object):
             last = sw == len(sched) - 1
             ng_next = ng if last else sched[sw + 1] + 1
             cur, nxt = bufs[sw % 2], bufs[(sw + 1) % 2]
-            yield cur, ng, w["state"], w["f1"], w["f2"], (ptr(nxt), ptr(w["step"]), weights, nseg,
-                                                          ng_next, int(last))
+            yield cur, ng, w["state"], w["f1"], w["f2"], (nxt.data_ptr(), w["step"].data_ptr(),
+                                                          weights.value, ng_next, int(last))
             ng = ng_next
 
     def _dai_yuan_dev(self, w, i, grad, grad0, L, nseg):
@@ -433,8 +433,7 @@ class Solver(object):
         gradient and each line-search sweep -- are yielded as requests
         ("grad", GradArgs) and ("ls", LinesearchArgs, ngam, select) for the caller
         to make (run_ptycho_request, or one grouped call for many instances in
-        lock-step, then select_request); everything else is enqueued here on the
-        current stream."""
+        lock-step); everything else is enqueued here on the current stream."""
         st = stream()
         L = psi.numel()
         w = self._work(("ptycho", id(op)), nseg, psi.shape)
@@ -681,15 +680,8 @@ def run_ptycho_request(req, mdl, st):
         _call("pt_ptycho_grad", a.h, a.grad, a.psi, a.data, a.hh, a.lamd, a.rho, a.rho_dev,
               a.coefptycho, a.coefdata, mdl, st)
     else:
-        nxt, step, weights, _, ng_next, last = req[3]
+        nxt, step, weights, ng_next, last = req[3]
         _call("pt_ptycho_linesearch_sweep", a, nxt, step, weights, req[2], ng_next, last, mdl, st)
-
-
-def select_request(req, st):
-    """The selection of a ("ls", ...) request whose two terms are evaluated."""
-    a, (nxt, step, weights, nseg, ng_next, last) = req[1], req[3]
-    _call("pt_k_ls_select", a.skip, a.gammas, nxt, step, a.f1, a.f2, weights, nseg, req[2],
-          ng_next, last, st)
 
 
 def _dp(t, k=0):

@@ -231,3 +231,80 @@ def test_group_entries_match_single_calls():
     # one handle twice in a group: refused before any launch
     with pytest.raises(_lib.PtError, match="twice"):
         _lib.call("pt_ptycho_grad_group", (_lib.GradArgs * 2)(ga[0], ga[0]), 2, mdl, st)
+
+
+def test_group_sweep_decides_as_single_sweeps():
+    """pt_ptycho_linesearch_sweep_group on instances on and off the tile path
+    against pt_ptycho_linesearch_sweep at a near tie: the rho term's weight is
+    walked in steps of one rounding through the value at which the two terms'
+    changes cancel, so a sum that differs in its last bit decides otherwise.  The
+    direction's entries span many powers of two, so that the order of an FP64 sum
+    shows in its last bits.
+    The same state, step and candidates at every weight, and both decisions met."""
+    import ctypes
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd.solver import Solver, _RHO
+    print("grouped sweep at a near tie", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    cplx = lambda sh: torch.complex(torch.randn(sh, device="cuda", generator=g),
+                                    torch.randn(sh, device="cuda", generator=g)) * 0.1
+    f64 = lambda *v: torch.tensor(v, dtype=torch.float64, device="cuda")
+    mdl, st = _lib.PT_MODEL["poisson"], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rows = []
+    for k, (n, step) in enumerate([(64, 4), (48, 4), (128, 4), (64, 16)]):
+        args, obj = _instance(n, 500 + k)
+        if step != 4:        # sparse: off the tile path
+            args = (args[0], objects.jittered_raster(args[6], n, n, 8, step, 1.0,
+                                                     np.random.default_rng(k)), *args[2:])
+        slv = Solver(*args)
+        op = slv._ptycho
+        sh = (slv.ntheta, slv.nz, slv.n)
+        psi = torch.exp(1j * cplx(sh).real).to(torch.complex64).contiguous()
+        d = slv.fwd_ptycho_batch_dev(psi)
+        data = torch.poisson(d * (1e2 / float(d.max())), generator=g).contiguous()
+        nseg, r = slv.nchunk, dict(slv=slv, keep=(psi, data))
+        r.update(blk=f64(1.0, 0.5, 0.5), cand=f64(*[0.0, 0.5, 0.25] * nseg), nxt=f64(*[0.0] * 3 * nseg),
+                 state=f64(*[0.5, 0.0] * nseg), step=f64(*[7.0] * 2 * nseg), w=f64(1.0, 1.0),
+                 f=f64(*[0.0] * 3 * nseg), f2=f64(*[0.0] * 3 * nseg),
+                 dir=cplx(sh) * torch.exp(4 * torch.randn(sh, device="cuda", generator=g)),
+                 h=cplx(sh) + 1, lamd=cplx(sh))
+        p = lambda key: r[key].data_ptr()
+        r["args"] = _lib.LinesearchArgs(op._h, p("f"), p("f2"), psi.data_ptr(), p("dir"),
+                                        data.data_ptr(), p("h"), p("lamd"), 0.0,
+                                        p("blk") + 8 * _RHO, p("cand"), op.Ntheta // nseg,
+                                        float(slv.coefptycho), float(slv.coefdata), p("state"))
+        r["sweep"] = _lib.SweepArgs(p("nxt"), p("step"), p("w"))
+        _lib.call("pt_ptycho_linesearch_group", r["args"], 1, 3, mdl, st)
+        r["tie"] = -float(r["f"][1] / r["f2"][1])
+        rows.append(r)
+    out = ("state", "step", "nxt")
+    arr = (_lib.LinesearchArgs * len(rows))(*[r["args"] for r in rows])
+    sw = (_lib.SweepArgs * len(rows))(*[r["sweep"] for r in rows])
+    seen = [set() for _ in rows]
+    for e in range(-24, 25):
+        got = []
+        for grouped in (False, True):
+            for r in rows:
+                r["state"].copy_(f64(*[0.5, 0.0] * r["slv"].nchunk))
+                r["step"].fill_(7.0)
+                r["nxt"].fill_(-1.0)
+                r["w"][1] = r["tie"] * (1.0 + e * 2.0 ** -52)
+            if grouped:
+                _lib.call("pt_ptycho_linesearch_sweep_group", arr, sw, len(rows), 3, 3, 0, mdl, st)
+            else:
+                for r in rows:
+                    _lib.call("pt_ptycho_linesearch_sweep", r["args"], *(
+                        r[k].data_ptr() for k in ("nxt", "step", "w")), 3, 3, 0, mdl, st)
+            got.append([[r[k].tolist() for k in out] for r in rows])
+        for k, (a, b) in enumerate(zip(*got)):
+            assert a == b, (e, k, a, b)
+            seen[k].add(a[0][0])
+    print("steps met", seen)
+    assert all(len(s) > 1 for s in seen)
+    with pytest.raises(_lib.PtError, match="twice"):
+        _lib.call("pt_ptycho_linesearch_sweep_group",
+                  (_lib.LinesearchArgs * 2)(rows[0]["args"], rows[0]["args"]),
+                  (_lib.SweepArgs * 2)(rows[0]["sweep"], rows[0]["sweep"]), 2, 3, 3, 0, mdl, st)
+    with pytest.raises(_lib.PtError, match="null argument .instance 1"):
+        _lib.call("pt_ptycho_linesearch_sweep_group", arr,
+                  (_lib.SweepArgs * 2)(rows[0]["sweep"], _lib.SweepArgs()), 2, 3, 3, 0, mdl, st)
