@@ -53,8 +53,8 @@ class BatchSolver:
         or a previous state, which may also carry rho, tau and Ru).  m0 is the
         index of the first iteration (the first two iterations of a run take
         piter + 32 ptychography CG steps).  grouped: the ptychography CG's
-        heavy launches of the instances too small to fill the device on
-        their own (fewer than GROUP_TILES overlap-add tiles) as grouped
+        heavy launches of the small instances (fewer than GROUP_TILES
+        overlap-add tiles, where launches count more than overlap) as grouped
         launches; every other instance makes its own launches on its
         stream.  graph (with grouped=False):
         from the third iteration on, one iteration of the whole batch is
@@ -167,10 +167,13 @@ class BatchSolver:
                 for req in g:
                     run_ptycho_request(req, mdl, stream())
 
-    # 16 x 16-pixel tiles of the object's angles below which an instance's
-    # own ptychography launches leave the device partly idle (256 CUs x 6
-    # resident line-search workgroups of 4 tiles each)
-    GROUP_TILES = 6144
+    # 16 x 16-pixel tiles of the object's angles below which an instance is
+    # grouped: its own launches are then so short that fewer of them gain more than
+    # the instances gain by overlapping on their streams.  ms per iteration of the
+    # whole batch, grouped / on streams: 16 of 48^3 (648 tiles) 13.9 / 17.5, 16 of
+    # 64^3 (1536) 15.8 / 17.9, 8 of 72^3 (2187) 10.0 / 10.1, 8 of 80^3 (3000) 12.0 /
+    # 11.2, 16 of 96^3 (5184) 33.8 / 29.0, 4 of 192^3 54.5 / 49.9.
+    GROUP_TILES = 2048
 
     def _small(self, i):
         """whether instance i takes part in the grouped launches"""

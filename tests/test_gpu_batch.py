@@ -308,3 +308,37 @@ def test_group_sweep_decides_as_single_sweeps():
     with pytest.raises(_lib.PtError, match="null argument .instance 1"):
         _lib.call("pt_ptycho_linesearch_sweep_group", arr,
                   (_lib.SweepArgs * 2)(rows[0]["sweep"], _lib.SweepArgs()), 2, 3, 3, 0, mdl, st)
+
+
+@pytest.mark.parametrize("n,count,small", [(48, 8, True), (96, 4, False)])
+def test_default_grouping_is_the_faster_way(n, count, small):
+    """Instances are grouped where that was measured faster than a stream each
+    (up to 64^3, not from 80^3 on), and by default an iteration of either kind takes
+    no longer than 1.15 times the faster of the two ways (48^3 on streams takes 1.3
+    times)."""
+    import time
+    from ptychotomo_amd.batch import BatchSolver
+    print(f"grouping {count} x {n}^3", flush=True)
+    insts = [_instance(n, 700 + i) for i in range(count)]
+    bs = BatchSolver.from_args([a for a, _ in insts])
+    assert [bs._small(i) for i in range(count)] == [small] * count
+    datas = []
+    for slv, (_, obj) in zip(bs.solvers, insts):
+        d = slv.fwd_ptycho_batch_dev(slv.exptomo(slv.fwd_tomo_batch(obj)))
+        datas.append(torch.poisson(d * (1e2 / float(d.max()))))
+    run = lambda st, niter, m0, grouped: bs.admm(datas, st, 3e-7, 4, 4, niter, "poisson",
+                                                 m0=m0, grouped=grouped)
+    run([_init(s) for s in bs.solvers], 3, 0, True)
+    states = [dict(s.state) for s in bs.solvers]
+    best = {}
+    for _ in range(4):
+        for name, tiles, grouped in (("default", None, True), ("all grouped", 1 << 40, True),
+                                     ("streams", None, False)):
+            bs.GROUP_TILES = BatchSolver.GROUP_TILES if tiles is None else tiles
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            run([dict(s) for s in states], 4, 3, grouped)
+            torch.cuda.synchronize()
+            best[name] = min(best.get(name, np.inf), time.perf_counter() - t)
+    print({k: f"{v * 250:.2f} ms/iteration" for k, v in best.items()})
+    assert best["default"] < 1.15 * min(best.values())
