@@ -981,6 +981,23 @@ __device__ __forceinline__ int group_find(const Group<A>& g, int b) {
   return i;
 }
 
+// tot[j] += the wave's sum of acc[j], j < ngam: lane j adds sum j, one LDS update for
+// all (one per candidate by lane 0 held the wave for each one's read: 5 halvings at
+// 64^2, 32 angles, 16 x 16 frames 132 -> 127 us, 7 halvings with 8 x 8 frames 137 ->
+// 131 us, at 256^2, 96 angles 776 -> 762 us)
+template <int NG>
+__device__ __forceinline__ void add_lane_sums(const double (&acc)[NG], int ngam, double* tot,
+                                              int lane) {
+  double mine = 0.0;
+#pragma unroll
+  for (int j = 0; j < NG; ++j) {
+    if (j >= ngam) break;
+    const double v = wave_sum(acc[j]);
+    mine = lane == j ? v : mine;
+  }
+  if (lane < NG) tot[lane] += mine;
+}
+
 template <int D, int MODEL, int NG, bool FULL>
 __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int bx, int gxn) {
   double* __restrict__ partial = A.partial;
@@ -1127,12 +1144,7 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
         acc[NG - 1] = t0;
       }
     }
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      if (j >= ngam) break;
-      const double v = wave_sum(acc[j]);
-      if (lane == 0) tot[0][wave][j] += v;
-    }
+    add_lane_sums<NG>(acc, ngam, tot[0][wave], lane);
     if (!hh) continue;
     // The functional's rho term (solver.py:213), change of
     // |h - (psi + g*d) + lamd/rho|^2 from g = 0 per pixel, over the pixels
@@ -1160,12 +1172,7 @@ __device__ __forceinline__ void minf_tile_body(const MinfTileArgs& A, int c, int
         }
       }
     }
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      if (j >= ngam) break;
-      const double v = wave_sum(acc[j]);
-      if (lane == 0) tot[1][wave][j] += v;
-    }
+    add_lane_sums<NG>(acc, ngam, tot[1][wave], lane);
   }
   __syncthreads();
   const int term = wave, j = lane;  // two waves: wave 0 the data term, wave 1 the rho term
