@@ -1333,6 +1333,15 @@ struct TileArgs {
   float cs, cp, cd, out_scale;
 };
 
+// a * b with the roundings spelled out: the gradient's FP64 transform takes the
+// rounded products, and the Poisson residual magnifies a change of their last bits
+// where the far field is small, so which product a multiply-add rounds first is not
+// left to the compiler (it chose otherwise for 8 x 8 frames that fill the detector
+// than for the rest)
+__device__ __forceinline__ float2 cmul_fma(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+
 // body of workgroup b of nb (one per tile).  MODEL: the gradient's data model (any
 // value for the adjoint).  FULL: the probe covers the frame, so every frame
 // element is added without a bounds check.
@@ -1413,7 +1422,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& A, int b, int nb) {
     } else {
       load_rows<D>(v, f, ps, t, r, nz, n, P, ox, oy, active);
 #pragma unroll
-      for (int k = 0; k < D; ++k) v[k] = cscale(cmul(prv(k), v[k]), cs);
+      for (int k = 0; k < D; ++k) v[k] = cscale(cmul_fma(prv(k), v[k]), cs);
       // a = coefptycho * F(c * prb * psi), rounded once after an FP64 transform
       float dv[D];
       frame_fwd64_w<D>(v, T, slot, r, cp, [&]() {
@@ -1575,7 +1584,7 @@ __device__ __forceinline__ void tile_body_w(const TileArgs& A, int b, int nb) {
         load_frame<D>(v, A.f + at, fr, n, P, o);
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const float2 q = cmul(prl[j * WAVE + lane], v[j]);
+          const float2 q = cmul_fma(prl[j * WAVE + lane], v[j]);
           x[j] = make_double2((double)q.x, (double)q.y);
         }
         fr.rows(x, T, tw);

@@ -863,3 +863,48 @@ def test_tomo_linesearch_groups_of_halvings(nt, nz, n):
         us = [_device_us(run, 5) for _, run, *_ in search(192, 128, 128, [1.0, 2.0 ** -9])]
         print("accepted in the first, second group:", us)
         assert us[1] < 2.8 * us[0], us
+
+
+@pytest.mark.parametrize("det,P,n,nz,step", [(8, 8, 40, 33, 3), (8, 8, 33, 40, 2), (8, 5, 33, 40, 2),
+                                             (16, 16, 64, 49, 4), (16, 11, 50, 61, 3),
+                                             (32, 32, 64, 64, 8), (64, 16, 64, 64, 6),
+                                             (64, 20, 90, 80, 9)])
+@pytest.mark.parametrize("model", ["poisson", "gaussian"])
+def test_ptycho_grad_rounds_its_products_alike(det, P, n, nz, step, model):
+    """The gradient's FP64 transforms take the products probe x object rounded
+    one way (a multiply-add whose second product is rounded first), whatever the
+    frame size and probe form: against FP64 from products rounded so, what is left
+    is the rounding of residual, FP32 inverse and sums, a few ulp.  With the
+    other product rounded first the Poisson residual differs by 3e-7 to 3e-6."""
+    from ptychotomo_amd import _lib, objects
+    from ptychotomo_amd._dev import ptr, stream
+    from ptychotomo_amd.ptychofft import ptychofft
+    print(f"grad products det={det} P={P} {model}", flush=True)
+    nt, cp, cd, rho = 3, np.float32(1.1), np.float32(0.9), 0.7
+    for seed in range(2):
+        rng = np.random.default_rng(1000 * det + 10 * P + seed)
+        scan = objects.jittered_raster(nt, nz, n, P, step, 1.0, rng)
+        S = scan.shape[2]
+        prb = objects.gaussian_probe(P, P / 4) * np.exp(1j * rng.standard_normal((P, P)))
+        prb = prb.astype(np.complex64)
+        op = ptychofft(nt, nz, n, nt, S, det, det, P)
+        sc, pr = dev(scan), dev(prb)
+        op.setobj(sc.data_ptr(), pr.data_ptr())
+        psi, h, lamd = (crandn(rng, (nt, nz, n)) for _ in range(3))
+        data = rng.poisson(4.0, (nt, S, det, det)).astype(np.float32)
+        a = [dev(v) for v in (psi, data, h, lamd)]
+        out = torch.zeros((nt, nz, n), dtype=torch.complex64, device="cuda")
+        _lib.call("pt_ptycho_grad", op._h, ptr(out), *(ptr(v) for v in a), rho, None, float(cp),
+                  float(cd), _lib.PT_MODEL[model], stream())
+        far = _product_far(psi, prb, scan, det, True) / det * np.float64(cp)
+        d, m = data * np.float64(cd), np.abs(far)
+        res = far - (d / (m ** 2 + 1e-32) if model == "poisson" else np.sqrt(d) / m) * far
+        res = np.fft.ifft2(res) * det * np.float64(cp)
+        ref = -rho * (h - psi.astype(np.complex128) + lamd / rho)
+        pos, o = np.floor(scan + 0.5).astype(int), (det - P) // 2
+        for t, s in np.ndindex(nt, S):
+            x, y = pos[:, t, s]
+            ref[t, y:y + P, x:x + P] += (res[t, s, o:o + P, o:o + P] * prb.conj()).T
+        e = rel(out.cpu().numpy(), ref)
+        print(f"rel {e:.2e}")
+        assert e < 2.5e-7, e
