@@ -908,3 +908,66 @@ def test_ptycho_grad_rounds_its_products_alike(det, P, n, nz, step, model):
         e = rel(out.cpu().numpy(), ref)
         print(f"rel {e:.2e}")
         assert e < 2.5e-7, e
+
+
+@pytest.mark.parametrize("nt,nz,ny,nx", [(3, 1, 5, 7), (5, 9, 33, 16), (2, 4, 1, 300)])
+def test_cg_step_passes(nt, nz, ny, nx):
+    """The element-wise passes of a cg_tomo step: pt_k_cg_resid (with and without
+    the previous step's update of Ru) and pt_k_cg_reg_grad, and their parts
+    pt_k_axpy_seg, pt_k_tomo_resid and pt_k_reg_grad with their sums, against
+    FP64.  A few FP32 operations per element: relative 1e-6."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    print(f"cg step passes {nt} {nz}x{ny}x{nx}", flush=True)
+    rng = np.random.default_rng(nx)
+    K, Ru, Rd, xi0 = (crandn(rng, (nt, nz, nx)) for _ in range(4))
+    u, grad, xi1 = crandn(rng, (nz, ny, nx)), crandn(rng, (nz, ny, nx)), crandn(rng, (3, nz, ny, nx))
+    z = lambda *v: torch.tensor(v, dtype=torch.float64, device="cuda")  # noqa: E731
+    step, rho, tau, sums = z(0.3, 0.0), z(0.7), z(1.9), z(-1.0, -1.0)
+    Kd, Rdd, xd, st = dev(K), dev(Rd), dev(xi0), stream()
+    for upd in (False, True):
+        r, r2, a, b = dev(np.zeros_like(Ru)), dev(np.zeros_like(Ru)), dev(Ru), dev(Ru)
+        _lib.call("pt_k_cg_resid", ptr(r), ptr(a), ptr(Rdd) if upd else None, ptr(step), ptr(Kd),
+                  ptr(xd), ptr(rho), Ru.size, st)
+        if upd:
+            _lib.call("pt_k_axpy_seg", ptr(b), ptr(step), ptr(Rdd), Ru.size, 1, st)
+        _lib.call("pt_k_tomo_resid", ptr(r2), ptr(sums), ptr(Kd), ptr(b), ptr(xd), 0.0, ptr(rho),
+                  Ru.size, st)
+        new = Ru.astype(np.complex128) + 0.3 * upd * Rd
+        e = K.astype(np.complex128) * new - xi0
+        ref = 0.7 * K.conj() * e
+        errs = [rel(a.cpu().numpy(), new), rel(r.cpu().numpy(), ref), rel(r2.cpu().numpy(), ref)]
+        print("Ru, r, r of the parts", errs)
+        assert max(errs) < 1e-6
+        assert rel(a.cpu().numpy(), b.cpu().numpy()) < 1e-7
+        assert rel(r.cpu().numpy(), r2.cpu().numpy()) < 5e-7
+        np.testing.assert_allclose(sums[0].item(), (np.abs(e) ** 2).sum(), rtol=1e-6)
+    ud, x1, g1, g2 = dev(u), dev(xi1), dev(grad), dev(grad)
+    _lib.call("pt_k_cg_reg_grad", ptr(g1), ptr(ud), ptr(x1), ptr(tau), nz, ny, nx, st)
+    _lib.call("pt_k_reg_grad", ptr(g2), ptr(sums), ptr(ud), ptr(x1), 0.0, ptr(tau), nz, ny, nx, st)
+    c, w = 2 / np.sqrt(3), np.zeros((3, nz, ny, nx), np.complex128)
+    U = u.astype(np.complex128)
+    w[0, :, :, :-1], w[1, :, :-1], w[2, :-1] = (np.diff(U, axis=k) * c for k in (2, 1, 0))
+    w -= xi1
+    d = w.sum(0)
+    d[:, :, 1:] -= w[0, :, :, :-1]
+    d[:, 1:] -= w[1, :, :-1]
+    d[1:] -= w[2, :-1]
+    ref = grad - 1.9 * c * d
+    errs = [rel(g1.cpu().numpy(), ref), rel(g2.cpu().numpy(), ref)]
+    print("grad, grad of the reducing pass", errs)
+    assert max(errs) < 1e-6
+    np.testing.assert_allclose(sums[0].item(), (np.abs(w) ** 2).sum(), rtol=1e-6)
+
+
+def test_intensity_of_a_far_field():
+    """pt_k_intensity (out = scale |x|^2) against numpy, with a length that is no
+    multiple of a wave."""
+    from ptychotomo_amd import _lib
+    from ptychotomo_amd._dev import ptr, stream
+    x = crandn(np.random.default_rng(3), (1037,))
+    out = torch.zeros(x.size, dtype=torch.float32, device="cuda")
+    xd = dev(x)
+    _lib.call("pt_k_intensity", ptr(out), ptr(xd), 0.4, x.size, stream())
+    ref = np.float64(np.float32(0.4)) * np.abs(x.astype(np.complex128)) ** 2
+    assert rel(out.cpu().numpy(), ref) < 3e-7
