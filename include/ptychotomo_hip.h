@@ -121,7 +121,10 @@ int pt_tomo_get_line_kernels(pt_tomo* h, int* reg);
 
 /* ptychofft::ptychofft(Ntheta, Nz, N, Ntheta0, Nscan, detx, dety, Nprb)
  * ptychofft.cu:5-33 (Ntheta0 is unused there and here).
- * Requires detx == dety in {8,16,32,64} and nprb <= detx. */
+ * Requires detx == dety in {8,16,32,64} and nprb <= detx.
+ * 64 x 64 frames with nprb > 16 run a lane per frame row: a line-search sweep of 6
+ * candidates takes about 0.8 ms per 1000 frames, with nprb <= 16 (one wave per frame)
+ * 0.025 ms; gradients and adjoints 2 to 7 times as long as with nprb <= 16. */
 int pt_ptycho_create(int ptheta, int nz, int n, int ntheta0, int nscan, int detx, int dety,
                      int nprb, pt_ptycho** out);
 /* ptychofft::~ptychofft  ptychofft.cu:35-46 */
@@ -269,9 +272,10 @@ int pt_ptycho_linesearch_sweep_group(const pt_ptycho_linesearch_args* a,
  * pt_ptycho_minf (the same kernels); its per-launch partial sums live in a
  * fixed per-device array of PT_MINF_NOALLOC_PARTIALS doubles (16 MiB, held
  * until the process ends) instead of the handle's buffer, and the call
- * allocates nothing.  A launch needing more partial sums than that (more
- * than ~1 M overlap-add tiles x candidates; the 256^3, 384-angle workload
- * with 8 candidates needs 1.6 M) fails with PT_ERR_SIZE.  Calls that
+ * allocates nothing.  A launch of more partial sums than that fails with
+ * PT_ERR_SIZE; on overlap-add tiles they are counted as two per tile and
+ * candidate (the limit is ~1 M tiles x candidates; the 256^3, 384-angle workload
+ * with 8 candidates counts 1.6 M), though the kernel writes fewer.  Calls that
  * overlap on one device share the array and race: serialise them (one
  * stream, or events). */
 #define PT_MINF_NOALLOC_PARTIALS (2 * 1024 * 1024)

@@ -1329,7 +1329,7 @@ struct TileArgs {
   const int* tile_start;
   const int* tile_patch;
   const int* tile_slot;
-  int nty, ntx, B, EB, nz, n, S, P, ox, oy, model;
+  int nty, ntx, B, EB, nz, n, S, P, ox, oy;
   float cs, cp, cd, out_scale;
 };
 
@@ -1850,12 +1850,12 @@ inline void tile_dispatch(int model, bool full, F&& fn) {
 }
 
 inline TileArgs tile_args(const pt_ptycho* h, const float2* gin, const float2* f, const float* data,
-                          float cp, float cd, float out_scale, int model) {
+                          float cp, float cd, float out_scale) {
   TileArgs A;
   A.scratch = h->scratch; A.gin = gin; A.f = f; A.data = data; A.prb = h->prb; A.pos = h->pos;
   A.shift = h->shift; A.tile_start = h->tile_start; A.tile_patch = h->tile_patch;
   A.tile_slot = h->tile_slot; A.nty = h->nty; A.ntx = h->ntx; A.B = h->B; A.EB = h->EB;
-  A.nz = h->nz; A.n = h->n; A.S = h->S; A.P = h->P; A.ox = h->ox; A.oy = h->oy; A.model = model;
+  A.nz = h->nz; A.n = h->n; A.S = h->S; A.P = h->P; A.ox = h->ox; A.oy = h->oy;
   A.cs = h->c; A.cp = cp; A.cd = cd; A.out_scale = out_scale;
   return A;
 }
@@ -1863,7 +1863,7 @@ inline TileArgs tile_args(const pt_ptycho* h, const float2* gin, const float2* f
 template <int D, int MODE>
 int run_tiles(pt_ptycho* h, const float2* gin, const float2* f, const float* data, float cp,
               float cd, float out_scale, int model, hipStream_t st) {
-  const TileArgs A = tile_args(h, gin, f, data, cp, cd, out_scale, model);
+  const TileArgs A = tile_args(h, gin, f, data, cp, cd, out_scale);
   ProfScope prof(MODE == TILE_GRAD ? "ptycho_grad_tile" : "ptycho_adj_tile", st);
   if constexpr (D >= 32) {
     if (wave_frames(h)) {
@@ -1892,9 +1892,9 @@ inline int minf_partials(pt_ptycho* h, size_t need, double* fixed, size_t fixed_
                          double** out) {
   if (fixed) {
     PT_REQUIRE(need <= fixed_cap, PT_ERR_SIZE,
-               "pt_ptycho_minf_noalloc: the launch needs " + std::to_string(need) +
-                   " partial sums, more than the fixed buffer's " + std::to_string(fixed_cap) +
-                   " (fewer angles per call, or pt_ptycho_minf)");
+               "pt_ptycho_minf_noalloc: " + std::to_string(need) + " partial sums (on overlap-add "
+                   "tiles counted as one per wave, tile and candidate) exceed the fixed buffer's " +
+                   std::to_string(fixed_cap) + " (fewer angles per call, or pt_ptycho_minf)");
     *out = fixed;
     return PT_OK;
   }
@@ -1993,7 +1993,8 @@ int run_minf(pt_ptycho* h, double* sums, const float2* f, const float2* dir, con
   if constexpr (D <= 16) if (!lagr && dir && minf_tile_path<D>(h)) {
     const int nbt = minf_tile_gx(h, chunk);
     const size_t nper = (size_t)nchunk * nbt * ngam;
-    // a fixed buffer has to hold one partial per wave and tile (the interface's bound)
+    // a fixed buffer's limit counts one partial per wave and tile, as the interface
+    // states it (the kernel writes one per workgroup)
     const size_t need = fixed ? (size_t)nchunk * chunk * h->nty * h->ntx * kMinfWaves * ngam : nper;
     double* part;
     int rc = minf_partials(h, rt.hh ? 2 * need : need, fixed, fixed_cap, &part);
@@ -2132,13 +2133,14 @@ int tiles_impl(pt_ptycho* h, float2* out, const float2* gin, const float2* f, co
   return run_fold<MODE>(h, out, f, hh, lamd, (float)rho, rho_dev, st);
 }
 
-// LDS budget of an overlap-add workgroup.  12 KB for frames up to 16 x 16
-// (13 resident per CU; a 16x16 probe gets 16 x 16 pixel tiles, extended to
-// 31 x 31).  40 KB for larger frames: at 32 x 32 the transpose buffers alone
-// take 8.4 KB, and in 12 KB the tiles would shrink to 8 pixels -- one patch
-// per tile at step 8 (half of the wave's frame slots idle) and ~25
-// overlapping tiles summed per pixel by the fold; at 40 KB a 32x32 probe gets
-// 32 x 32 pixel tiles extended to 63 x 63.
+// The extended tile takes what a workgroup of one wave (k_tile) leaves of this after
+// its transpose buffers.  12 KB for frames up to 16 x 16 (13 resident per CU; a 16 x
+// 16 probe gets 16 x 16 pixel tiles, extended to 31 x 31).  40 KB for larger frames:
+// a 32 x 32 probe gets 32 x 32 pixel tiles extended to 63 x 63, where in 12 KB the
+// tiles would shrink to 8 pixels -- one patch per tile at step 8 and ~25 overlapping
+// tiles summed per pixel by the fold.  One wave per frame (k_tile_w) keeps these tiles
+// and adds the buffers of its four waves and the staged probe: 57 KB for the gradient
+// of 32 x 32 frames, 51 KB for 64 x 64 ones with a 16 x 16 probe, two workgroups per CU.
 constexpr size_t kTileLdsBudget = 12 * 1024;
 constexpr size_t kTileLdsBudgetLarge = 40 * 1024;
 
@@ -2334,7 +2336,7 @@ static int run_grad_group(const pt_ptycho_grad_args* a, const int* idx, int n, i
     const pt_ptycho_grad_args& x = a[idx[k]];
     const pt_ptycho* h = x.h;
     g.a[k] = tile_args(h, nullptr, (const float2*)x.psi, x.data, x.coefptycho, x.coefdata,
-                       h->c * x.coefptycho, model);
+                       h->c * x.coefptycho);
     g.gx[k] = h->ntiles;
     g.start[k] = tot;
     tot += h->ntiles;

@@ -8,13 +8,14 @@
 // grid, N = 3n/2), restructured:
 //  * The checkerboard multiplications around each FFT are centred DFTs; they
 //    are realised as index rotations on load/store (free).
-//  * The 2N-point centred DFT of an input that is non-zero only on the
-//    central N points splits into two N-point DFTs (even outputs: plain
-//    input; odd outputs: input twisted by exp(-i pi j/N)).  All FFTs are
-//    N-point Stockham transforms: for n = 64, 128, 256, 512 register line
-//    FFTs (24 points per lane, compile-time passes, LDS only for the
-//    exchanges between passes), otherwise LDS transforms with a run-time
-//    mixed-radix plan (2/3/4/5/8).
+//  * The 2L-point centred DFT of an input that is non-zero only on the
+//    central L points splits into two L-point DFTs (even outputs: plain
+//    input; odd outputs: input twisted by exp(-i pi j/L)).  All FFTs are
+//    Stockham transforms of N points (the forward's grid lines and the detector
+//    lines) or n points (the adjoint's grid lines): for n = 64, 96, 128, 192, 256
+//    and 512 register line FFTs (24 points per lane; n-point lines of a power of
+//    two 16), compile-time passes with LDS only for the exchanges between them,
+//    otherwise LDS transforms with a run-time mixed-radix plan (2/3/4/5/8).
 //  * pad2 + circ + divphi are applied while loading the object rows; the
 //    adjoint's unpaddivphi + circ + crop are applied while storing them.  The
 //    adjoint only needs the n x n object points (the forward transforms the
@@ -211,8 +212,10 @@ __global__ __launch_bounds__(256) void k_col_fwd(float2* __restrict__ Bg, const 
 // ------------------------------------------------------------------ gridding kernel
 // Interpolation between the oversampled grid and the polar samples with the
 // Kaiser-Bessel kernel I0(beta sqrt(1 - (2d/w)^2)) / I0(beta) of width w = 8
-// grid points, beta = pi sqrt((w/s)^2 (s - 1/2)^2 - 0.8) for oversampling
-// s = 2 (Beatty, Nishimura and Pauly 2005); its Fourier transform
+// grid points, beta as pi sqrt((w/s)^2 (s - 1/2)^2 - 0.8) = 18.6389 for oversampling
+// s = 2 (Beatty, Nishimura and Pauly 2005).  kBeta is 4.5e-6 below that expression,
+// for which the aliasing error is the same to 1e-4 of itself (5.25e-8 rms over the
+// object); kernel and transform use the one value.  Its Fourier transform
 // w sinh(r)/r / I0(beta), r = sqrt(beta^2 - (pi w xi)^2), is divided out of the
 // object points (dphi).  The reference's Gaussian with 15 x 15 taps
 // (kernels.cuh:97-158, eps = 1e-6) approximates the same nonuniform Fourier
@@ -1412,7 +1415,11 @@ extern "C" int pt_tomo_set_theta(pt_tomo* h, const float* theta, pt_stream strea
   // Slices per work item (8 szb): as many as leave 4096 wavefronts (4 per SIMD),
   // since each staged weight and sample index then serves more products.
   // Entries per work item: at most 512, fewer in small problems, where the
-  // dense tiles around the grid's centre would outlast the others.
+  // dense tiles around the grid's centre would outlast the others; each chunk
+  // beyond a tile's first is a partial to write and add.  The share of 2048 work
+  // items is a compromise between the two: with 4096 the adjoint at 180^2 x 21
+  // slices, 201 angles takes 88 us instead of 94 and cg_tomo at 128^3 2175 instead of
+  // 2070, with 8192 that 2477, with 1024 the adjoint 104 and cg_tomo 2114.
   int szb = 4;
   while (szb > 1 && ntl * ((h->pzs / 8 + szb - 1) / szb) < 4096) szb /= 2;
   const long share = (long)ecnt[ntl] * ((h->pzs / 8 + szb - 1) / szb) / 2048;
