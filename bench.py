@@ -19,6 +19,7 @@ sample, run on this host's cores).
 import argparse
 import ctypes
 import json
+import math
 import os
 import sys
 import time
@@ -40,24 +41,29 @@ def kernel_bytes(tag, slv):
     N = 3 * n // 2
     S, D = slv.nscan, slv.ndety
     vol_t = 8 * nt * nz * n            # psi-sized complex64 array
-    if tag == "tomo_gather":            # 2N x 2N grid in, cropped projections out
-        return 8 * (2 * N) ** 2 * nz + vol_t
+    # the samples' disc of the forward's 2N x 2N and the adjoint's 2n x 2n grid
+    disc_f, disc_a = 8 * math.pi * N ** 2 * nz, 8 * math.pi * n ** 2 * nz
+    samples = 8 * nt * N * nz          # polar samples
+    if tag == "tomo_gather":            # grid in, polar samples out
+        return disc_f + samples
+    if tag == "tomo_line_idft":         # polar samples in, cropped projections out
+        return samples + vol_t
+    if tag == "tomo_adj_line":          # projections in, polar samples out
+        return vol_t + samples
     if tag == "tomo_scatter":           # polar samples in, grid out
-        return 8 * nt * N * nz + 8 * (2 * N) ** 2 * nz
+        return samples + disc_a
     if tag == "ptycho_grad_tile":       # psi in, data in, one psi-sized result out
         return vol_t + 4 * nt * S * D * D + vol_t
     if tag == "ptycho_minf":            # psi, d, h, lamd and data in (data and rho terms)
         return 4 * vol_t + 4 * nt * S * D * D
-    if tag == "tomo_col_fwd":           # N x 2N in, 2N x 2N out
-        return 8 * N * 2 * N * nz + 8 * (2 * N) ** 2 * nz
     if tag == "tomo_row_fwd":           # object in, N x 2N out
         return 8 * n * n * nz + 8 * N * 2 * N * nz
-    if tag == "tomo_col_adj":           # 2N x 2N in, n x 2N out
-        return 8 * (2 * N) ** 2 * nz + 8 * n * 2 * N * nz
-    if tag == "tomo_row_adj":           # n x 2N in, object out
-        return 8 * n * 2 * N * nz + 8 * n * n * nz
-    if tag == "tomo_fold":
-        return 8 * (2 * N) ** 2 * nz * 2
+    if tag == "tomo_col_fwd":           # N x 2N in, grid out
+        return 8 * N * 2 * N * nz + disc_f
+    if tag == "tomo_col_adj":           # grid in, n x 2n out
+        return disc_a + 8 * n * 2 * n * nz
+    if tag == "tomo_row_adj":           # n x 2n in, object out
+        return 8 * n * 2 * n * nz + 8 * n * n * nz
     return None
 
 
@@ -70,7 +76,6 @@ def minf_work(history, nchunk, piter):
     sweep schedule in order (the first CG step's schedule, then the later
     steps'); a step reaching 1e-12 ends at 0.  Also returns the number of
     Lagrangian evaluations (launched under their own tag)."""
-    import math
     from ptychotomo_amd.solver import _PSCHED_FIRST, _PSCHED_LATER
 
     def nsweeps(k, sched):
@@ -101,9 +106,10 @@ def minf_work(history, nchunk, piter):
 
 WARM_WEIGHTS = os.path.join(HERE, "ptychotomo_amd", "weights", "unet_warmstart_128.npz")
 
-TAGS = ["tomo_gather", "tomo_scatter", "tomo_fold", "tomo_row_fwd", "tomo_col_fwd",
-        "tomo_adj_line", "tomo_col_adj", "tomo_row_adj", "ptycho_grad_tile", "ptycho_fold",
-        "ptycho_minf"]
+TAGS = ["tomo_row_fwd", "tomo_col_fwd", "tomo_gather", "tomo_line_idft", "tomo_adj_line",
+        "tomo_scatter", "tomo_scatter_fix", "tomo_col_adj", "tomo_row_adj", "ptycho_grad_tile",
+        "ptycho_fold", "ptycho_minf"]
+GATHER_TAPS = 64        # 8 x 8 Kaiser-Bessel taps per polar sample and slice
 
 
 def prof_run(lib, tag, fn):
@@ -212,7 +218,7 @@ def config0_rates(log):
 
 def kernel_rates(slv, breakdown):
     """Per-launch rates of the probed kernels: algorithmic GB/s against HBM
-    and, for the USFFT gather (4 flops per complex x real tap, 225 taps per
+    and, for the USFFT gather (4 flops per complex x real tap, GATHER_TAPS per
     sample and slice), GFLOP/s against the FP32 vector peak.  The line-search
     kernel's rate is per full sweep (its launches include sweeps in which
     finished chunks exit at once)."""
@@ -231,7 +237,7 @@ def kernel_rates(slv, breakdown):
                  "algorithmic_bytes": nb, "GB_s": nb / (ms * 1e-3) / 1e9}
         r["frac_hbm"] = r["GB_s"] / HBM_PEAK_GBS
         if tag == "tomo_gather":
-            fl = 4.0 * 225 * slv.ntheta * N * slv.nz
+            fl = 4.0 * GATHER_TAPS * slv.ntheta * N * slv.nz
             r["flops"] = fl
             r["GFLOP_s"] = fl / (ms * 1e-3) / 1e9
             r["frac_fp32_vector"] = r["GFLOP_s"] / FP32_VECTOR_PEAK_GFLOPS
