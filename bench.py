@@ -9,7 +9,7 @@ iterations as in the reference), with all inputs resident in HBM.  W warm-up
 iterations (including the two piter+32 iterations of the reference
 schedule) precede K timed iterations.
 
-Prints one JSON line with the headline number, the roofline of the dominant
+Prints one JSON line (--full: the whole record to a file) with the headline number, the roofline of the dominant
 kernel (HIP events around each of its launches inside the timed region), the
 whole-volume operators' rates (tomography and ptychography forward/adjoint,
 GB/s against HBM, and against the same operators on the host) and the CPU
@@ -407,6 +407,8 @@ def main():
     ap.add_argument("--steps", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--workload", default="prod256")
+    ap.add_argument("--full", default=None, metavar="FILE",
+                    help="also write the whole record (traces, per-seed runs) as JSON")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--breakdown", action="store_true", help="per-kernel time per iteration")
     ap.add_argument("--no-breakdown-probe", action="store_true",
@@ -634,7 +636,32 @@ def main():
                            ("ptycho_fwd", "ptycho_fwd"), ("ptycho_adj", "ptycho_adj"))):
             out["operators"][name]["cpu_ms"] = cs[key] * 1e3
             out["operators"][name]["vs_cpu"] = cs[key] * 1e3 / out["operators"][name]["ms"]
-    print(json.dumps(out), flush=True)
+    if args.full:
+        with open(args.full, "w") as fh:
+            json.dump(out, fh)
+    print(result_line(out), flush=True)
+
+
+def result_line(out):
+    """The JSON line of a record: strict JSON, five digits per number, and
+    without the lists that only a closer look needs (the iterations' traces, the
+    per-seed runs, the network's layers beyond their rates), so that it stays well
+    under 8 KB; --full keeps everything."""
+    def short(v):
+        if isinstance(v, dict):
+            return {k: short(x) for k, x in v.items() if k not in ("plain_trace", "warm_trace",
+                                                                   "runs")}
+        if isinstance(v, (list, tuple)):
+            return [short(x) for x in v]
+        if isinstance(v, float):
+            return float(f"{v:.5g}") if math.isfinite(v) else None
+        return v
+    res = short(out)
+    for k in ("value", "ms_per_step"):
+        res[k] = out[k]
+    if "unet" in res:
+        res["unet"]["layers"] = {k: v["TFLOP_s"] for k, v in res["unet"]["layers"].items()}
+    return json.dumps(res, allow_nan=False)
 
 
 def time_to_tol(slv, data, w, run, niter, tol=1e-3):
