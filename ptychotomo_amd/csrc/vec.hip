@@ -1114,8 +1114,9 @@ __global__ void k_ls_select(double* __restrict__ state, const double* cand, doub
 // have been evaluated 10 us at 96 x 64^2, 48 us at 192 x 128^2, 400 us at 384 x 256^2
 // (bound: K, Ru, Rd, xi0, u, d, xi1 read once per group).  Up to kTLSmall blocks of
 // 1024 elements the first group has a sweep and all others share one; up to kTLLarge
-// the first three have one each; beyond that every group has.  Step accepted in the
-// first / second / third group: 23 / 75 / 77 us (96 x 64^2), 70 / 125 / 179 us
+// the first two have one each (a third for the third group costs cg_tomo at 128^3 0.7 %,
+// and steps below 2^-13 are rare); beyond that every group has.  Step accepted in the
+// first / second / third group: 23 / 75 / 77 us (96 x 64^2), 68 / 120 / 310 us
 // (192 x 128^2), 430 / 850 / 1260 us (384 x 256^2); with all groups after the first in
 // one sweep the latter took 70 / 295 / 304 and 418 / 2420 / 2430 us.  Half the blocks
 // up to kTLLarge: the selection then reads half the partials (at 192 x 128^2 75 -> 70
@@ -1250,7 +1251,7 @@ extern "C" int pt_k_tomo_linesearch(double* state, double* step, const void* K, 
   const FRegMinf fr{(const float2*)u, (const float2*)d, (const float2*)xi1, nullptr, kTLFirst + 1,
                     nz, ny, nx};
   // the first group of each sweep
-  static constexpr int few[] = {0, 1, kTLGroups}, some[] = {0, 1, 2, 3, kTLGroups},
+  static constexpr int few[] = {0, 1, kTLGroups}, some[] = {0, 1, 2, kTLGroups},
                        all[] = {0, 1, 2, 3, 4, 5, kTLGroups};
   const int* at = nb <= kTLSmall ? few : nb <= kTLLarge ? some : all;
   for (; at[0] < kTLGroups; ++at) {

@@ -805,7 +805,7 @@ def test_ptycho_fwd_patches_per_wave(det, P, n, step):
 @pytest.mark.parametrize("nt,nz,n", [(8, 32, 180), (130, 64, 128), (16, 208, 204)])
 def test_tomo_linesearch_groups_of_halvings(nt, nz, n):
     """pt_k_tomo_linesearch where all later groups of halvings share a sweep,
-    where the first three have their own and where every group has: the steps of
+    where the first two have their own and where every group has: the steps of
     the search made from its parts, accepted in each group and never.  And a step
     accepted at the tenth halving (second group) of a problem that memory bounds
     takes no longer than 2.8 times one accepted at the second (reading everything
